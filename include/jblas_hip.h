@@ -110,8 +110,8 @@ int jb_jmul_dev(int64_t M, int64_t N, int64_t P, double* D, const double* A, con
 
 /* jmul! in Float32 (the reference's jmul! is generic in T, src/gemm.jl:244-246):
  * D = A * X with the same recurrence in binary32 -- acc_1 = fl(A[i,1]*X[1,j]),
- * acc_n = fmaf(A[i,n], X[n,j], acc_{n-1}) in increasing n -- on a sequential-fma
- * kernel (vector ALUs), bit-identical, fringe included.  Leading dimensions M,
+ * acc_n = fmaf(A[i,n], X[n,j], acc_{n-1}) in increasing n -- on the FP32 matrix
+ * cores, whose chains are that recurrence, bit-identical, fringe included.  Leading dimensions M,
  * N, M.  Host pointers (synchronous) / device pointers on `stream`. */
 int jb_jmul_f32(int64_t M, int64_t N, int64_t P, float* D, const float* A, const float* X);
 int jb_jmul_f32_dev(int64_t M, int64_t N, int64_t P, float* D, const float* A, const float* X, void* stream);

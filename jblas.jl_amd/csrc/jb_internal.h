@@ -20,9 +20,9 @@ struct GemmArgs {
 };
 
 // ---- FP64 -----------------------------------------------------------------
-// Native FP64 MFMA GEMM (128x128 block tile, LDS double buffer).
+// Native FP64 MFMA GEMM; its chains are the jmul! recurrence bit for bit.
 hipError_t launch_dgemm_mfma(const GemmArgs& g, hipStream_t s);
-// Sequential-fma FP64 GEMM (bit-exact jmul! recurrence).
+// The jmul! recurrence on the vector ALUs (sequential fma).
 hipError_t launch_dgemm_recurrence(const GemmArgs& g, hipStream_t s);
 // kernel! (D += A*X) on the FP64 MFMA kernel: each chain starts from C and
 // every step is an fma; alpha/beta unused.
@@ -56,9 +56,8 @@ size_t emulated_flag_offset(int64_t m, int64_t n, int64_t k, int s, bool i8);
 size_t bf16x3_flag_offset(int64_t m, int64_t n, int64_t k);
 
 // ---- FP32 -----------------------------------------------------------------
+// Native FP32 MFMA GEMM; its chains are the jmul! recurrence in Float32 bit for bit.
 hipError_t launch_sgemm_mfma(const GemmArgs& g, hipStream_t s);
-// Sequential-fma FP32 GEMM (the jmul! recurrence in Float32, bit-exact).
-hipError_t launch_sgemm_recurrence(const GemmArgs& g, hipStream_t s);
 size_t bf16x3_workspace_bytes(int64_t m, int64_t n, int64_t k);
 // Non-finite inputs become NaN slices (every product they enter is NaN) and set
 // the two flags as in launch_dgemm_ozaki.

@@ -529,7 +529,8 @@ int jb_jmul(int64_t M, int64_t N, int64_t P, double* D, const double* A, const d
 
 // jmul! in Float32 (the reference's jmul! is generic in T, src/gemm.jl:244):
 // the same recurrence in binary32 (plain first product, then fmaf in
-// increasing k) on the sequential-fma kernel, bit-identical.
+// increasing k), bit-identical, on the FP32 MFMA kernel, whose chains are that
+// recurrence (800x900x840: 102 us on the vector ALUs, 18.8 us on the MFMA).
 extern "C++" {
 static int jmul_f32_locked(int64_t M, int64_t N, int64_t P, float* D, const float* A, const float* X, void* stream,
                            bool host) {
@@ -546,8 +547,8 @@ static int jmul_f32_locked(int64_t M, int64_t N, int64_t P, float* D, const floa
   g.C = D;
   g.ldc = M > 1 ? M : 1;
   auto run = [](const GemmArgs& d, hipStream_t s) {
-    const hipError_t e = launch_sgemm_recurrence(d, s);
-    return e == hipSuccess ? JB_OK : hip_fail(e, "sgemm_recurrence launch");
+    const hipError_t e = launch_sgemm_mfma(d, s);
+    return e == hipSuccess ? JB_OK : hip_fail(e, "sgemm_mfma launch");
   };
   if (!host) return run(g, (hipStream_t)stream);
   return run_staged(g, sizeof(float), false, run);

@@ -1,22 +1,20 @@
-// k_dgemm.hip -- FP64 GEMM kernels for gfx950.
+// k_dgemm.hip -- FP64 and FP32 GEMM kernels for gfx950.
 //
-// (1) dgemm_mfma: C = alpha*op(A)*op(B) + beta*C on v_mfma_f64_16x16x4f64.
-//     Replaces jmul!'s register-tiled AVX loop (src/gemm.jl:244-348): the CPU
-//     register tile (pick_kernel_size, src/kernel_structure.jl:76-99) becomes a
-//     64x64 wave tile of 4x4 MFMA blocks, and the software prefetch
-//     (src/memory_management.jl:181-277) becomes a double-buffered LDS stage
-//     fed by coalesced 16-byte global loads.  op(A)/op(B) transposition is
-//     absorbed by the loader's LDS write pattern.
+// (1) gemm_mfma: C = alpha*op(A)*op(B) + beta*C on v_mfma_f64_16x16x4f64 or
+//     v_mfma_f32_16x16x4f32.  Replaces jmul!'s register-tiled AVX loop
+//     (src/gemm.jl:244-348): the CPU register tile (pick_kernel_size,
+//     src/kernel_structure.jl:76-99) becomes a wave tile of 16x16 MFMA blocks,
+//     and the software prefetch (src/memory_management.jl:181-277) an LDS ring
+//     that direct global->LDS loads fill ahead of the MFMAs.  op(A)/op(B)
+//     transposition is absorbed by the ring's image.
 // (2) dgemm_recurrence: one fma chain per element in increasing k, the exact
-//     order of src/gemm.jl:86 (first product) and :165 (fma k-step), for
-//     bit-level parity with the reference recurrence.
-//
-// LDS holds each operand tile k-major ([k][row], rows contiguous) so that an
-// MFMA fragment read is 16 consecutive doubles per 16-lane group.
+//     order of src/gemm.jl:86 (first product) and :165 (fma k-step), on the
+//     vector ALUs: an independent restatement of (1)'s bits.
 #include "jb_internal.h"
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 namespace jb {
 namespace {
@@ -24,125 +22,46 @@ namespace {
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-// 16-byte vector of T.
-template <typename T> struct Vec16;
-template <> struct Vec16<double> { typedef double type __attribute__((ext_vector_type(2))); };
-template <> struct Vec16<float> { typedef float type __attribute__((ext_vector_type(4))); };
-
-constexpr int NT = 256;  // threads per block (4 waves)
-constexpr int BK = 16;   // k extent of one LDS stage
-
-// Column XOR of k-row k in a swizzled k-major LDS tile: flips bits 2-4 of the
-// row index, so a 16-row fragment read stays 16 consecutive elements.
-__device__ __forceinline__ int kswz(int k) { return 4 * ((k >> 1) & 7); }
-
-// Loads one R x BK operand tile (R rows of op(A) or columns of op(B)) into
-// registers, then writes it k-major into LDS.
-//   MN_CONTIG: element (r, kk) at P[(r0+r) + (k0+kk)*ld]  (A 'N', B 'T')
-//   otherwise: element (r, kk) at P[(k0+kk) + (r0+r)*ld]  (A 'T', B 'N')
-// VEC: 16-byte loads are legal (base 16B aligned, ld a multiple of 16/sizeof(T)).
-// NEGZ: elements outside the operand read as -0.0 instead of +0.0 (see the
-// FP64 MFMA kernel: a -0 padding product leaves every chain value unchanged).
-template <typename T, int R, bool MN_CONTIG, bool VEC, bool NEGZ = false>
-struct TileLoader {
-  static constexpr T PADV = NEGZ ? T(-0.0) : T(0);
-  static constexpr int VW = 16 / sizeof(T);          // elements per 16-byte vector
-  static constexpr int PER = R * BK / (VW * NT);     // vectors per thread
-  static_assert(PER >= 1 && PER * VW * NT == R * BK, "tile must split into whole 16-byte vectors per thread");
-  typedef typename Vec16<T>::type V;
-  V v[PER];
-
-  // full: the whole R x BK tile lies inside the operand (block-uniform); one
-  // uniform branch picks the unguarded or the guarded loads.
-  __device__ __forceinline__ void load(const T* __restrict__ P, int64_t ld, int64_t r0, int64_t k0, int64_t Rtot,
-                                       int64_t K, bool full) {
-    if (full)
-      load_tile<true>(P, ld, r0, k0, Rtot, K);
-    else
-      load_tile<false>(P, ld, r0, k0, Rtot, K);
-  }
-
-  template <bool FULL>
-  __device__ __forceinline__ void load_tile(const T* __restrict__ P, int64_t ld, int64_t r0, int64_t k0,
-                                            int64_t Rtot, int64_t K) {
-    const int t = threadIdx.x;
-    if (MN_CONTIG) {
-      constexpr int RV = R / VW;  // vectors per k column
-      const int r = VW * (t % RV), kb = t / RV;
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int kk = kb + (NT / RV) * i;
-        const T* src = P + (r0 + r) + (k0 + kk) * ld;
-        if (FULL && VEC) {
-          v[i] = *reinterpret_cast<const V*>(src);
-        } else if (FULL) {
-#pragma unroll
-          for (int e = 0; e < VW; ++e) v[i][e] = src[e];
-        } else {
-          const bool kok = (k0 + kk) < K;
-#pragma unroll
-          for (int e = 0; e < VW; ++e) v[i][e] = (kok && r0 + r + e < Rtot) ? src[e] : PADV;
-        }
-      }
-    } else {
-      constexpr int KV = BK / VW;  // vectors per row
-      const int kk = VW * (t % KV), rb = t / KV;
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int r = rb + (NT / KV) * i;
-        const T* src = P + (k0 + kk) + (r0 + r) * ld;
-        if (FULL && VEC) {
-          v[i] = *reinterpret_cast<const V*>(src);
-        } else if (FULL) {
-#pragma unroll
-          for (int e = 0; e < VW; ++e) v[i][e] = src[e];
-        } else {
-          const bool rok = (r0 + r) < Rtot;
-#pragma unroll
-          for (int e = 0; e < VW; ++e) v[i][e] = (rok && k0 + kk + e < K) ? src[e] : PADV;
-        }
-      }
-    }
-  }
-
-  // SWZ (k-contiguous loads only): row r of k-row k is stored at column
-  // r ^ kswz(k), which spreads the 8 k-rows one store instruction writes
-  // over distinct banks; readers apply the same XOR.
-  template <int STRIDE, bool SWZ = false>
-  __device__ __forceinline__ void store(T* S) const {
-    const int t = threadIdx.x;
-    if (MN_CONTIG) {
-      constexpr int RV = R / VW;
-      const int r = VW * (t % RV), kb = t / RV;
-#pragma unroll
-      for (int i = 0; i < PER; ++i) *reinterpret_cast<V*>(S + (kb + (NT / RV) * i) * STRIDE + r) = v[i];
-    } else {
-      constexpr int KV = BK / VW;
-      const int kk = VW * (t % KV), rb = t / KV;
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int r = rb + (NT / KV) * i;
-#pragma unroll
-        for (int e = 0; e < VW; ++e) S[(kk + e) * STRIDE + (SWZ ? (r ^ kswz(kk + e)) : r)] = v[i][e];
-      }
-    }
-  }
-};
-
 // ---------------------------------------------------------------------------
-// (1) MFMA GEMM: 128x128 block tile, 4 waves of 64x64 (4x4 MFMA blocks of
-//     16x16), or 64x64 with waves of 32x32 when the 128-tile grid would
-//     leave the device's last round mostly idle, or (FP64) 64x32 / 32x32 when even
-//     the 64-tiles are fewer than four per CU; BK=16 per LDS stage, two
-//     LDS stages; global loads are issued one full stage (128-tile) or four
-//     stages (64-tile) before their LDS store (the load latency, not the MFMA
-//     work, bounded the earlier form that loaded within the stage).  T = double uses
-//     v_mfma_f64_16x16x4f64, T = float v_mfma_f32_16x16x4f32.
+// (1) MFMA GEMM, T = double (v_mfma_f64_16x16x4f64) or float
+//     (v_mfma_f32_16x16x4f32).  Both instructions are a sequential fma chain
+//     over their four k values in lane-group order (checked on the device bit
+//     for bit, denormals and signed zeros included), so with lane group g
+//     supplying k = 4t+g every element is one fma chain in increasing k: the
+//     jmul! recurrence.
+//
+//     A block of WGM x WGN waves owns a BTM x BTN tile of C.  Operand stages of
+//     BK k stream through an LDS ring of NSLOT slots by direct global->LDS
+//     loads, NSLOT - 1 stages ahead, with one barrier per stage and an explicit
+//     vmcnt wait for the stage at hand (later stages stay in flight).
+//
+//     Bound: the matrix cores.  What kept them idle was vector instructions: an
+//     MFMA shares the wave's vector issue, and each address add or LDS store in the
+//     loop cost more matrix time than its own few cycles (8192^3 FP64 66.6 TF/s with
+//     register staging, the same with direct loads and 27 vector instructions per
+//     stage, 72.9 with the barrier inside the last MFMA group, 76.3 of 78.6 with
+//     none left).  So the loads are buffer loads (descriptor + scalar + lane
+//     offset, no arithmetic), the stages are unrolled over the ring (constant LDS
+//     offsets), and the next fragments are read behind the first MFMA row of a group.
+//     FP64, register-staged form -> this: 1024^3 TN 44.2 -> 35.2 us, 4096^3 64 -> 74
+//     TF/s, 2999x1777x2111 on odd leading dimensions 462 -> 382 us; FP32 8192^3 130
+//     -> 152 of 157 TF/s.
+//
+//     LDS images (no padding: the loads write 64 consecutive pieces):
+//       rows contiguous (A 'N', B 'T'): [k][R], row r of k-row k at r ^ rswz(k);
+//       k contiguous (A 'T', B 'N'):    [R][BK] in 16-byte chunks, chunk c of
+//                                       row r at c ^ cswz(r).
+//     The XORs spread the 16 rows and 4 k of one fragment read over all 64
+//     banks; the loads apply them to the global address of each lane.
+//
+//     VEC: 16 bytes per lane (16-byte aligned bases, leading dimensions and the
+//     contiguous extent multiples of the vector); otherwise 4 bytes per lane,
+//     which serves any size and leading dimension through the same LDS image.
+//     Rows past the operand read its last row again (those results are not
+//     stored).  A last stage shorter than BK reads clamped k, and the
+//     fragments replace it: -0.0 from A and +0.0 from B, whose product -0 leaves
+//     every chain value unchanged.
 // ---------------------------------------------------------------------------
-#ifndef DG_PAD_BYTES
-#define DG_PAD_BYTES 32
-#endif
-
 template <typename T> struct Mfma;
 template <> struct Mfma<double> {
   typedef d4 acc_t;
@@ -160,29 +79,135 @@ template <> struct Mfma<float> {
   static __device__ __forceinline__ int prow(int r, int g) { return 4 * g + r; }
 };
 
-// BTM x BTN block tile, 4 waves of (BTM/2) x (BTN/2): 128 x 128, 64 x 64 (for
-// problems with too few 128-tiles to fill the device) or 64 x 32 (about one
-// 64-tile per CU: two 64 x 32 workgroups per CU then hide each other's
-// barrier and LDS latency).
-template <typename T, bool TA, bool TB, bool VEC, int BTM, int BTN>
-__global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(int64_t M, int64_t N, int64_t K, T alpha,
-                                                          const T* __restrict__ A, int64_t lda,
-                                                          const T* __restrict__ B, int64_t ldb, T beta,
-                                                          T* __restrict__ C, int64_t ldc, int tiles_m, int tiles_n,
-                                                          int acc_from_c) {
-  // LDS row stride in elements.  FP64: tile extent + 16 (144, 80 or 48), so
-  // the k-rows read by lane groups g and g+1 of a ds_read_b64 start 32 banks
-  // apart (no bank conflicts); the k-contiguous operands (A 'T', B 'N') are
-  // stored with the row XOR kswz(k), without which their 8-k-row stores would
-  // hit the same banks at this stride.  FP32: extent plus DG_PAD_BYTES.
-  constexpr bool F64 = sizeof(T) == 8;
-  constexpr int STRIDE_A = F64 ? BTM + 16 : BTM + DG_PAD_BYTES / (int)sizeof(T);
-  constexpr int STRIDE_B = F64 ? BTN + 16 : BTN + DG_PAD_BYTES / (int)sizeof(T);
-  constexpr int WIM = BTM / 32, WIN = BTN / 32;  // 16 x 16 MFMA blocks per wave along m, n
-  constexpr bool SWA = F64 && TA, SWB = F64 && !TB;
-  __shared__ __attribute__((aligned(16))) T As[2][BK * STRIDE_A];
-  __shared__ __attribute__((aligned(16))) T Bs[2][BK * STRIDE_B];
+// sched_barrier mask: vector and scalar ALU instructions may cross, memory instructions and MFMAs keep their order
+constexpr int SCHED_ALU = 6;
+#define JB_LDS __attribute__((address_space(3)))
+#define JB_INLINE __attribute__((always_inline))  // lambdas of the kernel: never outlined
+
+// One wave's load of 64 x LB bytes into LDS at dst, lane l's from base + so + vo (base and so wave-uniform).
+template <int LB>
+__device__ __forceinline__ void ring_load(gptr<const void> base, uint32_t vo, uint32_t so, char* dst) {
+#ifdef __HIP_DEVICE_COMPILE__  // the descriptor type exists on the device only
+  __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(const void*)base, 0, 0xffffffffu, 0x00027000);
+  if constexpr (LB == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (JB_LDS void*)dst, 16, vo, so, 0, 0);
+  else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (JB_LDS void*)dst, 4, vo, so, 0, 0);
+#endif
+}
+
+// One operand (R rows of op(A) or columns of op(B)) of the kernel below.
+//   RC: element (r, k) at P[r + k*ld], else at P[k + r*ld].
+//   WIDE: a lane's byte offset inside a stage may exceed 32 bits.
+template <typename T, int R, int BK, bool RC, bool VEC, int NW, bool WIDE>
+struct RingOperand {
+  static constexpr int EB = sizeof(T);
+  static constexpr int LB = VEC ? 16 : 4;                  // bytes per lane of one load
+  static constexpr int PB = 64 * LB;                       // bytes per load (one wave)
+  static constexpr int BYTES = R * BK * EB;                // one stage
+  static constexpr int NP = BYTES / PB / NW;               // loads per wave and stage
+  static_assert(NP >= 1 && NP * NW * PB == BYTES, "a stage must split into whole loads per wave");
+  static constexpr int ROWB = BK * EB;                     // k contiguous: bytes of one row,
+  static constexpr int CPR = ROWB / 16;                    // its 16-byte chunks,
+  static constexpr int RPB = ROWB < 256 ? 256 / ROWB : 1;  // and rows per 256 bytes (one pass over the banks)
+  static constexpr int EPL = PB / EB;                      // elements per load
+  static constexpr int KPL = EPL >= R ? EPL / R : 1;       // rows contiguous: k-rows per load,
+  static constexpr int LPK = EPL >= R ? 1 : R / EPL;       // or loads per k-row
+  static constexpr int RPL = ROWB <= PB ? PB / ROWB : 0;   // k contiguous: rows per load
+  static_assert(RC || RPL >= 1, "a load covers whole rows");
+  // The k-rows 4t..4t+3 of one fragment read must start 128 bytes (T = double,
+  // two per pass over the banks) or 64 bytes (T = float) apart.
+  static __device__ __forceinline__ int rswz(int k) {
+    if (EB == 8) return 16 * (k & 1);
+    return R >= 64 ? 16 * (k & 3) : 16 * ((k >> 1) & 1);
+  }
+  static_assert(!RC || R >= 32, "the row swizzle stays inside a k-row");
+  static __device__ __forceinline__ int cswz(int r) { return (r / RPB) & (CPR - 1); }
+
+  // LDS element of (r, k); r in [0, R), k in [0, BK)
+  static __device__ __forceinline__ int at(int r, int k) {
+    if (RC) return k * R + (r ^ rswz(k));
+    return r * BK + (((k * EB / 16) ^ cswz(r)) * 16 + (k * EB) % 16) / EB;
+  }
+
+  typedef typename std::conditional<WIDE, int64_t, uint32_t>::type Off;
+  Off off[NP];  // this lane's byte offset in load i of a stage, from the load's wave-uniform address
+  // ld: leading dimension; rmax: last row (vector start) that may be read, relative to the tile's first
+  __device__ __forceinline__ void init(int64_t ld, int rmax, int wave, int lane) {
+    const int lb = lane * LB;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int p = wave + NW * i;
+      if (RC) {
+        const int kl = KPL > 1 ? (lb / EB) / R : 0, rl = (lb / EB) % (KPL > 1 ? R : EPL);
+        const int r = min(((p % LPK) * EPL + rl) ^ rswz(p * KPL / LPK + kl), rmax);
+        off[i] = (Off)r * EB + (Off)kl * (Off)ld * EB + lb % EB;
+      } else {
+        const int row = p * RPL + lb / ROWB;
+        const int k = (((lb % ROWB) / 16 ^ cswz(row)) * 16 + lb % 16) / EB;
+        off[i] = (Off)min(row, rmax) * (Off)ld * EB + k * EB + lb % EB;
+      }
+    }
+  }
+  // Load i of this wave's share of the stage at k0 into LDS at `dst` (the operand's part of a slot).
+  __device__ __forceinline__ void issue(gptr<const T> P, int64_t ld, int64_t k0, int wave, char* dst, int i) const {
+    const int p = wave + NW * i;
+    const int64_t k = RC ? p * KPL / LPK : 0;  // uniform: first k-row of the load
+    if constexpr (WIDE) {
+      put((gptr<const char>)(P + (RC ? (k0 + k) * ld : k0)) + off[i], dst + p * PB);
+    } else {
+      // A buffer load adds the stage's base (descriptor), the load's offset (scalar)
+      // and the lane's by itself: no vector address arithmetic is left in the loop
+      // (a vector instruction holds up the FP64 matrix pipe).
+      ring_load<LB>(P + (RC ? k0 * ld : k0), off[i], (uint32_t)k * (uint32_t)ld * EB, dst + p * PB);
+    }
+  }
+  // The same for the last stage, shorter than BK: k clamped to kmax (last vector start).
+  static __device__ __forceinline__ void issue_tail(gptr<const T> P, int64_t ld, int64_t k0, int rmax, int64_t kmax,
+                                                    int wave, int lane, char* dst, int i) {
+    asm volatile("" : "+v"(lane));  // the addresses are formed here, not ahead of the main loop
+    const int p = wave + NW * i, lb = lane * LB;
+    gptr<const T> src;
+    if (RC) {
+      const int kl = KPL > 1 ? (lb / EB) / R : 0, rl = (lb / EB) % (KPL > 1 ? R : EPL);
+      const int k = p * KPL / LPK + kl;
+      src = P + min(((p % LPK) * EPL + rl) ^ rswz(k), rmax) + min<int64_t>(k0 + k, kmax) * ld;
+    } else {
+      const int row = p * RPL + lb / ROWB;
+      const int k = (((lb % ROWB) / 16 ^ cswz(row)) * 16 + lb % 16) / EB;
+      src = P + (int64_t)min(row, rmax) * ld + min<int64_t>(k0 + k, kmax);
+    }
+    put((gptr<const char>)src + lb % EB, dst + p * PB);
+  }
+  static __device__ __forceinline__ void put(gptr<const char> src, char* dst) {
+    if constexpr (VEC) __builtin_amdgcn_global_load_lds((gptr<const void>)src, (JB_LDS void*)dst, 16, 0, 0);
+    else __builtin_amdgcn_global_load_lds((gptr<const void>)src, (JB_LDS void*)dst, 4, 0, 0);
+  }
+};
+
+// s_waitcnt: at most N vector-memory operations outstanding and every LDS read returned.
+template <int N>
+__device__ __forceinline__ void wait_ring() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
+}
+
+template <typename T, bool TA, bool TB, bool VEC, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK,
+          int NSLOT_, int MINW>
+__global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
+    int64_t M, int64_t N, int64_t K, T alpha, const T* __restrict__ A_, int64_t lda, const T* __restrict__ B_, int64_t ldb,
+    T beta, T* __restrict__ C, int64_t ldc, int tiles_m, int tiles_n, int acc_from_c) {
+  constexpr int NW = WGM * WGN;
+  typedef RingOperand<T, BTM, BK, !TA, VEC, NW, WIDE> OA;
+  typedef RingOperand<T, BTN, BK, TB, VEC, NW, WIDE> OB;
+  constexpr int WIM = BTM / WGM / 16, WIN = BTN / WGN / 16;  // 16 x 16 MFMA blocks per wave along m, n
+  constexpr int STAGE_B = OA::BYTES + OB::BYTES;
+  constexpr int NLD = OA::NP + OB::NP;  // loads per wave and stage
+  constexpr int NSLOT = (NSLOT_ - 2) * NLD < 64 ? NSLOT_ : 63 / NLD + 2;  // the loads a wait leaves in flight fit its counter
+  constexpr int VW = VEC ? 16 / (int)sizeof(T) : 1;
+  constexpr int NT4 = BK / 4;  // MFMA k-groups per stage
+  static_assert(NT4 % 2 == 0, "the fragment buffers alternate over whole stages");
+  __shared__ __attribute__((aligned(1024))) char ring[NSLOT * STAGE_B];
   typedef typename Mfma<T>::acc_t acc_t;
+  gptr<const T> A = as_global(A_), B = as_global(B_);
 
   const int nblocks = tiles_m * tiles_n;
   const int tile = xcd_remap(blockIdx.x, nblocks, 8);
@@ -190,31 +215,42 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(int64_t M, int64_t N, 
   tile_coords(tile, tiles_m, tiles_n, 8, tm, tn);
   const int64_t m0 = (int64_t)tm * BTM, n0 = (int64_t)tn * BTN;
 
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int wm0 = (wave % 2) * (BTM / 2), wn0 = (wave / 2) * (BTN / 2);
+  const int lane = threadIdx.x % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int wm0 = (wave % WGM) * (BTM / WGM), wn0 = (wave / WGM) * (BTN / WGN);
   const int g = lane / 16, l16 = lane % 16;
 
-  // PD register sets carry the next PD stages: a stage's loads are issued PD
-  // stages before its LDS store.  The smaller tiles run where the grid has
-  // about one tile per CU and a stage is only 16 MFMAs per wave or fewer, far
-  // shorter than a global load, so they keep 4 stages in flight; the 128-tile
-  // keeps 1.
-  constexpr int PD = BTM == 128 ? 1 : 4;
-  TileLoader<T, BTM, !TA, VEC, F64> la[PD];  // FP64: A's k-padding is -0.0 (below)
-  TileLoader<T, BTN, TB, VEC> lb[PD];
-  const bool fullA = m0 + BTM <= M, fullB = n0 + BTN <= N;
+  gptr<const T> At = A + (TA ? m0 * lda : m0), Bt = B + (TB ? n0 : n0 * ldb);
+  const int ramax = (int)min<int64_t>(M - m0 - (TA ? 1 : VW), BTM);
+  const int rbmax = (int)min<int64_t>(N - n0 - (TB ? VW : 1), BTN);
+  const int64_t kamax = K - (TA ? VW : 1), kbmax = K - (TB ? 1 : VW);
+  const int nst = (int)((K + BK - 1) / BK);
+  const int nfull = (int)(K / BK);
+  OA oa;
+  OB ob;
+  oa.init(lda, ramax, wave, lane);
+  ob.init(ldb, rbmax, wave, lane);
+  // load i of stage st; tail: the last stage, shorter than BK
+  auto issue = [&](int st, int slot, int i, auto tail) JB_INLINE {
+    char* dst = ring + slot * STAGE_B;
+    const int64_t k0 = (int64_t)st * BK;
+    if (decltype(tail)::value) {
+      if (i < OA::NP) OA::issue_tail(At, lda, k0, ramax, kamax, wave, lane, dst, i);
+      else OB::issue_tail(Bt, ldb, k0, rbmax, kbmax, wave, lane, dst + OA::BYTES, i - OA::NP);
+    } else {
+      if (i < OA::NP) oa.issue(At, lda, k0, wave, dst, i);
+      else ob.issue(Bt, ldb, k0, wave, dst + OA::BYTES, i - OA::NP);
+    }
+  };
 
-  // FP64 chains start from -0.0: the first MFMA step fma(a, x, -0.0) is then
-  // exactly fl(a * x) for every input, the plain first product of the
-  // reference recurrence (src/gemm.jl:86), signed zeros included (a start of
-  // +0.0 would turn an all -0 chain into +0).  The k-steps past K that the
-  // last 16-k stage pads must leave the chain unchanged too: A pads with -0.0
-  // and B with +0.0, so each padding product is -0 and x + (-0) == x for
-  // every x, zeros included.  Callers route k == 0 elsewhere.
+  // Chains start from -0.0: the first MFMA step fma(a, x, -0.0) is then exactly
+  // fl(a * x) for every input, the plain first product of the reference
+  // recurrence (src/gemm.jl:86), signed zeros included (a start of +0.0 would
+  // turn an all -0 chain into +0).  Callers route k == 0 elsewhere.
   // acc_from_c (kernel! semantics, src/kernels.jl:225-233): each chain starts
   // from the element of C instead, every k-step an fma; the caller passes
   // alpha = 1, beta = 0, so the epilogue stores the chain value itself.
-  constexpr T acc0 = F64 ? T(-0.0) : T(0);
+  constexpr T acc0 = T(-0.0);
   acc_t acc[WIM][WIN];
 #pragma unroll
   for (int i = 0; i < WIM; ++i)
@@ -234,77 +270,101 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(int64_t M, int64_t N, 
     }
   }
 
-  const int nkt = (int)((K + BK - 1) / BK);
-  // Stage j travels in register set j % PD: loaded as soon as stage j - PD
-  // left that set for LDS, stored to LDS buffer j & 1 near the end of stage
-  // j - 1.
-  auto load_stage = [&](auto& xa, auto& xb, int kt) {
-    const int64_t k0 = (int64_t)kt * BK;
-    const bool fk = k0 + BK <= K;
-    xa.load(A, lda, m0, k0, M, K, fullA && fk);
-    xb.load(B, ldb, n0, k0, N, K, fullB && fk);
-  };
-  load_stage(la[0], lb[0], 0);
-  la[0].template store<STRIDE_A, SWA>(As[0]);
-  lb[0].template store<STRIDE_B, SWB>(Bs[0]);
 #pragma unroll
-  for (int j = 1; j <= PD; ++j)
-    if (j < nkt) load_stage(la[j % PD], lb[j % PD], j);
-  __syncthreads();
+  for (int d = 0; d < NSLOT; ++d)
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      if (d < nfull) issue(d, d, i, std::false_type());
+      else if (d < nst) issue(d, d, i, std::true_type());
+    }
 
-  // MFMA t of a stage covers k = 4t..4t+3; lane group g supplies k = 4t+g.
-  // Swizzled column (w0 + 16i + l16) ^ kswz(4t + g): with t < 4, kswz(4t + g) =
-  // 16 (t >> 1) + 8 (t & 1) + 4 (g >> 1), and w0 is a multiple of 16, so it is
-  // 16 ((w0/16 + i) ^ (t >> 1)) + (l16 ^ (8 (t & 1) + 4 (g >> 1))): a
-  // compile-time block offset (per wave) plus one of two per-lane columns.
-  static_assert(BK == 16, "swizzle decomposition assumes four MFMA k-groups per stage");
-  const int sw0 = l16 ^ (4 * (g >> 1)), sw1 = l16 ^ (8 + 4 * (g >> 1));
-  const int bm0 = wm0 / 16, bn0 = wn0 / 16;
-  auto frags = [&](const T* as, const T* bs, int t, T (&a)[WIM], T (&b)[WIN]) {
-    const int swc = (t & 1) ? sw1 : sw0;
+  T a[2][WIM], b[2][WIN];
+  auto frags = [&](int slot, int t, T (&x)[WIM], T (&y)[WIN]) JB_INLINE {
+    const T* as = reinterpret_cast<const T*>(ring + slot * STAGE_B);
+    const T* bs = reinterpret_cast<const T*>(ring + slot * STAGE_B + OA::BYTES);
 #pragma unroll
-    for (int i = 0; i < WIM; ++i)
-      a[i] = as[(4 * t + g) * STRIDE_A + (SWA ? 16 * ((bm0 + i) ^ (t >> 1)) + swc : wm0 + 16 * i + l16)];
+    for (int i = 0; i < WIM; ++i) x[i] = as[OA::at(wm0 + 16 * i + l16, 4 * t + g)];
 #pragma unroll
-    for (int j = 0; j < WIN; ++j)
-      b[j] = bs[(4 * t + g) * STRIDE_B + (SWB ? 16 * ((bn0 + j) ^ (t >> 1)) + swc : wn0 + 16 * j + l16)];
+    for (int j = 0; j < WIN; ++j) y[j] = bs[OB::at(wn0 + 16 * j + l16, 4 * t + g)];
   };
-
-  for (int kt0 = 0; kt0 < nkt; kt0 += PD)
+  // Waits for this wave's loads of stage st (all but those of the later stages in
+  // flight) and its LDS reads, then for every wave.  A plain barrier: the fence of
+  // __syncthreads() would wait for all loads.
+  auto arrive = [&](int st, auto steady) JB_INLINE {
+    const int later = nst - 1 - st;
+    if (decltype(steady)::value || later >= NSLOT - 2) wait_ring<(NSLOT - 2) * NLD>();
+    else if (NSLOT >= 4 && later == NSLOT - 3) wait_ring<(NSLOT >= 4 ? NSLOT - 3 : 0) * NLD>();
+    else wait_ring<0>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // Stage st in slot `slot`, whose first fragments are in a[0], b[0].  In its last
+  // MFMA group the block meets once: stage st + 1 has landed and every wave has
+  // read all of stage st, so its slot takes stage st + NSLOT and the next stage's
+  // first fragments are read while that group's MFMAs run.
+  // TAIL: the short last stage.  STEADY: stage st + NSLOT is a whole stage.
+  auto stage = [&](int st, int slot, int nslot, auto tail, auto steady) JB_INLINE {
+    constexpr bool TAIL = decltype(tail)::value, STEADY = decltype(steady)::value;
 #pragma unroll
-  for (int d = 0; d < PD; ++d) {
-    const int kt = kt0 + d;
-    if (kt >= nkt) break;
-    const int nset = (d + 1) % PD;  // register set of stage kt+1 (compile-time)
-    const int cur = kt & 1;
-    const T* as = As[cur];
-    const T* bs = Bs[cur];
-    T a[2][WIM], b[2][WIN];
-    frags(as, bs, 0, a[0], b[0]);
+    for (int t = 0; t < NT4; ++t) {
+      const int cur = t & 1;
+      if (TAIL) {
+        const bool past = (int64_t)st * BK + 4 * t + g >= K;
 #pragma unroll
-    for (int t = 0; t < BK / 4; ++t) {
-      if (t + 1 < BK / 4) frags(as, bs, t + 1, a[(t + 1) & 1], b[(t + 1) & 1]);
+        for (int i = 0; i < WIM; ++i) a[cur][i] = past ? T(-0.0) : a[cur][i];
+#pragma unroll
+        for (int j = 0; j < WIN; ++j) b[cur][j] = past ? T(0.0) : b[cur][j];
+      }
+      auto ahead = [&]() JB_INLINE {
+        if (t + 1 < NT4) {
+          frags(slot, t + 1, a[cur ^ 1], b[cur ^ 1]);
+        } else if (STEADY || st + 1 < nst) {
+          arrive(st + 1, steady);
+          frags(nslot, 0, a[cur ^ 1], b[cur ^ 1]);
+        }
+        __builtin_amdgcn_sched_barrier(SCHED_ALU);
+      };
+      // The next group's fragments are read behind the first row of MFMAs (whose
+      // wait for this group's then covers nothing else).
+      if (WIM == 1) ahead();
       // D'[p][q] = sum_k X[p][k] Y[k][q] with X = op(B)^T block (p -> n) and Y = op(A)^T
       // block (q -> m), so a 16-lane group holds 16 consecutive rows of one column of C
-      // (coalesced column-major stores).  The f64 MFMA is a sequential fma chain over
-      // its four k values in lane-group order, so each dot product is one fma chain in
-      // increasing k, as in the reference recurrence.
+      // (coalesced column-major stores).
 #pragma unroll
-      for (int i = 0; i < WIM; ++i)
+      for (int i = 0; i < WIM; ++i) {
 #pragma unroll
-        for (int j = 0; j < WIN; ++j) acc[i][j] = Mfma<T>::mma(b[t & 1][j], a[t & 1][i], acc[i][j]);
-      // The next stage goes to the other LDS buffer (last read before the
-      // previous barrier) one MFMA group before the end, so its writes
-      // complete under the last group instead of in front of the barrier;
-      // the registers then take the stage after it.
-      if (t == BK / 4 - 2 && kt + 1 < nkt) {
-        la[nset].template store<STRIDE_A, SWA>(As[cur ^ 1]);
-        lb[nset].template store<STRIDE_B, SWB>(Bs[cur ^ 1]);
-        if (kt + 1 + PD < nkt) load_stage(la[nset], lb[nset], kt + 1 + PD);
+        for (int j = 0; j < WIN; ++j) acc[i][j] = Mfma<T>::mma(b[cur][j], a[cur][i], acc[i][j]);
+        __builtin_amdgcn_sched_barrier(SCHED_ALU);
+        if (i == 0 && WIM > 1) ahead();
+        if (t + 1 == NT4) {
+          constexpr int PI = (NLD + WIM - 1) / WIM;
+#pragma unroll
+          for (int q = PI * i; q < PI * (i + 1) && q < NLD; ++q) {
+            if (STEADY) issue(st + NSLOT, slot, q, std::false_type());
+            else if (!TAIL && st + NSLOT < nfull) issue(st + NSLOT, slot, q, std::false_type());
+            else if (!TAIL && st + NSLOT < nst) issue(st + NSLOT, slot, q, std::true_type());
+          }
+        }
       }
+      __builtin_amdgcn_sched_barrier(SCHED_ALU);
     }
-    __syncthreads();
-  }
+  };
+  arrive(0, std::false_type());
+  frags(0, 0, a[0], b[0]);
+  int st = 0, slot = 0, nslot = 1;
+  auto next = [&]() JB_INLINE {
+    ++st;
+    slot = nslot;
+    nslot = nslot + 1 == NSLOT ? 0 : nslot + 1;
+  };
+  // unrolled over the ring, so that every LDS address is a constant offset from a few lane registers
+  for (; st + 2 * NSLOT - 1 < nfull; st += NSLOT)
+#pragma unroll
+    for (int d = 0; d < NSLOT; ++d)
+      stage(st + d, d, d + 1 == NSLOT ? 0 : d + 1, std::false_type(), std::true_type());
+  for (; st < nfull; next()) stage(st, slot, nslot, std::false_type(), std::false_type());
+  if (st < nst) stage(st, slot, nslot, std::true_type(), std::false_type());
 
   if (m0 + BTM <= M && n0 + BTN <= N) {
     // Interior tile: for each 16-row strip, the beta*C loads are issued
@@ -347,22 +407,47 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(int64_t M, int64_t N, 
 }
 
 // ---------------------------------------------------------------------------
-// (2) Sequential-fma GEMM (bit-exact recurrence, FP64 or FP32): 64x64 block tile,
-//     each thread a 4x4 register tile, BK=16 LDS stage.
+// (2) Sequential-fma FP64 GEMM (the recurrence on the vector ALUs): 64x64 block
+//     tile, each thread a 4x4 register tile, BK=16 LDS stage.
 // ---------------------------------------------------------------------------
-constexpr int RB = 64;
-// LDS row stride: one 16-byte vector of padding (66 doubles, 68 floats), so rows
-// stay 16-byte aligned for the vector stores and start on different banks
-template <typename T>
-constexpr int rstride() { return RB + 16 / (int)sizeof(T); }
+constexpr int NT = 256;      // threads per block
+constexpr int BK = 16;       // k extent of one LDS stage
+constexpr int RB = 64;       // tile rows and columns
+constexpr int RSTRIDE = 66;  // LDS row stride in doubles
 
-template <typename T, bool TA, bool TB>
-__global__ __launch_bounds__(NT, 2) void gemm_recurrence_kernel(int64_t M, int64_t N, int64_t K, T alpha,
-                                                                const T* __restrict__ A, int64_t lda,
-                                                                const T* __restrict__ B, int64_t ldb, T beta,
-                                                                T* __restrict__ C, int64_t ldc, int tiles_m,
-                                                                int tiles_n) {
-  constexpr int RSTRIDE = rstride<T>();
+// One RB x BK operand tile, element by element: registers, then LDS k-major.
+//   RC: element (r, kk) at P[(r0+r) + (k0+kk)*ld] (A 'N', B 'T'), else at P[(k0+kk) + (r0+r)*ld]
+template <bool RC>
+struct TileLoader {
+  static constexpr int PER = RB * BK / NT;
+  double v[PER];
+  static __device__ __forceinline__ int row(int e) { return RC ? e % RB : e / BK; }
+  static __device__ __forceinline__ int kof(int e) { return RC ? e / RB : e % BK; }
+  __device__ __forceinline__ void load(const double* __restrict__ P, int64_t ld, int64_t r0, int64_t k0, int64_t Rtot,
+                                       int64_t K) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = threadIdx.x + NT * i;
+      const int64_t r = r0 + row(e), k = k0 + kof(e);
+      v[i] = (r < Rtot && k < K) ? P[RC ? r + k * ld : k + r * ld] : 0.0;
+    }
+  }
+  __device__ __forceinline__ void store(double* S) const {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = threadIdx.x + NT * i;
+      S[kof(e) * RSTRIDE + row(e)] = v[i];
+    }
+  }
+};
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(NT, 2) void dgemm_recurrence_kernel(int64_t M, int64_t N, int64_t K, double alpha,
+                                                                 const double* __restrict__ A, int64_t lda,
+                                                                 const double* __restrict__ B, int64_t ldb, double beta,
+                                                                 double* __restrict__ C, int64_t ldc, int tiles_m,
+                                                                 int tiles_n) {
+  typedef double T;
   __shared__ __attribute__((aligned(16))) T As[BK * RSTRIDE];
   __shared__ __attribute__((aligned(16))) T Bs[BK * RSTRIDE];
   const int nblocks = tiles_m * tiles_n;
@@ -372,8 +457,8 @@ __global__ __launch_bounds__(NT, 2) void gemm_recurrence_kernel(int64_t M, int64
   const int64_t m0 = (int64_t)tm * RB, n0 = (int64_t)tn * RB;
   const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
 
-  TileLoader<T, RB, !TA, false> la;
-  TileLoader<T, RB, TB, false> lb;
+  TileLoader<!TA> la;
+  TileLoader<TB> lb;
   T acc[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -383,11 +468,11 @@ __global__ __launch_bounds__(NT, 2) void gemm_recurrence_kernel(int64_t M, int64
     }
 
   for (int64_t k0 = 0; k0 < K; k0 += BK) {
-    la.load(A, lda, m0, k0, M, K, false);
-    lb.load(B, ldb, n0, k0, N, K, false);
+    la.load(A, lda, m0, k0, M, K);
+    lb.load(B, ldb, n0, k0, N, K);
     __syncthreads();  // previous stage fully consumed
-    la.template store<RSTRIDE>(As);
-    lb.template store<RSTRIDE>(Bs);
+    la.store(As);
+    lb.store(Bs);
     __syncthreads();
     const int kmax = (int)min<int64_t>(BK, K - k0);
     int kk = 0;
@@ -443,83 +528,88 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 }  // namespace
 
-template <typename T, int BTM, int BTN>
+template <typename T, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int NSLOT, int MINW>
 static hipError_t launch_gemm_mfma_bt(const GemmArgs& g, hipStream_t s, int acc_from_c) {
   const int tiles_m = (int)((g.m + BTM - 1) / BTM), tiles_n = (int)((g.n + BTN - 1) / BTN);
   const int nblocks = tiles_m * tiles_n;
+  // 16-byte loads: aligned bases, and leading dimensions and contiguous extents of whole vectors
   constexpr int VW = 16 / sizeof(T);
-  const bool vec = aligned16(g.A) && aligned16(g.B) && (g.lda % VW == 0) && (g.ldb % VW == 0);
+  const bool vec = !WIDE && aligned16(g.A) && aligned16(g.B) && g.lda % VW == 0 && g.ldb % VW == 0 &&
+                   (g.ta ? g.k : g.m) % VW == 0 && (g.tb ? g.n : g.k) % VW == 0;
   auto A = static_cast<const T*>(g.A);
   auto B = static_cast<const T*>(g.B);
   auto C = static_cast<T*>(g.C);
   const T alpha = (T)g.alpha, beta = (T)g.beta;
   const char* tname = sizeof(T) == 8 ? "dgemm_mfma" : "sgemm_mfma";
-#define JB_LAUNCH(TA, TB, V)                                                                           \
-  hipLaunchKernelGGL((gemm_mfma_kernel<T, TA, TB, V, BTM, BTN>), dim3(nblocks), dim3(NT), 0, s, g.m, g.n, g.k, alpha, \
-                     A, g.lda, B, g.ldb, beta, C, g.ldc, tiles_m, tiles_n, acc_from_c)
+#define JB_LAUNCH_V(TA, TB, V)                                                                                          \
+  hipLaunchKernelGGL((gemm_mfma_kernel<T, TA, TB, V, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT, MINW>), dim3(nblocks),        \
+                     dim3(64 * WGM * WGN), 0, s, g.m, g.n, g.k, alpha, A, g.lda, B, g.ldb, beta, C, g.ldc, tiles_m,     \
+                     tiles_n, acc_from_c)
+#define JB_LAUNCH(TA, TB)                      \
+  do {                                         \
+    if (vec) JB_LAUNCH_V(TA, TB, !WIDE);     \
+    else JB_LAUNCH_V(TA, TB, false);         \
+  } while (0)
   timing_begin(s, tname);
-  if (vec) {
-    if (!g.ta && !g.tb) JB_LAUNCH(false, false, true);
-    else if (!g.ta && g.tb) JB_LAUNCH(false, true, true);
-    else if (g.ta && !g.tb) JB_LAUNCH(true, false, true);
-    else JB_LAUNCH(true, true, true);
-  } else {
-    if (!g.ta && !g.tb) JB_LAUNCH(false, false, false);
-    else if (!g.ta && g.tb) JB_LAUNCH(false, true, false);
-    else if (g.ta && !g.tb) JB_LAUNCH(true, false, false);
-    else JB_LAUNCH(true, true, false);
-  }
+  if (!g.ta && !g.tb) JB_LAUNCH(false, false);
+  else if (!g.ta && g.tb) JB_LAUNCH(false, true);
+  else if (g.ta && !g.tb) JB_LAUNCH(true, false);
+  else JB_LAUNCH(true, true);
+#undef JB_LAUNCH_V
 #undef JB_LAUNCH
   timing_end(s, tname);
   return hipGetLastError();
 }
 
-// Tile choice.  128-tiles run two blocks per CU (512 on the device at a time),
-// 64-tiles at least four and ~5 % below the 128-tile rate when both fill the
-// device; FP64 problems too small for four 64-tiles per CU take 64 x 32.  The
-// 128-tile grid is used when its last round of resident workgroups (512 for
-// FP64 on 256 CUs) is at least 90 % full (measured at n = 1536..8192:
-// 64-tiles win at 1536-3584 and 5120, 128-tiles at 4096, 6144, 8192).
-//
-// Round size of the 128-tile grid: the two workgroups per CU that the launch
-// bound guarantees, times the device's CU count.  (The occupancy query gives
-// FP32 three per CU; rounds of that size moved FP32 8192^3 to the 64-tile and
-// lost 6 %, so the rule stays on the guaranteed residency it was measured with.)
-static int64_t resident_128() { return 2 * (int64_t)std::max(runtime_compute_units(), 1); }
+// Ring configuration <waves along m, along n, k per stage, slots, waves per SIMD> of each tile.  A stage is 16 KB
+// (FP64 64-tile) to 32 KB; 128- and 64-tiles keep two slots and several workgroups per CU, whose waves fill each
+// other's barriers, the smaller tiles more slots, since their stages are shorter than a load's latency.
+template <typename T, int BTM, int BTN> struct Ring;
+template <> struct Ring<double, 128, 128> { static constexpr auto run = launch_gemm_mfma_bt<double, false, 128, 128, 2, 4, 16, 2, 4>; };
+template <> struct Ring<double, 64, 64> { static constexpr auto run = launch_gemm_mfma_bt<double, false, 64, 64, 2, 2, 16, 2, 4>; };
+template <> struct Ring<double, 64, 32> { static constexpr auto run = launch_gemm_mfma_bt<double, false, 64, 32, 2, 2, 16, 3, 4>; };
+template <> struct Ring<double, 32, 32> { static constexpr auto run = launch_gemm_mfma_bt<double, false, 32, 32, 2, 2, 16, 4, 4>; };
+template <> struct Ring<float, 128, 128> { static constexpr auto run = launch_gemm_mfma_bt<float, false, 128, 128, 2, 4, 32, 2, 4>; };
+template <> struct Ring<float, 64, 64> { static constexpr auto run = launch_gemm_mfma_bt<float, false, 64, 64, 2, 2, 32, 2, 4>; };
+template <> struct Ring<float, 64, 32> { static constexpr auto run = launch_gemm_mfma_bt<float, false, 64, 32, 2, 2, 32, 3, 4>; };
+template <> struct Ring<float, 32, 32> { static constexpr auto run = launch_gemm_mfma_bt<float, false, 32, 32, 2, 2, 32, 3, 4>; };
 
-// The 128-tile unless its last round of resident workgroups would be under
-// 90 % full; then the 64-tile (four times the tiles) fills the device better.
+// Tile choice: the tile whose fullest CU finishes first.  That CU runs
+// ceil(tiles / CUs) tiles, at the tile's own rate: larger tiles read less LDS per
+// MFMA and run faster, smaller ones spread a grid more evenly.  Rates relative to
+// the 128-tile, measured on full grids (2048^3 to 8192^3); one 128- or 64-tile
+// alone on its CU has no other workgroup to fill its barriers (5 and 10 % slower).
+// Measured, us (128 / 64 / 64x32 / 32): FP64 512^3 63 / 19.0 / 11.7 / 8.1, 1024^3
+// 124 / 37.6 / 36.7 / 36.9, 1536^3 178 / 146 / 119 / 119, 3072^3 1023 / 811 / 876 /
+// 943, 4096^3 1826 / 1961 / 2038 / 2209; FP32 800x840x900 60 / 20.3 / 20.4 / 18.8,
+// 3072^3 519 / 426 / 475 / 526, 4096^3 922 / 986 / 1074 / 1216.
 template <typename T>
 static hipError_t launch_gemm_mfma(const GemmArgs& g, hipStream_t s, int acc_from_c = 0) {
-  const int64_t tiles128 = ((g.m + 127) / 128) * ((g.n + 127) / 128);
-  const int64_t res = resident_128();
-  const int64_t slots = ((tiles128 + res - 1) / res) * res;
+  constexpr bool F64 = sizeof(T) == 8;
+  // A load's offset inside a stage spans up to 128 rows of ld elements (k contiguous) or 32 k of them (rows
+  // contiguous).  Past 32 bits (from 2^22 or 2^24 doubles on) the 64x32 tile with 64-bit addresses takes the problem.
+  const int64_t lim = ((int64_t)1 << 32) / (int64_t)sizeof(T);
+  if (g.lda >= lim / (g.ta ? 128 : 32) || g.ldb >= lim / (g.tb ? 32 : 128))
+    return launch_gemm_mfma_bt<T, true, 64, 32, 2, 2, F64 ? 16 : 32, 3, 2>(g, s, acc_from_c);
   // testing: pin one variant ("128", "64", "64x32", "32")
   const char* force = getenv("JB_GEMM_TILE");
   if (force && *force) {
-    if (!strcmp(force, "128")) return launch_gemm_mfma_bt<T, 128, 128>(g, s, acc_from_c);
-    if (!strcmp(force, "64")) return launch_gemm_mfma_bt<T, 64, 64>(g, s, acc_from_c);
-    if constexpr (sizeof(T) == 8) {  // FP32 64 x 32 and 32 x 32 would leave threads without a whole vector
-      if (!strcmp(force, "64x32")) return launch_gemm_mfma_bt<T, 64, 32>(g, s, acc_from_c);
-      if (!strcmp(force, "32")) return launch_gemm_mfma_bt<T, 32, 32>(g, s, acc_from_c);
-    }
+    if (!strcmp(force, "128")) return Ring<T, 128, 128>::run(g, s, acc_from_c);
+    if (!strcmp(force, "64")) return Ring<T, 64, 64>::run(g, s, acc_from_c);
+    if (!strcmp(force, "64x32")) return Ring<T, 64, 32>::run(g, s, acc_from_c);
+    if (!strcmp(force, "32")) return Ring<T, 32, 32>::run(g, s, acc_from_c);
   }
-  if ((double)tiles128 >= 0.9 * (double)slots) return launch_gemm_mfma_bt<T, 128, 128>(g, s, acc_from_c);
-  // FP64 with fewer than four 64-tiles per CU: 64 x 32 tiles (two per CU hide
-  // each other's barrier and LDS waits; measured +40 % at 512^3, +10 % at
-  // 1536^3, even at 2048^3 where the 64-tile grid has 4 per CU), and 32 x 32
-  // tiles where even the 64 x 32 grid has fewer than four per CU (waves of
-  // 16 x 16, four workgroups per CU: +31 % at 512^3, +25 % at 768^3, +4 % at
-  // 1024^3 over 64 x 32)
-  if constexpr (sizeof(T) == 8) {
-    const int64_t cus4 = 4 * (int64_t)std::max(runtime_compute_units(), 1);
-    const int64_t tiles64 = ((g.m + 63) / 64) * ((g.n + 63) / 64);
-    const int64_t tiles64x32 = ((g.m + 63) / 64) * ((g.n + 31) / 32);
-    if (tiles64 < cus4)
-      return tiles64x32 < cus4 ? launch_gemm_mfma_bt<T, 32, 32>(g, s, acc_from_c)
-                               : launch_gemm_mfma_bt<T, 64, 32>(g, s, acc_from_c);
-  }
-  return launch_gemm_mfma_bt<T, 64, 64>(g, s, acc_from_c);
+  const int64_t cus = std::max(runtime_compute_units(), 1);
+  auto cost = [&](int bm, int bn, double rate, double alone) {
+    const int64_t tiles = ((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn);
+    const int64_t rounds = (tiles + cus - 1) / cus;
+    return (double)(rounds * bm * bn) / (rounds == 1 ? rate * alone : rate);
+  };
+  const double c128 = cost(128, 128, 1.0, 0.95), c64 = cost(64, 64, F64 ? 0.96 : 0.91, 0.90);
+  const double c64x32 = cost(64, 32, F64 ? 0.885 : 0.83, 1.0), c32 = cost(32, 32, F64 ? 0.81 : 0.74, 1.0);
+  if (c128 <= std::min(c64, std::min(c64x32, c32))) return Ring<T, 128, 128>::run(g, s, acc_from_c);
+  if (c64 <= std::min(c64x32, c32)) return Ring<T, 64, 64>::run(g, s, acc_from_c);
+  return c64x32 < c32 ? Ring<T, 64, 32>::run(g, s, acc_from_c) : Ring<T, 32, 32>::run(g, s, acc_from_c);
 }
 
 hipError_t launch_dgemm_mfma(const GemmArgs& g, hipStream_t s) { return launch_gemm_mfma<double>(g, s); }
@@ -532,40 +622,24 @@ hipError_t launch_dgemm_mfma_acc(const GemmArgs& g, hipStream_t s) {
 }
 hipError_t launch_sgemm_mfma(const GemmArgs& g, hipStream_t s) { return launch_gemm_mfma<float>(g, s); }
 
-template <typename T>
-hipError_t launch_gemm_recurrence(const GemmArgs& g, hipStream_t s, const char* name) {
+hipError_t launch_dgemm_recurrence(const GemmArgs& g, hipStream_t s) {
   const int tiles_m = (int)((g.m + RB - 1) / RB), tiles_n = (int)((g.n + RB - 1) / RB);
   const int nblocks = tiles_m * tiles_n;
-  auto A = static_cast<const T*>(g.A);
-  auto B = static_cast<const T*>(g.B);
-  auto C = static_cast<T*>(g.C);
-  const T alpha = (T)g.alpha, beta = (T)g.beta;
-#define JB_LAUNCH(TA, TB)                                                                                    \
-  hipLaunchKernelGGL((gemm_recurrence_kernel<T, TA, TB>), dim3(nblocks), dim3(NT), 0, s, g.m, g.n, g.k, alpha, \
-                     A, g.lda, B, g.ldb, beta, C, g.ldc, tiles_m, tiles_n)
-  timing_begin(s, name);
-  if (!g.ta && !g.tb) {
-    JB_LAUNCH(false, false);
-  } else if (!g.ta && g.tb) {
-    JB_LAUNCH(false, true);
-  } else if (g.ta && !g.tb) {
-    JB_LAUNCH(true, false);
-  } else {
-    JB_LAUNCH(true, true);
-  }
+  auto A = static_cast<const double*>(g.A);
+  auto B = static_cast<const double*>(g.B);
+  auto C = static_cast<double*>(g.C);
+#define JB_LAUNCH(TA, TB)                                                                                         \
+  hipLaunchKernelGGL((dgemm_recurrence_kernel<TA, TB>), dim3(nblocks), dim3(NT), 0, s, g.m, g.n, g.k, g.alpha, A, \
+                     g.lda, B, g.ldb, g.beta, C, g.ldc, tiles_m, tiles_n)
+  timing_begin(s, "dgemm_recurrence");
+  if (!g.ta && !g.tb) JB_LAUNCH(false, false);
+  else if (!g.ta && g.tb) JB_LAUNCH(false, true);
+  else if (g.ta && !g.tb) JB_LAUNCH(true, false);
+  else JB_LAUNCH(true, true);
 #undef JB_LAUNCH
-  timing_end(s, name);
+  timing_end(s, "dgemm_recurrence");
   return hipGetLastError();
 }
-
-hipError_t launch_dgemm_recurrence(const GemmArgs& g, hipStream_t s) {
-  return launch_gemm_recurrence<double>(g, s, "dgemm_recurrence");
-}
-
-hipError_t launch_sgemm_recurrence(const GemmArgs& g, hipStream_t s) {
-  return launch_gemm_recurrence<float>(g, s, "sgemm_recurrence");
-}
-
 
 hipError_t launch_scale_f64(int64_t m, int64_t n, double beta, double* C, int64_t ldc, hipStream_t s) {
   if (m == 0 || n == 0) return hipSuccess;

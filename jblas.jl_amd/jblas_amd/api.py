@@ -160,9 +160,8 @@ def nonfinite_check(*, stream=None) -> None:
 def jmul_(D, A, X, *, stream=None):
     """D = A*X (jmul!, src/gemm.jl:244-348): the reference's per-element fma
     recurrence, bit-identical, with the fringe rows/columns written too.
-    Float64 (FP64 MFMA kernel, whose chains are that recurrence) or Float32
-    (the recurrence in binary32 on the sequential-fma kernel; the reference's
-    jmul! is generic in T, dense operands only)."""
+    Float64 or Float32 (the reference's jmul! is generic in T; Float32 takes
+    dense operands only), on the MFMA kernel, whose chains are that recurrence."""
     d, a, x = _Operand(D, True, "D"), _Operand(A, False, "A"), _Operand(X, False, "X")
     M, N = a.rows, a.cols
     if x.rows != N or d.rows != M or d.cols != x.cols:
