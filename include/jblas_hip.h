@@ -310,8 +310,8 @@ int jb_autotune_load(const char* path);
 /* Query the choice for one problem shape on its own: tile id (0 = 64x64 MFMA
  * tile, 1 = 32x32 MFMA tile, 2 = the whole problem in one work item on the
  * vector ALUs for m, n, k <= 64 -- fastmul!'s form, src/kernels.jl:202-208 --,
- * and, FP64 and 3xBF16 only, each run by a persistent kernel of its own:
- * 3 = 128x128, 4 = 128x64, 5 = 64x128 MFMA tiles) and split-K, from the table
+ * and, FP64 and 3xBF16 only, 3 = 128x128, 4 = 128x64, 5 = 64x128 MFMA tiles;
+ * FP64 tiles 0 and 1 run in 128x64 work items that skip what lies outside C) and split-K, from the table
  * or the static rule (FP64: the tile with the least padded area per unit of its
  * measured rate; 3xBF16: 64x128; native FP32: 64x64 or 32x32).  A plan may raise the split of
  * statically chosen problems while the group has fewer work items than the

@@ -9,10 +9,10 @@
 //   * work items (problem, output tile, k-split) sorted by decreasing cost
 //     are pulled from a device counter by a grid of CU-filling workgroups,
 //     so uneven problems load-balance;
-//   * tile shapes 64x64 and 32x32 (4 waves each) are device functions of
-//     one kernel, chosen per work item; the 128-row/column tiles (FP64 and
-//     3xBF16) run in kernels of their own, one per tile shape and transpose
-//     combination, launched concurrently with it;
+//   * the native methods' MFMA tiles run in persistent kernels per tile shape,
+//     transpose combination and load width (k_grouped_ring.h), the 3xBF16
+//     128-row/column tiles per shape and combination, the other 3xBF16 tiles and
+//     the small problems in one more; a plan's kernels run concurrently;
 //   * split-K partials go to a workspace slot per (tile, split); the last
 //     split to finish (per-tile arrival counter) sums them in split order,
 //     so results are deterministic;
@@ -29,6 +29,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "jb_grouped.h"
 #include "jb_runtime.h"
 
 namespace jb {
@@ -39,45 +40,6 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
-constexpr int GNT = 256;  // 4 waves
-// (Operand and result pointers come from problem descriptors in memory: every
-// access goes through as_global, jb_internal.h.)
-// Work-item configurations: 0 = 64x64 MFMA tile, 1 = 32x32 MFMA tile, 2 = the
-// whole problem on the vector ALUs (m, n, k <= SMALL_MAX, one split); FP64 and
-// 3xBF16 only, run by persistent kernels of their own whose register budget is
-// the large tile's (so the others keep four workgroups per CU): 3 = 128x128,
-// 4 = 128x64, 5 = 64x128 MFMA tiles.
-constexpr int NCFG = 6;
-constexpr int CFG_BM[NCFG] = {64, 32, 64, 128, 128, 64};  // tile rows
-constexpr int CFG_BN[NCFG] = {64, 32, 64, 128, 64, 128};  // tile columns
-constexpr int CFG_SMALL = 2;
-constexpr int CFG_LARGE = 3;
-constexpr int CFG_TALL = 4;
-constexpr int CFG_WIDE = 5;
-constexpr int SMALL_MAX = 64;
-__host__ __device__ constexpr bool large_cfg(int cfg) { return cfg >= CFG_LARGE; }
-
-// Device descriptor of one problem.
-struct GProb {
-  const void* A;
-  const void* B;
-  void* C;
-  void* part;         // split-K partials: tiles * splitk slabs of BM*BN elements
-  int64_t m, n, k, lda, ldb, ldc;
-  double alpha, beta;
-  int ta, tb, cfg, splitk;
-  int tiles_m, tiles_n;
-  int64_t kchunk;     // k per split (multiple of 32)
-  int counter_base;   // index of this problem's first per-tile arrival counter
-  int pad_;
-};
-struct GItem {
-  int prob, tile, split, pad_;
-};
-
-// ---------------------------------------------------------------------------
-// operand staging (generic strides, coalesced along the contiguous index)
-// ---------------------------------------------------------------------------
 // The thread index as an opaque value, read once per work item: offsets derived
 // from it are then formed inside the work loop of the persistent kernel rather
 // than hoisted out of it and held in registers for all eight tile variants at
@@ -88,424 +50,7 @@ __device__ __forceinline__ int work_item_tid() {
   return t;
 }
 
-// RC: the R index is the contiguous one (stride 1), else the k index is.
-// NEGZ: elements outside the operand read as -0.0 (FP64 A operand: a -0
-// padding product leaves every chain value unchanged, zeros included).
-template <typename T, int R, int BK, bool RC, bool NEGZ = false>
-struct GLoader {
-  static constexpr int PER = R * BK / GNT;
-  T v[PER];
-  int tid;  // thread index (see work_item_tid)
-  __device__ explicit GLoader(int t) : tid(t) {}
-  static __device__ __forceinline__ int row_of(int e) { return RC ? (e % R) : (e / BK); }
-  static __device__ __forceinline__ int k_of(int e) { return RC ? (e / R) : (e % BK); }
-  __device__ __forceinline__ void load(gptr<const T> P, int64_t ld, int64_t r0, int64_t k0, int64_t Rtot,
-                                       int64_t Kend) {
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int e = tid + GNT * i;
-      const int64_t gr = r0 + row_of(e), gk = k0 + k_of(e);
-      v[i] = (gr < Rtot && gk < Kend) ? (RC ? P[gr + gk * ld] : P[gk + gr * ld]) : (NEGZ ? T(-0.0) : T(0));
-    }
-  }
-  // the same with the vector-loader interface (element loads in every mode)
-  static __device__ __forceinline__ int mode(bool, bool, bool) { return 0; }
-  __device__ __forceinline__ void load(gptr<const T> P, int64_t ld, int64_t r0, int64_t k0, int64_t Rtot,
-                                       int64_t Kend, int) {
-    load(P, ld, r0, k0, Rtot, Kend);
-  }
-  template <int STRIDE, bool SWZ>
-  __device__ __forceinline__ void store(T* S) const {
-    static_assert(!SWZ, "element staging is not swizzled");
-    store_kmajor<STRIDE>(S);
-  }
-  // k-major [kk][r] (MFMA fp64/fp32 operands)
-  template <int STRIDE>
-  __device__ __forceinline__ void store_kmajor(T* S) const {
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int e = tid + GNT * i;
-      S[k_of(e) * STRIDE + row_of(e)] = v[i];
-    }
-  }
-};
-
-// Staging of one R x 16 FP64 operand tile in 16-byte vectors (two doubles
-// along the contiguous index), k range [k0, Kend):
-//   RC (rows contiguous): vector i of thread t holds rows 2 (t % (R/2)) + {0,1}
-//                         of k-row t / (R/2) + (2 GNT / R) i
-//   otherwise:            vector i holds k 2 (t % 8) + {0,1} of row t / 8 + 32 i
-// Load modes (uniform per work item and stage):
-//   LD_FULL  the tile lies inside the operand, 16-byte loads are aligned;
-//   LD_VPRED aligned, and the operand's extent along the vector is even, so a
-//            vector (even start) is wholly inside or wholly outside: one
-//            predicate per vector;
-//   LD_ELEM  each element loaded on its own.
-// Elements outside the operand read as PADV.
-enum { LD_FULL = 0, LD_VPRED = 1, LD_ELEM = 2 };
-template <int R, bool RC, bool NEGZ>
-struct GVecLoader {
-  static constexpr int BK = 16;
-  static constexpr int PER = R * BK / (2 * GNT);
-  static_assert(PER >= 1 && PER * 2 * GNT == R * BK, "tile must split into whole vectors per thread");
-  static constexpr double PADV = NEGZ ? -0.0 : 0.0;
-  typedef double V __attribute__((ext_vector_type(2)));
-  V v[PER];
-  int tid;
-  __device__ explicit GVecLoader(int t) : tid(t) {}
-  __device__ __forceinline__ int r_of(int i) const { return RC ? 2 * (tid % (R / 2)) : tid / 8 + (2 * GNT / BK) * i; }
-  __device__ __forceinline__ int k_of(int i) const { return RC ? tid / (R / 2) + (2 * GNT / R) * i : 2 * (tid % 8); }
-  // the mode of a stage: vec = aligned vectors, even = even extent along the vector
-  static __device__ __forceinline__ int mode(bool vec, bool even, bool full) {
-    return vec && full ? LD_FULL : (vec && even ? LD_VPRED : LD_ELEM);
-  }
-  // FULLPATH = false: LD_FULL is served by the predicated path (fewer live
-  // registers in a kernel at its register limit)
-  template <bool FULLPATH = true>
-  __device__ __forceinline__ void load(gptr<const double> P, int64_t ld, int64_t r0, int64_t k0, int64_t Rtot,
-                                       int64_t Kend, int md) {
-    if (FULLPATH && md == LD_FULL) {
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int64_t gr = r0 + r_of(i), gk = k0 + k_of(i);
-        v[i] = *(gptr<const V>)(RC ? P + gr + gk * ld : P + gk + gr * ld);
-      }
-    } else if (md != LD_ELEM) {
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int64_t gr = r0 + r_of(i), gk = k0 + k_of(i);
-        v[i] = (gr < Rtot && gk < Kend) ? *(gptr<const V>)(RC ? P + gr + gk * ld : P + gk + gr * ld)
-                                        : V{PADV, PADV};
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int64_t gr = r0 + r_of(i), gk = k0 + k_of(i);
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const int64_t r = RC ? gr + e : gr, k = RC ? gk : gk + e;
-          v[i][e] = (r < Rtot && k < Kend) ? (RC ? P[r + k * ld] : P[k + r * ld]) : PADV;
-        }
-      }
-    }
-  }
-  // k-major [k][row] at row stride STRIDE; SWZ (k-contiguous operands): row r
-  // of k-row k sits at column r ^ lswz(k), so the two k-rows of one store
-  // instruction's lanes fall in distinct banks.
-  template <int STRIDE, bool SWZ>
-  __device__ __forceinline__ void store(double* S) const {
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int r = r_of(i), k = k_of(i);
-      if (RC) {
-        *reinterpret_cast<V*>(S + k * STRIDE + r) = v[i];
-      } else {
-#pragma unroll
-        for (int e = 0; e < 2; ++e) S[(k + e) * STRIDE + (SWZ ? (r ^ lswz(k + e)) : r)] = v[i][e];
-      }
-    }
-  }
-  static __device__ __forceinline__ int lswz(int k) { return 4 * ((k >> 1) & 7); }
-};
-
-// The vector mode conditions of one operand: `vec` (16-byte aligned base, even
-// leading dimension) and `even` (even extent along the vector: rows for RC,
-// the k range end otherwise).
-template <bool RC>
-__device__ __forceinline__ void vec_conditions(const void* P, int64_t ld, int64_t rows, int64_t kend, bool& vec,
-                                               bool& even) {
-  vec = ((reinterpret_cast<uintptr_t>(P) & 15) == 0) && (ld % 2 == 0);
-  even = RC ? rows % 2 == 0 : kend % 2 == 0;
-}
-
-// Operand staging of the MFMA tiles: 16-byte vectors for FP64, elements for FP32.
-template <typename T, int R, bool RC, bool NEGZ>
-struct TileLoaderOf {
-  typedef GLoader<T, R, 16, RC, NEGZ> type;
-};
-template <int R, bool RC, bool NEGZ>
-struct TileLoaderOf<double, R, RC, NEGZ> {
-  typedef GVecLoader<R, RC, NEGZ> type;
-};
-
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-
-template <typename T> struct GMfma;
-template <> struct GMfma<double> {
-  typedef d4 acc_t;
-  static __device__ __forceinline__ acc_t mma(double x, double y, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int prow(int r, int g) { return 4 * r + g; }
-};
-template <> struct GMfma<float> {
-  typedef f4 acc_t;
-  static __device__ __forceinline__ acc_t mma(float x, float y, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int prow(int r, int g) { return 4 * g + r; }
-};
-
-// Result element (i, j) of tile (tm, tn): with one split it goes straight to
-// C through the alpha/beta epilogue, otherwise to this split's partial slab.
-template <typename T, int BM, int BN>
-__device__ __forceinline__ void put_result(const GProb& P, int tm, int tn, int split, int i, int j, T v) {
-  if (P.splitk == 1) {
-    const int64_t m = (int64_t)tm * BM + i, n = (int64_t)tn * BN + j;
-    if (m < P.m && n < P.n) {
-      gptr<T> C = as_global(static_cast<T*>(P.C));
-      T c;
-      if (P.k == 0) {  // no products (k == 0 or alpha == 0): C = beta*C, 0 for beta == 0
-        c = (T)P.beta != T(0) ? (T)P.beta * C[m + n * P.ldc] : T(0);
-      } else {
-        c = (T)P.alpha * v;
-        if ((T)P.beta != T(0)) c = fma((T)P.beta, C[m + n * P.ldc], c);
-      }
-      C[m + n * P.ldc] = c;
-    }
-  } else {
-    const int tile = tm * P.tiles_n + tn;
-    gptr<T> slab = as_global(static_cast<T*>(P.part)) + ((int64_t)tile * P.splitk + split) * (BM * BN);
-    slab[i + j * BM] = v;
-  }
-}
-
-// After every thread stored its partials: the last split of the tile to
-// arrive sums all partials in split order and applies the epilogue.
-template <typename T, int BM, int BN, int NTH = GNT>
-__device__ void splitk_combine(const GProb& P, int tm, int tn, int* counters, int* sflag) {
-  if (P.splitk == 1) return;
-  const int tile = tm * P.tiles_n + tn;
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) *sflag = atomicAdd(counters + P.counter_base + tile, 1);
-  __syncthreads();
-  if (*sflag != P.splitk - 1) return;  // not the last split of this tile
-  __threadfence();
-  gptr<const T> slab = as_global(static_cast<const T*>(P.part)) + ((int64_t)tile * P.splitk) * (BM * BN);
-  gptr<T> C = as_global(static_cast<T*>(P.C));
-  const T alpha = (T)P.alpha, beta = (T)P.beta;
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  for (int e = threadIdx.x; e < BM * BN; e += NTH) {
-    const int i = e % BM, j = e / BM;
-    const int64_t m = m0 + i, n = n0 + j;
-    if (m < P.m && n < P.n) {
-      T s = slab[e];
-      for (int q = 1; q < P.splitk; ++q) s += slab[(int64_t)q * (BM * BN) + e];
-      T c = alpha * s;
-      if (beta != T(0)) c = fma(beta, C[m + n * P.ldc], c);
-      C[m + n * P.ldc] = c;
-    }
-  }
-}
-
-// Native MFMA tile (T = double: f64 MFMA, T = float: f32 MFMA).
-template <typename T, int BM, int BN, bool TA, bool TB>
-__device__ void native_tile(const GProb& P, int tm, int tn, int split, char* smem, int* counters, int* sflag) {
-  constexpr int BK = 16;
-  constexpr int SA = BM + 16 / (int)sizeof(T) * 2, SB = BN + 16 / (int)sizeof(T) * 2;
-  constexpr int IM = BM / 32, JN = BN / 32;  // 16x16 blocks per wave (2 x 2 waves)
-  typedef typename GMfma<T>::acc_t acc_t;
-  T* As = reinterpret_cast<T*>(smem);
-  T* Bs = As + 2 * BK * SA;
-  const int tid = work_item_tid();
-  const int lane = tid % 64, wave = tid / 64;
-  const int wm0 = (wave % 2) * (BM / 2), wn0 = (wave / 2) * (BN / 2);
-  const int g = lane / 16, l16 = lane % 16;
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  const int64_t kb = (int64_t)split * P.kchunk;
-  const int64_t ke = min(P.k, kb + P.kchunk);
-  gptr<const T> A = as_global(static_cast<const T*>(P.A));
-  gptr<const T> B = as_global(static_cast<const T*>(P.B));
-  // op(A) rows contiguous when A is not transposed, op(B) columns when B is;
-  // FP64 operands travel in 16-byte vectors
-  typename TileLoaderOf<T, BM, !TA, sizeof(T) == 8>::type la(tid);
-  typename TileLoaderOf<T, BN, TB, false>::type lb(tid);
-  bool va, ea, vb, eb;
-  vec_conditions<!TA>(P.A, P.lda, P.m, ke, va, ea);
-  vec_conditions<TB>(P.B, P.ldb, P.n, ke, vb, eb);
-  const bool fa = m0 + BM <= P.m, fb = n0 + BN <= P.n;
-  auto load_stage = [&](int64_t k0) {
-    const bool fk = k0 + BK <= ke;
-    la.load(A, P.lda, m0, k0, P.m, ke, la.mode(va, ea, fa && fk));
-    lb.load(B, P.ldb, n0, k0, P.n, ke, lb.mode(vb, eb, fb && fk));
-  };
-  // FP64 chains start from -0.0 and A's k-padding is -0.0: the first step is
-  // exactly the plain product and padding products leave the chain unchanged,
-  // so each split is the reference recurrence bit for bit, zeros included.
-  constexpr T acc0 = sizeof(T) == 8 ? T(-0.0) : T(0);
-  acc_t acc[IM][JN];
-#pragma unroll
-  for (int i = 0; i < IM; ++i)
-#pragma unroll
-    for (int j = 0; j < JN; ++j) acc[i][j] = acc_t{acc0, acc0, acc0, acc0};
-  const int nkt = (int)((ke - kb + BK - 1) / BK);
-  __syncthreads();  // LDS may still be read by the previous work item
-  load_stage(kb);
-  la.template store<SA, false>(As);
-  lb.template store<SB, false>(Bs);
-  // Stage kt+1 travels in registers during stage kt: loaded right after stage
-  // kt went to LDS, stored to the other buffer before stage kt's last MFMA
-  // group, so a load has a whole stage to arrive and the LDS writes finish
-  // under MFMAs.
-  if (nkt > 1) load_stage(kb + BK);
-  __syncthreads();
-  for (int kt = 0; kt < nkt; ++kt) {
-    const int cur = kt & 1;
-    const T* as = As + cur * BK * SA;
-    const T* bs = Bs + cur * BK * SB;
-#pragma unroll
-    for (int t = 0; t < BK / 4; ++t) {
-      T a[IM], b[JN];
-#pragma unroll
-      for (int i = 0; i < IM; ++i) a[i] = as[(4 * t + g) * SA + wm0 + 16 * i + l16];
-#pragma unroll
-      for (int j = 0; j < JN; ++j) b[j] = bs[(4 * t + g) * SB + wn0 + 16 * j + l16];
-#pragma unroll
-      for (int i = 0; i < IM; ++i)
-#pragma unroll
-        for (int j = 0; j < JN; ++j) acc[i][j] = GMfma<T>::mma(b[j], a[i], acc[i][j]);
-      if (t == BK / 4 - 2 && kt + 1 < nkt) {
-        la.template store<SA, false>(As + (cur ^ 1) * BK * SA);
-        lb.template store<SB, false>(Bs + (cur ^ 1) * BK * SB);
-        if (kt + 2 < nkt) load_stage(kb + (int64_t)(kt + 2) * BK);
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < IM; ++i)
-#pragma unroll
-    for (int j = 0; j < JN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        put_result<T, BM, BN>(P, tm, tn, split, wm0 + 16 * i + l16, wn0 + 16 * j + GMfma<T>::prow(r, g), acc[i][j][r]);
-  splitk_combine<T, BM, BN>(P, tm, tn, counters, sflag);
-}
-
-// BM x BN FP64 tile (128x128, 128x64 or 64x128): four waves of (BM/2)x(BN/2)
-// (blocks of v_mfma_f64_16x16x4f64), 16 k per LDS stage, two LDS buffers,
-// the next stage's loads one stage ahead in registers.  Same chain semantics
-// as native_tile: chains start from -0.0, A's padding is -0.0, each k-split
-// is one fma chain in increasing k.
-template <int BM, int BN, bool TA, bool TB>
-__device__ void large_tile_f64(const GProb& P, int tm, int tn, int split, char* smem, int* counters, int* sflag) {
-  // LDS row strides extent + 16 doubles: lane groups g, g+1 of a fragment read start 32 banks apart
-  constexpr int BK = 16, STA = BM + 16, STB = BN + 16;
-  constexpr int IM = BM / 32, JN = BN / 32;
-  constexpr bool SWA = TA, SWB = !TB;  // k-contiguous operands are stored swizzled
-  double* const As = reinterpret_cast<double*>(smem);
-  double* const Bs = As + 2 * BK * STA;
-  const int tid = work_item_tid();
-  const int lane = tid % 64, wave = tid / 64;
-  const int wm0 = (wave % 2) * (BM / 2), wn0 = (wave / 2) * (BN / 2);
-  const int g = lane / 16, l16 = lane % 16;
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  const int64_t kb = (int64_t)split * P.kchunk;
-  const int64_t ke = min(P.k, kb + P.kchunk);
-  gptr<const double> A = as_global(static_cast<const double*>(P.A));
-  gptr<const double> B = as_global(static_cast<const double*>(P.B));
-  GVecLoader<BM, !TA, true> la(tid);
-  GVecLoader<BN, TB, false> lb(tid);
-  // 16-byte loads: aligned bases and even leading dimensions (k0 and the
-  // vectors' start rows are even)
-  bool va, ea, vb, eb;
-  vec_conditions<!TA>(P.A, P.lda, P.m, ke, va, ea);
-  vec_conditions<TB>(P.B, P.ldb, P.n, ke, vb, eb);
-  const bool fa = m0 + BM <= P.m, fb = n0 + BN <= P.n;
-  d4 acc[IM][JN];
-#pragma unroll
-  for (int i = 0; i < IM; ++i)
-#pragma unroll
-    for (int j = 0; j < JN; ++j) acc[i][j] = d4{-0.0, -0.0, -0.0, -0.0};
-  const int nkt = (int)((ke - kb + BK - 1) / BK);
-  auto load_stage = [&](int kt) {
-    const int64_t k0 = kb + (int64_t)kt * BK;
-    const bool fk = k0 + BK <= ke;
-    if (fa && fb && fk && va && vb) {
-      la.template load<true>(A, P.lda, m0, k0, P.m, ke, LD_FULL);
-      lb.template load<true>(B, P.ldb, n0, k0, P.n, ke, LD_FULL);
-    } else {
-      la.template load<false>(A, P.lda, m0, k0, P.m, ke, la.mode(va, ea, false));
-      lb.template load<false>(B, P.ldb, n0, k0, P.n, ke, lb.mode(vb, eb, false));
-    }
-  };
-  __syncthreads();  // LDS may still be read by the previous work item
-  load_stage(0);
-  la.template store<STA, SWA>(As);
-  lb.template store<STB, SWB>(Bs);
-  if (nkt > 1) load_stage(1);
-  __syncthreads();
-  // Swizzled column of (w0 + 16 i + l16) in k-row 4t + g: 16 ((w0/16 + i) ^ (t >> 1))
-  // + (l16 ^ (8 (t & 1) + 4 (g >> 1))) for t < 4 (w0 a multiple of 16).
-  const int sw0 = l16 ^ (4 * (g >> 1)), sw1 = l16 ^ (8 + 4 * (g >> 1));
-  const int bm0 = wm0 / 16, bn0 = wn0 / 16;
-  auto frags = [&](const double* as, const double* bs, int t, double (&a)[IM], double (&b)[JN]) {
-    const int swc = (t & 1) ? sw1 : sw0;
-#pragma unroll
-    for (int i = 0; i < IM; ++i)
-      a[i] = as[(4 * t + g) * STA + (SWA ? 16 * ((bm0 + i) ^ (t >> 1)) + swc : wm0 + 16 * i + l16)];
-#pragma unroll
-    for (int j = 0; j < JN; ++j)
-      b[j] = bs[(4 * t + g) * STB + (SWB ? 16 * ((bn0 + j) ^ (t >> 1)) + swc : wn0 + 16 * j + l16)];
-  };
-  for (int kt = 0; kt < nkt; ++kt) {
-    const int cur = kt & 1;
-    const double* as = As + cur * BK * STA;
-    const double* bs = Bs + cur * BK * STB;
-    double a[2][IM], b[2][JN];
-    frags(as, bs, 0, a[0], b[0]);
-#pragma unroll
-    for (int t = 0; t < BK / 4; ++t) {
-      if (t + 1 < BK / 4) frags(as, bs, t + 1, a[(t + 1) & 1], b[(t + 1) & 1]);
-#pragma unroll
-      for (int i = 0; i < IM; ++i)
-#pragma unroll
-        for (int j = 0; j < JN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[t & 1][j], a[t & 1][i], acc[i][j], 0, 0, 0);
-      if (t == BK / 4 - 2 && kt + 1 < nkt) {
-        la.template store<STA, SWA>(As + (cur ^ 1) * BK * STA);
-        lb.template store<STB, SWB>(Bs + (cur ^ 1) * BK * STB);
-        if (kt + 2 < nkt) load_stage(kt + 2);
-      }
-    }
-    __syncthreads();
-  }
-  // results: a 16-lane group holds 16 consecutive rows of one column
-  if (P.splitk == 1) {
-    gptr<double> C = as_global(static_cast<double*>(P.C));
-    const double alpha = P.alpha, beta = P.beta;
-#pragma unroll
-    for (int i = 0; i < IM; ++i) {
-      const int64_t m = m0 + wm0 + 16 * i + l16;
-      if (m >= P.m) continue;
-#pragma unroll
-      for (int j = 0; j < JN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int64_t n = n0 + wn0 + 16 * j + GMfma<double>::prow(r, g);
-          if (n < P.n) {  // as put_result: k == 0 (or alpha == 0) gives beta*C, +0 for beta == 0
-            gptr<double> c = C + m + n * P.ldc;
-            double v;
-            if (P.k == 0) v = beta != 0.0 ? beta * *c : 0.0;
-            else v = beta != 0.0 ? fma(beta, *c, alpha * acc[i][j][r]) : alpha * acc[i][j][r];
-            *c = v;
-          }
-        }
-    }
-  } else {
-    gptr<double> slab =
-        as_global(static_cast<double*>(P.part)) + ((int64_t)(tm * P.tiles_n + tn) * P.splitk + split) * (BM * BN);
-#pragma unroll
-    for (int i = 0; i < IM; ++i)
-#pragma unroll
-      for (int j = 0; j < JN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          slab[(wm0 + 16 * i + l16) + (wn0 + 16 * j + GMfma<double>::prow(r, g)) * BM] = acc[i][j][r];
-    splitk_combine<double, BM, BN>(P, tm, tn, counters, sflag);
-  }
-}
 
 // LDS rows of the 3xBF16 tile hold BK = 32 BF16 (64 bytes, four 16-byte chunks,
 // no padding); chunk c of row r is stored at chunk c ^ ((r >> 2) & 3), so the 16
@@ -714,7 +259,7 @@ __device__ void bf16x3_tile(const GProb& P, int tm, int tn, int split, char* sme
       for (int r = 0; r < 4; ++r)
         put_result<float, BM, BN>(P, tm, tn, split, wm0 + 16 * i + l16, wn0 + 16 * j + 4 * g + r,
                                   acc[0][i][j][r] + acc[1][i][j][r]);
-  splitk_combine<float, BM, BN>(P, tm, tn, counters, sflag);
+  splitk_combine<float, BM, GNT>(P, tm, tn, BN, counters, sflag);
 }
 
 // 3xBF16 tile of the 128-row/column shapes (128x128, 128x64, 64x128): WM x WN
@@ -831,7 +376,7 @@ __device__ void x3_large_tile(const GProb& P, int tm, int tn, int split, char* s
       for (int e = 0; e < 16; ++e)
         put_result<float, BM, BN>(P, tm, tn, split, wm0 + 32 * i + l32, wn0 + 32 * j + 8 * (e / 4) + 4 * hl + e % 4,
                                   acc[0][i][j][e] + acc[1][i][j][e]);
-  splitk_combine<float, BM, BN, NTH>(P, tm, tn, counters, sflag);
+  splitk_combine<float, BM, NTH>(P, tm, tn, BN, counters, sflag);
 }
 
 // Small problem (m, n, k <= 64) in one work item, the form of fastmul!
@@ -962,65 +507,28 @@ __device__ __forceinline__ void run_small(const GProb& P, int combo, char* smem)
   }
 }
 
-template <int KIND, int BM, bool TA, bool TB>
-__device__ __forceinline__ void run_tile(const GProb& P, int tm, int tn, int split, char* smem, int* counters,
-                                         int* sflag) {
-  if (KIND == 0) native_tile<double, BM, BM, TA, TB>(P, tm, tn, split, smem, counters, sflag);
-  else if (KIND == 1) native_tile<float, BM, BM, TA, TB>(P, tm, tn, split, smem, counters, sflag);
-  else bf16x3_tile<BM, BM, TA, TB>(P, tm, tn, split, smem, counters, sflag);
-}
-
-template <int KIND, int BM>
-__device__ __forceinline__ void run_combo(const GProb& P, int combo, int tm, int tn, int split, char* smem,
-                                          int* counters, int* sflag) {
+// The small items of the native methods (T = double or float), and the 3xBF16
+// method's 64x64, 32x32 and small items.
+template <int BM>
+__device__ __forceinline__ void run_x3_combo(const GProb& P, int combo, int tm, int tn, int split, char* smem,
+                                             int* counters, int* sflag) {
   switch (combo) {
-    case 0: run_tile<KIND, BM, false, false>(P, tm, tn, split, smem, counters, sflag); break;
-    case 1: run_tile<KIND, BM, false, true>(P, tm, tn, split, smem, counters, sflag); break;
-    case 2: run_tile<KIND, BM, true, false>(P, tm, tn, split, smem, counters, sflag); break;
-    default: run_tile<KIND, BM, true, true>(P, tm, tn, split, smem, counters, sflag); break;
+    case 0: bf16x3_tile<BM, BM, false, false>(P, tm, tn, split, smem, counters, sflag); break;
+    case 1: bf16x3_tile<BM, BM, false, true>(P, tm, tn, split, smem, counters, sflag); break;
+    case 2: bf16x3_tile<BM, BM, true, false>(P, tm, tn, split, smem, counters, sflag); break;
+    default: bf16x3_tile<BM, BM, true, true>(P, tm, tn, split, smem, counters, sflag); break;
   }
 }
 
-template <int KIND>
-__device__ __forceinline__ void dispatch_tile(const GProb& P, int combo, int tm, int tn, int split, char* smem,
-                                              int* counters, int* sflag) {
-  if (P.cfg == 0) run_combo<KIND, 64>(P, combo, tm, tn, split, smem, counters, sflag);
-  else if (P.cfg == 1) run_combo<KIND, 32>(P, combo, tm, tn, split, smem, counters, sflag);
-  else run_small<KIND>(P, combo, smem);
-}
-
-// Work queues of one persistent launch, one per XCD: queue x holds items
-// [qdesc[x], qdesc[x] + qdesc[NXCD + x]) of the launch's item array and is
-// drained through counter qnext[x].  Workgroups are dispatched to the XCDs
-// round-robin, so workgroup b pops from queue b % NXCD first: the tiles that
-// share operand panels were put in one queue and meet in one XCD's L2.  Once
-// its queue is drained a workgroup takes items from the others in turn.
-// Returns the item index, or -1 after every queue was found drained (each
-// workgroup then leaves; an item is taken exactly once, by the atomic on its
-// queue's counter).
-constexpr int NXCD = 8;
-__device__ __forceinline__ int pop_item(const int* __restrict__ qdesc, int* __restrict__ qnext, int& q, int& tries,
-                                        int* s_item) {
-  for (;;) {
-    if (threadIdx.x == 0) *s_item = atomicAdd(qnext + q, 1);
-    __syncthreads();
-    // uniform across the wave: descriptor loads become scalar loads into SGPRs
-    const int it = __builtin_amdgcn_readfirstlane(*s_item);
-    __syncthreads();
-    if (it < qdesc[NXCD + q]) return qdesc[q] + it;
-    if (++tries == NXCD) return -1;
-    q = (q + 1) % NXCD;
-  }
-}
-
-// KIND 0: FP64 native, 1: FP32 native, 2: FP32 3xBF16.
+// KIND 0: FP64 native, 1: FP32 native (small items only), 2: FP32 3xBF16.
 template <int KIND>
 __global__ __launch_bounds__(GNT, 2) void grouped_kernel(const GProb* __restrict__ probs, const GItem* __restrict__ items,
                                                          const int* __restrict__ qdesc, int* __restrict__ qnext,
                                                          int* __restrict__ counters) {
-  constexpr int SMEM = (KIND == 2) ? (2 * 3 * (64 + 64) * 32 * 2) : (2 * 16 * (64 + 8) * 2 * (KIND == 0 ? 8 : 4));
+  constexpr int E = KIND == 0 ? 8 : 4;
+  constexpr int SMEM = (KIND == 2) ? (2 * 3 * (64 + 64) * 32 * 2) : 64 * (64 + 16 / E) * E;
   __shared__ __attribute__((aligned(16))) char smem[SMEM];
-  static_assert(SMEM >= 64 * (64 + 16 / (KIND == 0 ? 8 : 4)) * (KIND == 0 ? 8 : 4), "small path stages op(B) in LDS");
+  static_assert(SMEM >= 64 * (64 + 16 / E) * E, "small path stages op(B) in LDS");
   __shared__ int s_item, s_flag;
   int q = blockIdx.x % NXCD, tries = 0;
   for (;;) {
@@ -1028,32 +536,15 @@ __global__ __launch_bounds__(GNT, 2) void grouped_kernel(const GProb* __restrict
     if (it < 0) break;
     const GItem w = items[it];
     const GProb P = probs[w.prob];
-    const int tm = w.tile / P.tiles_n, tn = w.tile % P.tiles_n;
     const int combo = (P.ta ? 2 : 0) + (P.tb ? 1 : 0);
-    dispatch_tile<KIND>(P, combo, tm, tn, w.split, smem, counters, &s_flag);
-  }
-}
-
-// The FP64 items of one 128-row/column tile shape and transpose combination,
-// pulled from their own queues (one kernel per shape and combination: a kernel
-// holding several tile variants exceeds the register budget of two
-// workgroups per CU).
-template <int BM, int BN, bool TA, bool TB>
-__global__ __launch_bounds__(GNT, 2) void grouped_large_kernel(const GProb* __restrict__ probs,
-                                                               const GItem* __restrict__ items,
-                                                               const int* __restrict__ qdesc, int* __restrict__ qnext,
-                                                               int* __restrict__ counters) {
-  constexpr int SMEM = 2 * 16 * ((BM + 16) + (BN + 16)) * 8;  // two buffers of A and B: 16 k-rows of stride extent + 16
-  __shared__ __attribute__((aligned(16))) char smem[SMEM];
-  __shared__ int s_item, s_flag;
-  int q = blockIdx.x % NXCD, tries = 0;
-  for (;;) {
-    const int it = pop_item(qdesc, qnext, q, tries, &s_item);
-    if (it < 0) break;
-    const GItem w = items[it];
-    const GProb P = probs[w.prob];
-    const int tm = w.tile / P.tiles_n, tn = w.tile % P.tiles_n;
-    large_tile_f64<BM, BN, TA, TB>(P, tm, tn, w.split, smem, counters, &s_flag);
+    if (KIND == 2 && P.cfg != CFG_SMALL) {
+      const int tm = w.tile / P.tiles_n, tn = w.tile % P.tiles_n;
+      if (P.cfg == 0) run_x3_combo<64>(P, combo, tm, tn, w.split, smem, counters, &s_flag);
+      else run_x3_combo<32>(P, combo, tm, tn, w.split, smem, counters, &s_flag);
+    } else {
+      __syncthreads();  // the previous item's op(B) may still be read
+      run_small<KIND>(P, combo, smem);
+    }
   }
 }
 
@@ -1193,16 +684,12 @@ bool choose(int method, int64_t m, int64_t n, int64_t k, int& cfg, int& splitk) 
 // ---------------------------------------------------------------------------
 // plans
 // ---------------------------------------------------------------------------
-// persistent launches of a plan: L = 4 (cfg - CFG_LARGE) + 2 ta + tb for the
-// 128-row/column FP64 tiles (one kernel per tile shape and transpose
-// combination), then the kernel of the other tiles
-constexpr int NLAUNCH = 13;
-
-// Relative duration of one work item of problem g (MFMA work of one k-split
-// of one tile plus a fixed epilogue share).
-double item_cost(const GProb& g) {
-  return (double)CFG_BM[g.cfg] * CFG_BN[g.cfg] * (double)std::max<int64_t>(g.kchunk, 32) + 4096.0;
-}
+// Persistent launches of a plan, by kernel.  Native methods: for each ring tile
+// (ring_of) and transpose combination one with 16-byte and one with 4-byte
+// operand loads, then one per combination for leading dimensions past 32-bit
+// offsets.  3xBF16: one per 128-row/column tile shape and combination (L < 12).
+// Last, one for the other items.
+constexpr int L_WIDE = 3 * 4 * 2, L_OTHER = L_WIDE + 4, NLAUNCH = L_OTHER + 1;
 
 // forced choice for the autotuner's trial launches: cfg >= 0 forces one choice
 // on every problem; otherwise `over` (bucket -> choice) is consulted before the table
@@ -1267,46 +754,77 @@ int validate_descs(int method, int64_t count, const jb_gemm_desc* d) {
 
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Resident workgroups per CU of a persistent kernel, from the device's
-// register and LDS budget for that kernel (queried once per kernel and device,
-// under the runtime lock; the persistent grid is this times the CU count).
-// kind 0-2: the kernel of the 64x64 / 32x32 / small items of method kind 0-2;
-// 3: the 128-row/column FP64 kernels (the 128x128 one's budget); 4: the
-// 128x128 3xBF16 kernels; 5: the 128x64 and 64x128 3xBF16 kernels.
-hipError_t grouped_occupancy(int kind, int* occ) {
-  static int cached[6] = {0, 0, 0, 0, 0, 0};
-  static int cached_device = -1;
-  if (cached_device != rt().device) {
-    for (int& c : cached) c = 0;
-    cached_device = rt().device;
-  }
-  if (cached[kind] == 0) {
-    int n = 0;
-    hipError_t e;
-    switch (kind) {
-      case 0: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, grouped_kernel<0>, GNT, 0); break;
-      case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, grouped_kernel<1>, GNT, 0); break;
-      case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, grouped_kernel<2>, GNT, 0); break;
-      case 3: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, grouped_large_kernel<128, 128, true, true>, GNT, 0); break;
-      case 4:
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, grouped_large_x3_kernel<128, 128, true, true>,
-                                                         X3Waves<128, 128>::NTH, 0);
-        break;
-      default: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, grouped_large_x3_kernel<128, 64, true, true>, GNT, 0); break;
-    }
-    if (e != hipSuccess) return e;
-    cached[kind] = std::min(std::max(n, 1), 8);
-  }
-  *occ = cached[kind];
-  return hipSuccess;
+// The kernel of launch L (see NLAUNCH) of a plan of method kind `kind`.
+GroupedKernel launch_kernel(int kind, int L) {
+  static const GroupedKernelFn x3[12] = {
+      grouped_large_x3_kernel<128, 128, false, false>, grouped_large_x3_kernel<128, 128, false, true>,
+      grouped_large_x3_kernel<128, 128, true, false>,  grouped_large_x3_kernel<128, 128, true, true>,
+      grouped_large_x3_kernel<128, 64, false, false>,  grouped_large_x3_kernel<128, 64, false, true>,
+      grouped_large_x3_kernel<128, 64, true, false>,   grouped_large_x3_kernel<128, 64, true, true>,
+      grouped_large_x3_kernel<64, 128, false, false>,  grouped_large_x3_kernel<64, 128, false, true>,
+      grouped_large_x3_kernel<64, 128, true, false>,   grouped_large_x3_kernel<64, 128, true, true>};
+  if (L == L_OTHER) return {kind == 0 ? grouped_kernel<0> : kind == 1 ? grouped_kernel<1> : grouped_kernel<2>, GNT};
+  if (kind == 2) return {x3[L], L < 4 ? X3Waves<128, 128>::NTH : GNT};
+  if (L >= L_WIDE) return {kind == 0 ? grouped_ring_f64_wide_ld(L - L_WIDE) : grouped_ring_f32_wide_ld(L - L_WIDE), GNT};
+  const int which = L / 8, combo = L / 2 % 4;
+  const bool vec = L % 2 == 0;
+  if (kind == 1) return {grouped_ring_f32(which, combo, vec), GNT};
+  return {vec ? grouped_ring_f64_vec(which, combo) : grouped_ring_f64(which, combo), GNT};
 }
 
-// The occupancy kind (grouped_occupancy) of launch L < NLAUNCH - 1 of a plan of
-// method kind `kind`, and of the 128-row/column kernels as a whole (L < 0: the
-// device fill of plan_choices).
-int large_occ_kind(int kind, int L) {
-  if (kind == 0) return 3;
-  return (L >= 0 && L < 4) ? 4 : 5;
+// Byte offsets inside an operand stage (up to 128 rows or 32 k of ld elements) past 32 bits.
+bool wide_ld(int kind, const GProb& g) {
+  const int64_t lim = ((int64_t)1 << 32) / (128 * (kind == 0 ? 8 : 4));
+  return kind != 2 && std::max(g.lda, g.ldb) >= lim;
+}
+
+// The ring tile (k_grouped_ring.h) of a native problem, and the extent of the work
+// items its tiles run in: FP64 64x64 and 32x32 tiles share 128x64 items.
+int ring_of(int kind, int cfg) { return kind == 1 ? (cfg == 1 ? 2 : 0) : (cfg == CFG_WIDE ? 1 : 0); }
+int item_rows(int kind, const GProb& g) { return kind == 0 && !wide_ld(kind, g) && g.cfg < 2 ? 128 : CFG_BM[g.cfg]; }
+int item_cols(int kind, const GProb& g) { return kind == 0 && !wide_ld(kind, g) && g.cfg < 2 ? 64 : CFG_BN[g.cfg]; }
+
+// The launch of problem g's items.
+int launch_of(int kind, const GProb& g) {
+  const int combo = 2 * g.ta + g.tb;
+  if (g.cfg == CFG_SMALL || (kind == 2 && !large_cfg(g.cfg))) return L_OTHER;
+  if (kind == 2) return 4 * (g.cfg - CFG_LARGE) + combo;
+  if (wide_ld(kind, g)) return L_WIDE + combo;
+  const int vw = kind == 0 ? 2 : 4;
+  const bool vec = ((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.B)) & 15) == 0 &&
+                   g.lda % vw == 0 && g.ldb % vw == 0 && (g.ta ? g.k : g.m) % vw == 0 &&
+                   (g.tb ? g.n : g.k) % vw == 0;
+  return 8 * ring_of(kind, g.cfg) + 2 * combo + (vec ? 0 : 1);
+}
+
+// Relative duration of one work item of problem g (MFMA work of one k-split of
+// one tile, of what reaches into C where the kernel skips the rest, plus a fixed
+// epilogue share).
+double item_cost(int kind, const GProb& g) {
+  const int64_t rows = item_rows(kind, g), cols = item_cols(kind, g);
+  const double area = kind == 2 ? (double)(rows * cols) : (double)(std::min(rows, g.m) * std::min(cols, g.n));
+  return area * (double)std::max<int64_t>(g.kchunk, 32) + 4096.0;
+}
+
+// Resident workgroups per CU of launch L's kernel, from the device's register and
+// LDS budget for it (queried once per kernel and device, under the runtime lock;
+// the persistent grid is this times the CU count).
+hipError_t grouped_occupancy(int kind, int L, int* occ) {
+  static int cached[3][NLAUNCH] = {};
+  static int cached_device = -1;
+  if (cached_device != rt().device) {
+    memset(cached, 0, sizeof cached);
+    cached_device = rt().device;
+  }
+  if (cached[kind][L] == 0) {
+    const GroupedKernel k = launch_kernel(kind, L);
+    int n = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(k.fn), k.threads, 0);
+    if (e != hipSuccess) return e;
+    cached[kind][L] = std::min(std::max(n, 1), 8);
+  }
+  *occ = cached[kind][L];
+  return hipSuccess;
 }
 
 // Builds the device-side problem/work lists of a plan (no launch).
@@ -1320,9 +838,11 @@ int large_occ_kind(int kind, int L) {
 int plan_choices(int method, int64_t count, const jb_gemm_desc* d, const Forced& forced, std::vector<GProb>& probs,
                  double* flops) {
   const int kind = kind_of(method);
+  // resident workgroups per CU: of the native methods' 128x64 (FP32: 64x64) tile
+  // kernel; 3xBF16: of the 64x64 / 32x32 kernel, and of the 128-row/column ones
   int occ = 0, occ_large = 1;
-  hipError_t e = grouped_occupancy(kind, &occ);
-  if (e == hipSuccess && kind != 1) e = grouped_occupancy(large_occ_kind(kind, -1), &occ_large);
+  hipError_t e = grouped_occupancy(kind, kind == 2 ? L_OTHER : 0, &occ);
+  if (e == hipSuccess && kind == 2) e = grouped_occupancy(kind, 4 * (CFG_TALL - CFG_LARGE), &occ_large);
   if (e != hipSuccess) return hip_fail(e, "grouped plan: occupancy query");
   std::vector<char> dflt;
   *flops = 0;
@@ -1362,24 +882,26 @@ int plan_choices(int method, int64_t count, const jb_gemm_desc* d, const Forced&
       }
     }
     fit_choice(kind, g.m, g.n, g.k, g.cfg, g.splitk);
-    g.tiles_m = (int)((g.m + CFG_BM[g.cfg] - 1) / CFG_BM[g.cfg]);
-    g.tiles_n = (int)((g.n + CFG_BN[g.cfg] - 1) / CFG_BN[g.cfg]);
+    if (g.cfg != CFG_SMALL && wide_ld(kind, g)) g.cfg = 0;
+    g.tiles_m = (int)((g.m + item_rows(kind, g) - 1) / item_rows(kind, g));
+    g.tiles_n = (int)((g.n + item_cols(kind, g) - 1) / item_cols(kind, g));
     *flops += 2.0 * (double)g.m * (double)g.n * (double)x.k;
     probs.push_back(g);
     dflt.push_back(is_default && g.cfg != CFG_SMALL);
   }
   const int64_t cus = rt().info.compute_units;
   const int64_t fill[2] = {cus * std::max(occ, 1), cus * std::max(occ_large, 1)};
-  int64_t items[2] = {0, 0};  // work items of the two persistent kernels
-  for (auto& g : probs) items[large_cfg(g.cfg)] += (int64_t)g.tiles_m * g.tiles_n * std::max(g.splitk, 1);
+  auto pool = [&](const GProb& g) { return kind == 2 && large_cfg(g.cfg) ? 1 : 0; };
+  int64_t items[2] = {0, 0};  // work items of each pool
+  for (auto& g : probs) items[pool(g)] += (int64_t)g.tiles_m * g.tiles_n * std::max(g.splitk, 1);
   for (;;) {
     int best = -1;
     double best_cost = 0;
     for (size_t i = 0; i < probs.size(); ++i) {
       const GProb& g = probs[i];
-      const int q = large_cfg(g.cfg);
+      const int q = pool(g);
       if (!dflt[i] || items[q] >= fill[q] || g.splitk >= 64 || g.k / (2 * g.splitk) < 256) continue;
-      const double cost = (double)CFG_BM[g.cfg] * CFG_BN[g.cfg] * (double)g.k / g.splitk;
+      const double cost = (double)item_rows(kind, g) * item_cols(kind, g) * (double)g.k / g.splitk;
       if (cost > best_cost) {
         best_cost = cost;
         best = (int)i;
@@ -1387,7 +909,7 @@ int plan_choices(int method, int64_t count, const jb_gemm_desc* d, const Forced&
     }
     if (best < 0) break;
     GProb& g = probs[best];
-    items[large_cfg(g.cfg)] += (int64_t)g.tiles_m * g.tiles_n * g.splitk;
+    items[pool(g)] += (int64_t)g.tiles_m * g.tiles_n * g.splitk;
     g.splitk *= 2;
   }
   // k per split: a multiple of 32, and no split comes out empty
@@ -1405,8 +927,6 @@ int plan_build(int method, int64_t count, const jb_gemm_desc* d, const Forced& f
   P.kind = kind_of(method);
   const size_t elt = P.kind == 0 ? 8 : 4;
   hipError_t e;
-  int occ = 0;
-  if ((e = grouped_occupancy(P.kind, &occ)) != hipSuccess) return hip_fail(e, "grouped plan: occupancy query");
   std::vector<GProb> probs;
   int rc = plan_choices(method, count, d, forced, probs, &P.flops);
   if (rc) return rc;
@@ -1423,9 +943,9 @@ int plan_build(int method, int64_t count, const jb_gemm_desc* d, const Forced& f
     if (g.splitk > 1) {
       counters += ntiles;
       part_off[pi] = part_elems;
-      part_elems += (size_t)ntiles * g.splitk * CFG_BM[g.cfg] * CFG_BN[g.cfg];
+      part_elems += (size_t)ntiles * g.splitk * item_rows(P.kind, g) * item_cols(P.kind, g);
     }
-    prob_cost[pi] = item_cost(g) * ntiles * g.splitk;
+    prob_cost[pi] = item_cost(P.kind, g) * ntiles * g.splitk;
     nall += (size_t)ntiles * g.splitk;
   }
   if (nall >= ((size_t)1 << 31) || (size_t)counters >= ((size_t)1 << 30))
@@ -1448,10 +968,10 @@ int plan_build(int method, int64_t count, const jb_gemm_desc* d, const Forced& f
   std::vector<GItem> seq;
   for (int pi : order) {
     const GProb& g = probs[pi];
-    const int L = large_cfg(g.cfg) ? 4 * (g.cfg - CFG_LARGE) + 2 * g.ta + g.tb : NLAUNCH - 1;
+    const int L = launch_of(P.kind, g);
     const int ntiles = g.tiles_m * g.tiles_n;
     const int nitems = ntiles * g.splitk;
-    const double c = item_cost(g);
+    const double c = item_cost(P.kind, g);
     const int per_run = (nitems + NXCD - 1) / NXCD;
     const int gr = std::max(1, std::min(g.tiles_m, (int)std::lround(std::sqrt((double)per_run))));
     seq.clear();
@@ -1512,8 +1032,8 @@ int plan_build(int method, int64_t count, const jb_gemm_desc* d, const Forced& f
       for (auto& w : q[L][x]) items.push_back(w.second);
       P.litems[L] += (int)q[L][x].size();
     }
-    int occ_l = occ;
-    if (L < NLAUNCH - 1 && P.litems[L] > 0 && (e = grouped_occupancy(large_occ_kind(P.kind, L), &occ_l)) != hipSuccess)
+    int occ_l = 1;
+    if (P.litems[L] > 0 && (e = grouped_occupancy(P.kind, L, &occ_l)) != hipSuccess)
       return hip_fail(e, "grouped plan: occupancy query");
     P.lgrid[L] = std::max(1, std::min(P.litems[L], cus * occ_l));
   }
@@ -1557,22 +1077,6 @@ int plan_build(int method, int64_t count, const jb_gemm_desc* d, const Forced& f
   return JB_OK;
 }
 
-typedef void (*GroupedKernelFn)(const GProb*, const GItem*, const int*, int*, int*);
-const GroupedKernelFn kLargeKernels[NLAUNCH - 1] = {
-    grouped_large_kernel<128, 128, false, false>, grouped_large_kernel<128, 128, false, true>,
-    grouped_large_kernel<128, 128, true, false>,  grouped_large_kernel<128, 128, true, true>,
-    grouped_large_kernel<128, 64, false, false>,  grouped_large_kernel<128, 64, false, true>,
-    grouped_large_kernel<128, 64, true, false>,   grouped_large_kernel<128, 64, true, true>,
-    grouped_large_kernel<64, 128, false, false>,  grouped_large_kernel<64, 128, false, true>,
-    grouped_large_kernel<64, 128, true, false>,   grouped_large_kernel<64, 128, true, true>};
-const GroupedKernelFn kLargeX3Kernels[NLAUNCH - 1] = {
-    grouped_large_x3_kernel<128, 128, false, false>, grouped_large_x3_kernel<128, 128, false, true>,
-    grouped_large_x3_kernel<128, 128, true, false>,  grouped_large_x3_kernel<128, 128, true, true>,
-    grouped_large_x3_kernel<128, 64, false, false>,  grouped_large_x3_kernel<128, 64, false, true>,
-    grouped_large_x3_kernel<128, 64, true, false>,   grouped_large_x3_kernel<128, 64, true, true>,
-    grouped_large_x3_kernel<64, 128, false, false>,  grouped_large_x3_kernel<64, 128, false, true>,
-    grouped_large_x3_kernel<64, 128, true, false>,   grouped_large_x3_kernel<64, 128, true, true>};
-
 // Enqueues [reset counters, 128-row/column persistent kernels, persistent kernel] on s.
 hipError_t plan_enqueue(const GroupedPlanImpl& P, hipStream_t s) {
   if (P.nitems == 0) return hipSuccess;
@@ -1592,18 +1096,8 @@ hipError_t plan_enqueue(const GroupedPlanImpl& P, hipStream_t s) {
     }
     const int* qd = P.qdesc + L * 2 * NXCD;
     int* qn = P.next + L * NXCD;
-    // the 128x128 3xBF16 kernels run workgroups of 8 waves
-    const dim3 grid(P.lgrid[L]), block(P.kind == 2 && L < 4 ? X3Waves<128, 128>::NTH : GNT);
-    if (L < NLAUNCH - 1) {
-      hipLaunchKernelGGL(P.kind == 0 ? kLargeKernels[L] : kLargeX3Kernels[L], grid, block, 0, ls, P.probs, P.items, qd, qn,
-                         tiles);
-    } else if (P.kind == 0) {
-      hipLaunchKernelGGL(grouped_kernel<0>, grid, block, 0, ls, P.probs, P.items, qd, qn, tiles);
-    } else if (P.kind == 1) {
-      hipLaunchKernelGGL(grouped_kernel<1>, grid, block, 0, ls, P.probs, P.items, qd, qn, tiles);
-    } else {
-      hipLaunchKernelGGL(grouped_kernel<2>, grid, block, 0, ls, P.probs, P.items, qd, qn, tiles);
-    }
+    const GroupedKernel k = launch_kernel(P.kind, L);
+    hipLaunchKernelGGL(k.fn, dim3(P.lgrid[L]), dim3(k.threads), 0, ls, P.probs, P.items, qd, qn, tiles);
     if (j >= 0) {
       if ((e = hipEventRecord(P.join[j], ls)) != hipSuccess) return e;
       if ((e = hipStreamWaitEvent(s, P.join[j], 0)) != hipSuccess) return e;

@@ -10,238 +10,31 @@
 // (2) dgemm_recurrence: one fma chain per element in increasing k, the exact
 //     order of src/gemm.jl:86 (first product) and :165 (fma k-step), on the
 //     vector ALUs: an independent restatement of (1)'s bits.
-#include "jb_internal.h"
+#include "jb_ring.h"
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
-#include <type_traits>
 
 namespace jb {
 namespace {
 
-typedef double d4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-
 // ---------------------------------------------------------------------------
-// (1) MFMA GEMM, T = double (v_mfma_f64_16x16x4f64) or float
-//     (v_mfma_f32_16x16x4f32).  Both instructions are a sequential fma chain
-//     over their four k values in lane-group order (checked on the device bit
-//     for bit, denormals and signed zeros included), so with lane group g
-//     supplying k = 4t+g every element is one fma chain in increasing k: the
-//     jmul! recurrence.
-//
-//     A block of WGM x WGN waves owns a BTM x BTN tile of C.  Operand stages of
-//     BK k stream through an LDS ring of NSLOT slots by direct global->LDS
-//     loads, NSLOT - 1 stages ahead, with one barrier per stage and an explicit
-//     vmcnt wait for the stage at hand (later stages stay in flight).
-//
-//     Bound: the matrix cores.  What kept them idle was vector instructions: an
-//     MFMA shares the wave's vector issue, and each address add or LDS store in the
-//     loop cost more matrix time than its own few cycles (8192^3 FP64 66.6 TF/s with
-//     register staging, the same with direct loads and 27 vector instructions per
-//     stage, 72.9 with the barrier inside the last MFMA group, 76.3 of 78.6 with
-//     none left).  So the loads are buffer loads (descriptor + scalar + lane
-//     offset, no arithmetic), the stages are unrolled over the ring (constant LDS
-//     offsets), and the next fragments are read behind the first MFMA row of a group.
-//     FP64, register-staged form -> this: 1024^3 TN 44.2 -> 35.2 us, 4096^3 64 -> 74
-//     TF/s, 2999x1777x2111 on odd leading dimensions 462 -> 382 us; FP32 8192^3 130
-//     -> 152 of 157 TF/s.
-//
-//     LDS images (no padding: the loads write 64 consecutive pieces):
-//       rows contiguous (A 'N', B 'T'): [k][R], row r of k-row k at r ^ rswz(k);
-//       k contiguous (A 'T', B 'N'):    [R][BK] in 16-byte chunks, chunk c of
-//                                       row r at c ^ cswz(r).
-//     The XORs spread the 16 rows and 4 k of one fragment read over all 64
-//     banks; the loads apply them to the global address of each lane.
-//
-//     VEC: 16 bytes per lane (16-byte aligned bases, leading dimensions and the
-//     contiguous extent multiples of the vector); otherwise 4 bytes per lane,
-//     which serves any size and leading dimension through the same LDS image.
-//     Rows past the operand read its last row again (those results are not
-//     stored).  A last stage shorter than BK reads clamped k, and the
-//     fragments replace it: -0.0 from A and +0.0 from B, whose product -0 leaves
-//     every chain value unchanged.
+// (1) MFMA GEMM: one block per tile of C (jb_ring.h).
 // ---------------------------------------------------------------------------
-template <typename T> struct Mfma;
-template <> struct Mfma<double> {
-  typedef d4 acc_t;
-  static __device__ __forceinline__ acc_t mma(double x, double y, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, c, 0, 0, 0);
-  }
-  // Row p of the 16x16 result held in item r of a lane of group g = lane/16.
-  static __device__ __forceinline__ int prow(int r, int g) { return 4 * r + g; }
-};
-template <> struct Mfma<float> {
-  typedef f4 acc_t;
-  static __device__ __forceinline__ acc_t mma(float x, float y, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int prow(int r, int g) { return 4 * g + r; }
-};
-
-// sched_barrier mask: vector and scalar ALU instructions may cross, memory instructions and MFMAs keep their order
-constexpr int SCHED_ALU = 6;
-#define JB_LDS __attribute__((address_space(3)))
-#define JB_INLINE __attribute__((always_inline))  // lambdas of the kernel: never outlined
-
-// One wave's load of 64 x LB bytes into LDS at dst, lane l's from base + so + vo (base and so wave-uniform).
-template <int LB>
-__device__ __forceinline__ void ring_load(gptr<const void> base, uint32_t vo, uint32_t so, char* dst) {
-#ifdef __HIP_DEVICE_COMPILE__  // the descriptor type exists on the device only
-  __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(const void*)base, 0, 0xffffffffu, 0x00027000);
-  if constexpr (LB == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (JB_LDS void*)dst, 16, vo, so, 0, 0);
-  else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (JB_LDS void*)dst, 4, vo, so, 0, 0);
-#endif
-}
-
-// One operand (R rows of op(A) or columns of op(B)) of the kernel below.
-//   RC: element (r, k) at P[r + k*ld], else at P[k + r*ld].
-//   WIDE: a lane's byte offset inside a stage may exceed 32 bits.
-template <typename T, int R, int BK, bool RC, bool VEC, int NW, bool WIDE>
-struct RingOperand {
-  static constexpr int EB = sizeof(T);
-  static constexpr int LB = VEC ? 16 : 4;                  // bytes per lane of one load
-  static constexpr int PB = 64 * LB;                       // bytes per load (one wave)
-  static constexpr int BYTES = R * BK * EB;                // one stage
-  static constexpr int NP = BYTES / PB / NW;               // loads per wave and stage
-  static_assert(NP >= 1 && NP * NW * PB == BYTES, "a stage must split into whole loads per wave");
-  static constexpr int ROWB = BK * EB;                     // k contiguous: bytes of one row,
-  static constexpr int CPR = ROWB / 16;                    // its 16-byte chunks,
-  static constexpr int RPB = ROWB < 256 ? 256 / ROWB : 1;  // and rows per 256 bytes (one pass over the banks)
-  static constexpr int EPL = PB / EB;                      // elements per load
-  static constexpr int KPL = EPL >= R ? EPL / R : 1;       // rows contiguous: k-rows per load,
-  static constexpr int LPK = EPL >= R ? 1 : R / EPL;       // or loads per k-row
-  static constexpr int RPL = ROWB <= PB ? PB / ROWB : 0;   // k contiguous: rows per load
-  static_assert(RC || RPL >= 1, "a load covers whole rows");
-  // The k-rows 4t..4t+3 of one fragment read must start 128 bytes (T = double,
-  // two per pass over the banks) or 64 bytes (T = float) apart.
-  static __device__ __forceinline__ int rswz(int k) {
-    if (EB == 8) return 16 * (k & 1);
-    return R >= 64 ? 16 * (k & 3) : 16 * ((k >> 1) & 1);
-  }
-  static_assert(!RC || R >= 32, "the row swizzle stays inside a k-row");
-  static __device__ __forceinline__ int cswz(int r) { return (r / RPB) & (CPR - 1); }
-
-  // LDS element of (r, k); r in [0, R), k in [0, BK)
-  static __device__ __forceinline__ int at(int r, int k) {
-    if (RC) return k * R + (r ^ rswz(k));
-    return r * BK + (((k * EB / 16) ^ cswz(r)) * 16 + (k * EB) % 16) / EB;
-  }
-
-  typedef typename std::conditional<WIDE, int64_t, uint32_t>::type Off;
-  Off off[NP];  // this lane's byte offset in load i of a stage, from the load's wave-uniform address
-  // ld: leading dimension; rmax: last row (vector start) that may be read, relative to the tile's first
-  __device__ __forceinline__ void init(int64_t ld, int rmax, int wave, int lane) {
-    const int lb = lane * LB;
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int p = wave + NW * i;
-      if (RC) {
-        const int kl = KPL > 1 ? (lb / EB) / R : 0, rl = (lb / EB) % (KPL > 1 ? R : EPL);
-        const int r = min(((p % LPK) * EPL + rl) ^ rswz(p * KPL / LPK + kl), rmax);
-        off[i] = (Off)r * EB + (Off)kl * (Off)ld * EB + lb % EB;
-      } else {
-        const int row = p * RPL + lb / ROWB;
-        const int k = (((lb % ROWB) / 16 ^ cswz(row)) * 16 + lb % 16) / EB;
-        off[i] = (Off)min(row, rmax) * (Off)ld * EB + k * EB + lb % EB;
-      }
-    }
-  }
-  // Load i of this wave's share of the stage at k0 into LDS at `dst` (the operand's part of a slot).
-  __device__ __forceinline__ void issue(gptr<const T> P, int64_t ld, int64_t k0, int wave, char* dst, int i) const {
-    const int p = wave + NW * i;
-    const int64_t k = RC ? p * KPL / LPK : 0;  // uniform: first k-row of the load
-    if constexpr (WIDE) {
-      put((gptr<const char>)(P + (RC ? (k0 + k) * ld : k0)) + off[i], dst + p * PB);
-    } else {
-      // A buffer load adds the stage's base (descriptor), the load's offset (scalar)
-      // and the lane's by itself: no vector address arithmetic is left in the loop
-      // (a vector instruction holds up the FP64 matrix pipe).
-      ring_load<LB>(P + (RC ? k0 * ld : k0), off[i], (uint32_t)k * (uint32_t)ld * EB, dst + p * PB);
-    }
-  }
-  // The same for the last stage, shorter than BK: k clamped to kmax (last vector start).
-  static __device__ __forceinline__ void issue_tail(gptr<const T> P, int64_t ld, int64_t k0, int rmax, int64_t kmax,
-                                                    int wave, int lane, char* dst, int i) {
-    asm volatile("" : "+v"(lane));  // the addresses are formed here, not ahead of the main loop
-    const int p = wave + NW * i, lb = lane * LB;
-    gptr<const T> src;
-    if (RC) {
-      const int kl = KPL > 1 ? (lb / EB) / R : 0, rl = (lb / EB) % (KPL > 1 ? R : EPL);
-      const int k = p * KPL / LPK + kl;
-      src = P + min(((p % LPK) * EPL + rl) ^ rswz(k), rmax) + min<int64_t>(k0 + k, kmax) * ld;
-    } else {
-      const int row = p * RPL + lb / ROWB;
-      const int k = (((lb % ROWB) / 16 ^ cswz(row)) * 16 + lb % 16) / EB;
-      src = P + (int64_t)min(row, rmax) * ld + min<int64_t>(k0 + k, kmax);
-    }
-    put((gptr<const char>)src + lb % EB, dst + p * PB);
-  }
-  static __device__ __forceinline__ void put(gptr<const char> src, char* dst) {
-    if constexpr (VEC) __builtin_amdgcn_global_load_lds((gptr<const void>)src, (JB_LDS void*)dst, 16, 0, 0);
-    else __builtin_amdgcn_global_load_lds((gptr<const void>)src, (JB_LDS void*)dst, 4, 0, 0);
-  }
-};
-
-// s_waitcnt: at most N vector-memory operations outstanding and every LDS read returned.
-template <int N>
-__device__ __forceinline__ void wait_ring() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
-}
-
-template <typename T, bool TA, bool TB, bool VEC, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK,
-          int NSLOT_, int MINW>
+template <typename T, bool TA, bool TB, bool VEC, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int NSLOT,
+          int MINW>
 __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
-    int64_t M, int64_t N, int64_t K, T alpha, const T* __restrict__ A_, int64_t lda, const T* __restrict__ B_, int64_t ldb,
+    int64_t M, int64_t N, int64_t K, T alpha, const T* __restrict__ A, int64_t lda, const T* __restrict__ B, int64_t ldb,
     T beta, T* __restrict__ C, int64_t ldc, int tiles_m, int tiles_n, int acc_from_c) {
-  constexpr int NW = WGM * WGN;
-  typedef RingOperand<T, BTM, BK, !TA, VEC, NW, WIDE> OA;
-  typedef RingOperand<T, BTN, BK, TB, VEC, NW, WIDE> OB;
-  constexpr int WIM = BTM / WGM / 16, WIN = BTN / WGN / 16;  // 16 x 16 MFMA blocks per wave along m, n
-  constexpr int STAGE_B = OA::BYTES + OB::BYTES;
-  constexpr int NLD = OA::NP + OB::NP;  // loads per wave and stage
-  constexpr int NSLOT = (NSLOT_ - 2) * NLD < 64 ? NSLOT_ : 63 / NLD + 2;  // the loads a wait leaves in flight fit its counter
-  constexpr int VW = VEC ? 16 / (int)sizeof(T) : 1;
-  constexpr int NT4 = BK / 4;  // MFMA k-groups per stage
-  static_assert(NT4 % 2 == 0, "the fragment buffers alternate over whole stages");
-  __shared__ __attribute__((aligned(1024))) char ring[NSLOT * STAGE_B];
-  typedef typename Mfma<T>::acc_t acc_t;
-  gptr<const T> A = as_global(A_), B = as_global(B_);
+  typedef RingTile<T, TA, TB, VEC, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT> Tile;
+  constexpr int WIM = Tile::WIM, WIN = Tile::WIN;
+  __shared__ __attribute__((aligned(1024))) char ring[Tile::SMEM];
 
   const int nblocks = tiles_m * tiles_n;
-  const int tile = xcd_remap(blockIdx.x, nblocks, 8);
   int tm, tn;
-  tile_coords(tile, tiles_m, tiles_n, 8, tm, tn);
+  tile_coords(xcd_remap(blockIdx.x, nblocks, 8), tiles_m, tiles_n, 8, tm, tn);
   const int64_t m0 = (int64_t)tm * BTM, n0 = (int64_t)tn * BTN;
-
-  const int lane = threadIdx.x % 64;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-  const int wm0 = (wave % WGM) * (BTM / WGM), wn0 = (wave / WGM) * (BTN / WGN);
-  const int g = lane / 16, l16 = lane % 16;
-
-  gptr<const T> At = A + (TA ? m0 * lda : m0), Bt = B + (TB ? n0 : n0 * ldb);
-  const int ramax = (int)min<int64_t>(M - m0 - (TA ? 1 : VW), BTM);
-  const int rbmax = (int)min<int64_t>(N - n0 - (TB ? VW : 1), BTN);
-  const int64_t kamax = K - (TA ? VW : 1), kbmax = K - (TB ? 1 : VW);
-  const int nst = (int)((K + BK - 1) / BK);
-  const int nfull = (int)(K / BK);
-  OA oa;
-  OB ob;
-  oa.init(lda, ramax, wave, lane);
-  ob.init(ldb, rbmax, wave, lane);
-  // load i of stage st; tail: the last stage, shorter than BK
-  auto issue = [&](int st, int slot, int i, auto tail) JB_INLINE {
-    char* dst = ring + slot * STAGE_B;
-    const int64_t k0 = (int64_t)st * BK;
-    if (decltype(tail)::value) {
-      if (i < OA::NP) OA::issue_tail(At, lda, k0, ramax, kamax, wave, lane, dst, i);
-      else OB::issue_tail(Bt, ldb, k0, rbmax, kbmax, wave, lane, dst + OA::BYTES, i - OA::NP);
-    } else {
-      if (i < OA::NP) oa.issue(At, lda, k0, wave, dst, i);
-      else ob.issue(Bt, ldb, k0, wave, dst + OA::BYTES, i - OA::NP);
-    }
-  };
+  Tile tile(ring, threadIdx.x);
 
   // Chains start from -0.0: the first MFMA step fma(a, x, -0.0) is then exactly
   // fl(a * x) for every input, the plain first product of the reference
@@ -251,159 +44,28 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
   // from the element of C instead, every k-step an fma; the caller passes
   // alpha = 1, beta = 0, so the epilogue stores the chain value itself.
   constexpr T acc0 = T(-0.0);
-  acc_t acc[WIM][WIN];
+  typename Tile::Acc acc;
 #pragma unroll
   for (int i = 0; i < WIM; ++i)
 #pragma unroll
-    for (int j = 0; j < WIN; ++j) acc[i][j] = acc_t{acc0, acc0, acc0, acc0};
+    for (int j = 0; j < WIN; ++j) acc[i][j] = typename Tile::acc_t{acc0, acc0, acc0, acc0};
   if (acc_from_c) {
 #pragma unroll
     for (int i = 0; i < WIM; ++i) {
-      const int64_t m = m0 + wm0 + 16 * i + l16;
+      const int64_t m = m0 + tile.row(i);
 #pragma unroll
       for (int j = 0; j < WIN; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int64_t n = n0 + wn0 + 16 * j + Mfma<T>::prow(r, g);
+          const int64_t n = n0 + tile.col(j, r);
           if (m < M && n < N) acc[i][j][r] = C[m + n * ldc];
         }
     }
   }
+  tile.begin(as_global(A) + (TA ? m0 * lda : m0), lda, as_global(B) + (TB ? n0 : n0 * ldb), ldb, M - m0, N - n0, K);
+  tile.run(acc);
 
-#pragma unroll
-  for (int d = 0; d < NSLOT; ++d)
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      if (d < nfull) issue(d, d, i, std::false_type());
-      else if (d < nst) issue(d, d, i, std::true_type());
-    }
-
-  T a[2][WIM], b[2][WIN];
-  auto frags = [&](int slot, int t, T (&x)[WIM], T (&y)[WIN]) JB_INLINE {
-    const T* as = reinterpret_cast<const T*>(ring + slot * STAGE_B);
-    const T* bs = reinterpret_cast<const T*>(ring + slot * STAGE_B + OA::BYTES);
-#pragma unroll
-    for (int i = 0; i < WIM; ++i) x[i] = as[OA::at(wm0 + 16 * i + l16, 4 * t + g)];
-#pragma unroll
-    for (int j = 0; j < WIN; ++j) y[j] = bs[OB::at(wn0 + 16 * j + l16, 4 * t + g)];
-  };
-  // Waits for this wave's loads of stage st (all but those of the later stages in
-  // flight) and its LDS reads, then for every wave.  A plain barrier: the fence of
-  // __syncthreads() would wait for all loads.
-  auto arrive = [&](int st, auto steady) JB_INLINE {
-    const int later = nst - 1 - st;
-    if (decltype(steady)::value || later >= NSLOT - 2) wait_ring<(NSLOT - 2) * NLD>();
-    else if (NSLOT >= 4 && later == NSLOT - 3) wait_ring<(NSLOT >= 4 ? NSLOT - 3 : 0) * NLD>();
-    else wait_ring<0>();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-  // Stage st in slot `slot`, whose first fragments are in a[0], b[0].  In its last
-  // MFMA group the block meets once: stage st + 1 has landed and every wave has
-  // read all of stage st, so its slot takes stage st + NSLOT and the next stage's
-  // first fragments are read while that group's MFMAs run.
-  // TAIL: the short last stage.  STEADY: stage st + NSLOT is a whole stage.
-  auto stage = [&](int st, int slot, int nslot, auto tail, auto steady) JB_INLINE {
-    constexpr bool TAIL = decltype(tail)::value, STEADY = decltype(steady)::value;
-#pragma unroll
-    for (int t = 0; t < NT4; ++t) {
-      const int cur = t & 1;
-      if (TAIL) {
-        const bool past = (int64_t)st * BK + 4 * t + g >= K;
-#pragma unroll
-        for (int i = 0; i < WIM; ++i) a[cur][i] = past ? T(-0.0) : a[cur][i];
-#pragma unroll
-        for (int j = 0; j < WIN; ++j) b[cur][j] = past ? T(0.0) : b[cur][j];
-      }
-      auto ahead = [&]() JB_INLINE {
-        if (t + 1 < NT4) {
-          frags(slot, t + 1, a[cur ^ 1], b[cur ^ 1]);
-        } else if (STEADY || st + 1 < nst) {
-          arrive(st + 1, steady);
-          frags(nslot, 0, a[cur ^ 1], b[cur ^ 1]);
-        }
-        __builtin_amdgcn_sched_barrier(SCHED_ALU);
-      };
-      // The next group's fragments are read behind the first row of MFMAs (whose
-      // wait for this group's then covers nothing else).
-      if (WIM == 1) ahead();
-      // D'[p][q] = sum_k X[p][k] Y[k][q] with X = op(B)^T block (p -> n) and Y = op(A)^T
-      // block (q -> m), so a 16-lane group holds 16 consecutive rows of one column of C
-      // (coalesced column-major stores).
-#pragma unroll
-      for (int i = 0; i < WIM; ++i) {
-#pragma unroll
-        for (int j = 0; j < WIN; ++j) acc[i][j] = Mfma<T>::mma(b[cur][j], a[cur][i], acc[i][j]);
-        __builtin_amdgcn_sched_barrier(SCHED_ALU);
-        if (i == 0 && WIM > 1) ahead();
-        if (t + 1 == NT4) {
-          constexpr int PI = (NLD + WIM - 1) / WIM;
-#pragma unroll
-          for (int q = PI * i; q < PI * (i + 1) && q < NLD; ++q) {
-            if (STEADY) issue(st + NSLOT, slot, q, std::false_type());
-            else if (!TAIL && st + NSLOT < nfull) issue(st + NSLOT, slot, q, std::false_type());
-            else if (!TAIL && st + NSLOT < nst) issue(st + NSLOT, slot, q, std::true_type());
-          }
-        }
-      }
-      __builtin_amdgcn_sched_barrier(SCHED_ALU);
-    }
-  };
-  arrive(0, std::false_type());
-  frags(0, 0, a[0], b[0]);
-  int st = 0, slot = 0, nslot = 1;
-  auto next = [&]() JB_INLINE {
-    ++st;
-    slot = nslot;
-    nslot = nslot + 1 == NSLOT ? 0 : nslot + 1;
-  };
-  // unrolled over the ring, so that every LDS address is a constant offset from a few lane registers
-  for (; st + 2 * NSLOT - 1 < nfull; st += NSLOT)
-#pragma unroll
-    for (int d = 0; d < NSLOT; ++d)
-      stage(st + d, d, d + 1 == NSLOT ? 0 : d + 1, std::false_type(), std::true_type());
-  for (; st < nfull; next()) stage(st, slot, nslot, std::false_type(), std::false_type());
-  if (st < nst) stage(st, slot, nslot, std::true_type(), std::false_type());
-
-  if (m0 + BTM <= M && n0 + BTN <= N) {
-    // Interior tile: for each 16-row strip, the beta*C loads are issued
-    // together, then the results stored.
-#pragma unroll
-    for (int i = 0; i < WIM; ++i) {
-      T* Ci = C + (m0 + wm0 + 16 * i + l16);
-      T cv[WIN][4];
-#pragma unroll
-      for (int j = 0; j < WIN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          cv[j][r] = beta != T(0) ? Ci[(n0 + wn0 + 16 * j + Mfma<T>::prow(r, g)) * ldc] : T(0);
-#pragma unroll
-      for (int j = 0; j < WIN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          T c = alpha * acc[i][j][r];
-          if (beta != T(0)) c = fma(beta, cv[j][r], c);
-          Ci[(n0 + wn0 + 16 * j + Mfma<T>::prow(r, g)) * ldc] = c;
-        }
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < WIM; ++i) {
-    const int64_t m = m0 + wm0 + 16 * i + l16;
-#pragma unroll
-    for (int j = 0; j < WIN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t n = n0 + wn0 + 16 * j + Mfma<T>::prow(r, g);
-        if (m < M && n < N) {
-          T c = alpha * acc[i][j][r];
-          if (beta != T(0)) c = fma(beta, C[m + n * ldc], c);
-          C[m + n * ldc] = c;
-        }
-      }
-  }
+  tile.store(acc, C + m0 + n0 * ldc, ldc, M - m0, N - n0, alpha, beta);
 }
 
 // ---------------------------------------------------------------------------
