@@ -827,23 +827,21 @@ hipError_t grouped_occupancy(int kind, int L, int* occ) {
   return hipSuccess;
 }
 
-// Builds the device-side problem/work lists of a plan (no launch).
+// Workgroups per CU up to which a group is split along k (plan_choices): of the
+// 64x64 / 32x32 tiles, and of the 128-row/column tiles, per method kind.  More than
+// the MFMA tiles' residency: shorter chains also round less, and these depths are
+// the ones the methods' accuracy was measured with.
+constexpr int FILL[3][2] = {{4, 2}, {8, 8}, {3, 2}};
+
 // Tile and split of every problem with m, n > 0 (in order), the plan's first
 // two passes: the table / tuner / static choice per problem, then the device
-// fill: while a persistent kernel (the 128x128 one, or the one for the other
-// tiles) has fewer work items than the device holds of its resident
-// workgroups (compute units x that kernel's occupancy), the split of its
-// statically chosen problem with the longest work items doubles, down to 256 k
-// per split.  Last, each split's k range is fixed.  flops: sum of 2 m n k.
+// fill: while the group has fewer tiles than FILL workgroups per compute unit (the
+// 128-row/column tiles and the others counted apart), the split of its statically
+// chosen problem with the longest tiles doubles, down to 256 k per split.  Last,
+// each split's k range is fixed.  flops: sum of 2 m n k.
 int plan_choices(int method, int64_t count, const jb_gemm_desc* d, const Forced& forced, std::vector<GProb>& probs,
                  double* flops) {
   const int kind = kind_of(method);
-  // resident workgroups per CU: of the native methods' 128x64 (FP32: 64x64) tile
-  // kernel; 3xBF16: of the 64x64 / 32x32 kernel, and of the 128-row/column ones
-  int occ = 0, occ_large = 1;
-  hipError_t e = grouped_occupancy(kind, kind == 2 ? L_OTHER : 0, &occ);
-  if (e == hipSuccess && kind == 2) e = grouped_occupancy(kind, 4 * (CFG_TALL - CFG_LARGE), &occ_large);
-  if (e != hipSuccess) return hip_fail(e, "grouped plan: occupancy query");
   std::vector<char> dflt;
   *flops = 0;
   for (int64_t i = 0; i < count; ++i) {
@@ -883,25 +881,24 @@ int plan_choices(int method, int64_t count, const jb_gemm_desc* d, const Forced&
     }
     fit_choice(kind, g.m, g.n, g.k, g.cfg, g.splitk);
     if (g.cfg != CFG_SMALL && wide_ld(kind, g)) g.cfg = 0;
-    g.tiles_m = (int)((g.m + item_rows(kind, g) - 1) / item_rows(kind, g));
-    g.tiles_n = (int)((g.n + item_cols(kind, g) - 1) / item_cols(kind, g));
     *flops += 2.0 * (double)g.m * (double)g.n * (double)x.k;
     probs.push_back(g);
     dflt.push_back(is_default && g.cfg != CFG_SMALL);
   }
   const int64_t cus = rt().info.compute_units;
-  const int64_t fill[2] = {cus * std::max(occ, 1), cus * std::max(occ_large, 1)};
-  auto pool = [&](const GProb& g) { return kind == 2 && large_cfg(g.cfg) ? 1 : 0; };
-  int64_t items[2] = {0, 0};  // work items of each pool
-  for (auto& g : probs) items[pool(g)] += (int64_t)g.tiles_m * g.tiles_n * std::max(g.splitk, 1);
+  auto tiles = [](const GProb& g) {
+    return (g.m + CFG_BM[g.cfg] - 1) / CFG_BM[g.cfg] * ((g.n + CFG_BN[g.cfg] - 1) / CFG_BN[g.cfg]);
+  };
+  int64_t items[2] = {0, 0};
+  for (auto& g : probs) items[large_cfg(g.cfg)] += tiles(g) * std::max(g.splitk, 1);
   for (;;) {
     int best = -1;
     double best_cost = 0;
     for (size_t i = 0; i < probs.size(); ++i) {
       const GProb& g = probs[i];
-      const int q = pool(g);
-      if (!dflt[i] || items[q] >= fill[q] || g.splitk >= 64 || g.k / (2 * g.splitk) < 256) continue;
-      const double cost = (double)item_rows(kind, g) * item_cols(kind, g) * (double)g.k / g.splitk;
+      const int q = large_cfg(g.cfg);
+      if (!dflt[i] || items[q] >= cus * FILL[kind][q] || g.splitk >= 64 || g.k / (2 * g.splitk) < 256) continue;
+      const double cost = (double)CFG_BM[g.cfg] * CFG_BN[g.cfg] * (double)g.k / g.splitk;
       if (cost > best_cost) {
         best_cost = cost;
         best = (int)i;
@@ -909,7 +906,7 @@ int plan_choices(int method, int64_t count, const jb_gemm_desc* d, const Forced&
     }
     if (best < 0) break;
     GProb& g = probs[best];
-    items[pool(g)] += (int64_t)g.tiles_m * g.tiles_n * g.splitk;
+    items[large_cfg(g.cfg)] += tiles(g) * g.splitk;
     g.splitk *= 2;
   }
   // k per split: a multiple of 32, and no split comes out empty
@@ -918,6 +915,8 @@ int plan_choices(int method, int64_t count, const jb_gemm_desc* d, const Forced&
     kc = std::max<int64_t>(32, (kc + 31) / 32 * 32);
     g.splitk = g.k == 0 ? 1 : (int)std::max<int64_t>(1, (g.k + kc - 1) / kc);
     g.kchunk = kc;
+    g.tiles_m = (int)((g.m + item_rows(kind, g) - 1) / item_rows(kind, g));
+    g.tiles_n = (int)((g.n + item_cols(kind, g) - 1) / item_cols(kind, g));
   }
   return JB_OK;
 }
