@@ -41,14 +41,14 @@ hipError_t launch_fastmul_f32(int64_t M, int64_t N, int64_t P, float* D, const f
 size_t ozaki_workspace_bytes(int64_t m, int64_t n, int64_t k, int s);
 // Split + slice-pair GEMM + compensated combine.  `ws` is device memory of
 // ozaki_workspace_bytes().  A row of op(A) or column of op(B) holding Inf or
-// NaN makes the C elements it feeds NaN and sets two device ints to 1: this
-// call's flag, an int at byte offset emulated_flag_offset() of `ws` (cleared
+// NaN makes the C elements it feeds NaN and sets two device ints to 1: with
+// `want_flag` this call's, an int at byte offset emulated_flag_offset() of `ws` (cleared
 // by the call itself), and `sticky`, which the call never clears.  No host
 // synchronisation.
-hipError_t launch_dgemm_ozaki(const GemmArgs& g, int s, void* ws, int* sticky, hipStream_t st);
+hipError_t launch_dgemm_ozaki(const GemmArgs& g, int s, void* ws, bool want_flag, int* sticky, hipStream_t st);
 // The same with INT8 slices (v_mfma_i32_32x32x32_i8, exact int32 level sums).
 size_t ozaki_i8_workspace_bytes(int64_t m, int64_t n, int64_t k, int s);
-hipError_t launch_dgemm_ozaki_i8(const GemmArgs& g, int s, void* ws, int* sticky, hipStream_t st);
+hipError_t launch_dgemm_ozaki_i8(const GemmArgs& g, int s, void* ws, bool want_flag, int* sticky, hipStream_t st);
 // Byte offset of the call's non-finite flag in the workspace of the emulated
 // DGEMM (BF16 or INT8 slices) and of the 3xBF16 SGEMM (whose planes have their
 // own layout).
@@ -61,7 +61,7 @@ hipError_t launch_sgemm_mfma(const GemmArgs& g, hipStream_t s);
 size_t bf16x3_workspace_bytes(int64_t m, int64_t n, int64_t k);
 // Non-finite inputs become NaN slices (every product they enter is NaN) and set
 // the two flags as in launch_dgemm_ozaki.
-hipError_t launch_sgemm_bf16x3(const GemmArgs& g, int nprod, void* ws, int* sticky, hipStream_t s);
+hipError_t launch_sgemm_bf16x3(const GemmArgs& g, int nprod, void* ws, bool want_flag, int* sticky, hipStream_t s);
 
 // ---- generator ------------------------------------------------------------
 hipError_t launch_fill_uniform(uint64_t seed, int64_t n, double* out, hipStream_t s);

@@ -718,7 +718,8 @@ static int ozaki_dev_locked(const GemmArgs& g, int s, bool i8, hipStream_t st, i
   void* ws = nullptr;
   int rc = ws_acquire(i8 ? ozaki_i8_workspace_bytes(g.m, g.n, g.k, s) : ozaki_workspace_bytes(g.m, g.n, g.k, s), st, &ws);
   if (rc) return rc;
-  hipError_t e = i8 ? launch_dgemm_ozaki_i8(g, s, ws, rt().sticky, st) : launch_dgemm_ozaki(g, s, ws, rt().sticky, st);
+  hipError_t e = i8 ? launch_dgemm_ozaki_i8(g, s, ws, host_flag != nullptr, rt().sticky, st)
+                    : launch_dgemm_ozaki(g, s, ws, host_flag != nullptr, rt().sticky, st);
   if (e == hipSuccess && host_flag)
     e = hipMemcpyAsync(host_flag, static_cast<char*>(ws) + emulated_flag_offset(g.m, g.n, g.k, s, i8), sizeof(int),
                        hipMemcpyDeviceToHost, st);
@@ -770,7 +771,7 @@ int jb_dgemm_ozaki_noalloc_dev(char transA, char transB, int64_t m, int64_t n, i
     e = launch_scale_f64(m, n, beta, C, ldc, st);
   } else {
     tl_no_timing = true;
-    e = launch_dgemm_ozaki(g, nslices, sp + JB_SCRATCH_HEADER, reinterpret_cast<int*>(sp), st);
+    e = launch_dgemm_ozaki(g, nslices, sp + JB_SCRATCH_HEADER, false, reinterpret_cast<int*>(sp), st);
     tl_no_timing = false;
   }
   return e == hipSuccess ? JB_OK : hip_fail(e, "dgemm_ozaki (allocation-free) launch");
@@ -821,7 +822,7 @@ static int sgemm_dev_locked(const GemmArgs& g, int method, int nprod, hipStream_
   void* ws = nullptr;
   int rc = ws_acquire(bf16x3_workspace_bytes(g.m, g.n, g.k), s, &ws);
   if (rc) return rc;
-  e = launch_sgemm_bf16x3(g, nprod, ws, rt().sticky, s);
+  e = launch_sgemm_bf16x3(g, nprod, ws, host_flag != nullptr, rt().sticky, s);
   if (e == hipSuccess && host_flag)
     e = hipMemcpyAsync(host_flag, static_cast<char*>(ws) + bf16x3_flag_offset(g.m, g.n, g.k), sizeof(int),
                        hipMemcpyDeviceToHost, s);

@@ -114,11 +114,11 @@ __device__ __forceinline__ unsigned long long abs_bits(double x) {
   return (unsigned long long)__double_as_longlong(fabs(x));
 }
 
-__global__ __launch_bounds__(256) void absmax_rows_kernel(const double* __restrict__ P, int64_t sk, int64_t R,
-                                                          int64_t K, unsigned long long* __restrict__ maxbits) {
-  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void absmax_rows(const double* __restrict__ P, int64_t sk, int64_t R, int64_t K,
+                                            unsigned long long* __restrict__ maxbits, int64_t bx, int64_t by) {
+  const int64_t r = bx * 256 + threadIdx.x;
   if (r >= R) return;
-  const int64_t k0 = (int64_t)blockIdx.y * AM_RKC;
+  const int64_t k0 = by * AM_RKC;
   const int64_t nk = min<int64_t>(AM_RKC, K - k0);
   const double* __restrict__ p = P + r + k0 * sk;
   unsigned long long m = 0ull;
@@ -134,12 +134,11 @@ __global__ __launch_bounds__(256) void absmax_rows_kernel(const double* __restri
   atomicMax(maxbits + r, m);
 }
 
-__global__ __launch_bounds__(256) void absmax_kcontig_kernel(const double* __restrict__ P, int64_t sr, int64_t sk,
-                                                             int64_t R, int64_t K,
-                                                             unsigned long long* __restrict__ maxbits) {
+__device__ __forceinline__ void absmax_kcontig(const double* __restrict__ P, int64_t sr, int64_t sk, int64_t R, int64_t K,
+                                               unsigned long long* __restrict__ maxbits, int64_t bx, int64_t by) {
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int64_t rw = (int64_t)blockIdx.x * (4 * AM_WROWS) + (int64_t)wave * AM_WROWS;
-  const int64_t k0 = (int64_t)blockIdx.y * AM_KK;
+  const int64_t rw = bx * (4 * AM_WROWS) + (int64_t)wave * AM_WROWS;
+  const int64_t k0 = by * AM_KK;
 #pragma unroll 2
   for (int i = 0; i < AM_WROWS; ++i) {
     const int64_t r = rw + i;
@@ -160,12 +159,12 @@ __global__ __launch_bounds__(256) void absmax_kcontig_kernel(const double* __res
 // k contiguous with unit stride, 16-byte aligned rows: each lane loads two
 // doubles per instruction, four rows' loads in flight per wave (the general
 // form above issues 8-byte loads through a runtime stride).
-__global__ __launch_bounds__(256) void absmax_kunit_kernel(const double* __restrict__ P, int64_t sr, int64_t R,
-                                                           int64_t K, unsigned long long* __restrict__ maxbits) {
+__device__ __forceinline__ void absmax_kunit(const double* __restrict__ P, int64_t sr, int64_t R, int64_t K,
+                                             unsigned long long* __restrict__ maxbits, int64_t bx, int64_t by) {
   typedef double V2 __attribute__((ext_vector_type(2)));
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int64_t rw = (int64_t)blockIdx.x * (4 * AM_WROWS) + (int64_t)wave * AM_WROWS;
-  const int64_t k0 = (int64_t)blockIdx.y * AM_KK;
+  const int64_t rw = bx * (4 * AM_WROWS) + (int64_t)wave * AM_WROWS;
+  const int64_t k0 = by * AM_KK;
   const bool full = k0 + AM_KK <= K;
   for (int i0 = 0; i0 < AM_WROWS; i0 += 4) {
     unsigned long long m[4] = {0ull, 0ull, 0ull, 0ull};
@@ -196,20 +195,31 @@ __global__ __launch_bounds__(256) void absmax_kunit_kernel(const double* __restr
   }
 }
 
-void launch_absmax(const double* P, int64_t sr, int64_t sk, int64_t R, int64_t K, unsigned long long* mb,
-                   hipStream_t st) {
-  if (R <= 0 || K <= 0) return;
-  if (sr != 1 && sk == 1 && (reinterpret_cast<uintptr_t>(P) & 15) == 0 && sr % 2 == 0)
-    hipLaunchKernelGGL(absmax_kunit_kernel,
-                       dim3((unsigned)((R + 4 * AM_WROWS - 1) / (4 * AM_WROWS)), (unsigned)((K + AM_KK - 1) / AM_KK)),
-                       dim3(256), 0, st, P, sr, R, K, mb);
-  else if (sr == 1)
-    hipLaunchKernelGGL(absmax_rows_kernel, dim3((unsigned)((R + 255) / 256), (unsigned)((K + AM_RKC - 1) / AM_RKC)),
-                       dim3(256), 0, st, P, sk, R, K, mb);
-  else
-    hipLaunchKernelGGL(absmax_kcontig_kernel,
-                       dim3((unsigned)((R + 4 * AM_WROWS - 1) / (4 * AM_WROWS)), (unsigned)((K + AM_KK - 1) / AM_KK)),
-                       dim3(256), 0, st, P, sr, sk, R, K, mb);
+// One operand of the split phase: op(A) rows (or op(B) columns) X(r, k) = P[r*sr + k*sk].
+template <typename T, typename D>
+struct SplitOperand {
+  const T* P;
+  int64_t sr, sk, R, Rpad;
+  D* planes;
+  int RB;                       // row block of the planes
+  unsigned long long* maxbits;  // FP64: of each row,
+  int* exps;                    // and its exponent
+  int64_t ax, ay;               // FP64: absmax blocks along rows and k
+};
+
+// Both operands' absmax in one launch (one dimension: A's blocks, then B's): a small
+// problem's two launches and the gap between them cost as much as the work.
+template <typename D>
+__global__ __launch_bounds__(256) void absmax_kernel(SplitOperand<double, D> a, SplitOperand<double, D> b, int64_t K) {
+  int64_t id = blockIdx.x;
+  const bool isb = id >= a.ax * a.ay;
+  const SplitOperand<double, D>& o = isb ? b : a;
+  if (isb) id -= a.ax * a.ay;
+  const int64_t bx = id % o.ax, by = id / o.ax;
+  if (o.sr != 1 && o.sk == 1 && (reinterpret_cast<uintptr_t>(o.P) & 15) == 0 && o.sr % 2 == 0)
+    absmax_kunit(o.P, o.sr, o.R, K, o.maxbits, bx, by);
+  else if (o.sr == 1) absmax_rows(o.P, o.sk, o.R, K, o.maxbits, bx, by);
+  else absmax_kcontig(o.P, o.sr, o.sk, o.R, K, o.maxbits, bx, by);
 }
 
 __global__ void zero_u64_kernel(unsigned long long* p, int64_t n) {
@@ -227,14 +237,20 @@ __device__ __forceinline__ uint16_t bf16_bits_exact(double d) {
 //     the padded Rpad x Kpad extent in 64 x 64 tiles; RB divides by 64.
 // ---------------------------------------------------------------------------
 template <int S>
-__global__ __launch_bounds__(256) void split_f64_kernel(const double* __restrict__ P, int64_t sr, int64_t sk, int64_t R,
-                                                        int64_t K, const unsigned long long* __restrict__ maxbits,
-                                                        int* __restrict__ exps, uint16_t* __restrict__ planes,
-                                                        int64_t plane_stride, int64_t Kpad, int RB,
-                                                        int* __restrict__ call_flag, int* __restrict__ sticky) {
+__global__ __launch_bounds__(256) void split_f64_kernel(SplitOperand<double, uint16_t> oa, SplitOperand<double, uint16_t> ob, int64_t K,
+                                              int64_t Kpad, int* __restrict__ call_flag, int* __restrict__ sticky) {
   __shared__ double tile[64][65];
   const int t = threadIdx.x;
-  const int64_t r0 = (int64_t)blockIdx.x * 64, k0 = (int64_t)blockIdx.y * 64;
+  // blocks along x: op(A)'s row tiles, then op(B)'s
+  const bool isb = (int64_t)blockIdx.x * 64 >= oa.Rpad;
+  const SplitOperand<double, uint16_t>& o = isb ? ob : oa;
+  const double* __restrict__ P = o.P;
+  const int64_t sr = o.sr, sk = o.sk, R = o.R, plane_stride = o.Rpad * Kpad;
+  const unsigned long long* __restrict__ maxbits = o.maxbits;
+  int* __restrict__ exps = o.exps;
+  uint16_t* __restrict__ planes = o.planes;
+  const int RB = o.RB;
+  const int64_t r0 = (int64_t)blockIdx.x * 64 - (isb ? oa.Rpad : 0), k0 = (int64_t)blockIdx.y * 64;
   const bool rows_contig = (sr == 1);
   {
     // all 16 loads of the thread in flight before the LDS stores
@@ -306,15 +322,20 @@ __device__ __forceinline__ int64_t plane_off8(int64_t row, int64_t k, int RB, in
 }
 
 template <int S>
-__global__ __launch_bounds__(256) void split_f64_i8_kernel(const double* __restrict__ P, int64_t sr, int64_t sk,
-                                                           int64_t R, int64_t K,
-                                                           const unsigned long long* __restrict__ maxbits,
-                                                           int* __restrict__ exps, uint8_t* __restrict__ planes,
-                                                           int64_t plane_stride, int64_t Kpad, int RB,
-                                                           int* __restrict__ call_flag, int* __restrict__ sticky) {
+__global__ __launch_bounds__(256) void split_f64_i8_kernel(SplitOperand<double, uint8_t> oa, SplitOperand<double, uint8_t> ob, int64_t K,
+                                              int64_t Kpad, int* __restrict__ call_flag, int* __restrict__ sticky) {
   __shared__ double tile[64][65];
   const int t = threadIdx.x;
-  const int64_t r0 = (int64_t)blockIdx.x * 64, k0 = (int64_t)blockIdx.y * 64;
+  // blocks along x: op(A)'s row tiles, then op(B)'s
+  const bool isb = (int64_t)blockIdx.x * 64 >= oa.Rpad;
+  const SplitOperand<double, uint8_t>& o = isb ? ob : oa;
+  const double* __restrict__ P = o.P;
+  const int64_t sr = o.sr, sk = o.sk, R = o.R, plane_stride = o.Rpad * Kpad;
+  const unsigned long long* __restrict__ maxbits = o.maxbits;
+  int* __restrict__ exps = o.exps;
+  uint8_t* __restrict__ planes = o.planes;
+  const int RB = o.RB;
+  const int64_t r0 = (int64_t)blockIdx.x * 64 - (isb ? oa.Rpad : 0), k0 = (int64_t)blockIdx.y * 64;
   const bool rows_contig = (sr == 1);
   {
     // all 16 loads of the thread in flight before the LDS stores
@@ -378,13 +399,19 @@ __device__ __forceinline__ uint16_t bf16_rn_bits(float f) {
 }
 __device__ __forceinline__ float bf16_to_f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
-__global__ __launch_bounds__(256) void split_f32_kernel(const float* __restrict__ P, int64_t sr, int64_t sk, int64_t R,
-                                                        int64_t K, uint16_t* __restrict__ planes, int64_t plane_stride,
-                                                        int64_t Kpad, int RB, int* __restrict__ call_flag,
+__global__ __launch_bounds__(256) void split_f32_kernel(SplitOperand<float, uint16_t> oa, SplitOperand<float, uint16_t> ob,
+                                                        int64_t K, int64_t Kpad, int* __restrict__ call_flag,
                                                         int* __restrict__ sticky) {
   __shared__ float tile[64][65];
   const int t = threadIdx.x;
-  const int64_t r0 = (int64_t)blockIdx.x * 64, k0 = (int64_t)blockIdx.y * 64;
+  // blocks along x: op(A)'s row tiles, then op(B)'s
+  const bool isb = (int64_t)blockIdx.x * 64 >= oa.Rpad;
+  const SplitOperand<float, uint16_t>& o = isb ? ob : oa;
+  const float* __restrict__ P = o.P;
+  const int64_t sr = o.sr, sk = o.sk, R = o.R, plane_stride = o.Rpad * Kpad;
+  uint16_t* __restrict__ planes = o.planes;
+  const int RB = o.RB;
+  const int64_t r0 = (int64_t)blockIdx.x * 64 - (isb ? oa.Rpad : 0), k0 = (int64_t)blockIdx.y * 64;
   const bool rows_contig = (sr == 1);
   {
     // all 16 loads of the thread in flight before the LDS stores
@@ -814,21 +841,41 @@ inline void strides_b(bool tb, int64_t ldb, int64_t& sr, int64_t& sk) {
   sk = tb ? ldb : 1;
 }
 
-template <int S>
-void launch_split_f64(const double* P, int64_t sr, int64_t sk, int64_t R, int64_t K, int64_t Rpad, int64_t Kpad, int RB,
-                      unsigned long long* mb, int* ex, uint16_t* planes, int* call_flag, int* sticky, hipStream_t st) {
-  hipLaunchKernelGGL(zero_u64_kernel, dim3((unsigned)std::min<int64_t>((Rpad + 255) / 256, 1024)), dim3(256), 0, st,
-                     mb, Rpad);
-  launch_absmax(P, sr, sk, R, K, mb, st);
-  hipLaunchKernelGGL(split_f64_kernel<S>, dim3((unsigned)(Rpad / 64), (unsigned)(Kpad / 64)), dim3(256), 0, st, P, sr,
-                     sk, R, K, mb, ex, planes, Rpad * Kpad, Kpad, RB, call_flag, sticky);
+template <typename T, typename D>
+void split_operands(const GemmArgs& g, const Layout& L, char* ws, int bn, SplitOperand<T, D>& a, SplitOperand<T, D>& b) {
+  auto set = [&](SplitOperand<T, D>& o, const void* P, int64_t R, int64_t Rpad, size_t planes, int RB, size_t mb, size_t ex) {
+    o.P = static_cast<const T*>(P);
+    o.R = R;
+    o.Rpad = Rpad;
+    o.planes = reinterpret_cast<D*>(ws + planes);
+    o.RB = RB;
+    o.maxbits = reinterpret_cast<unsigned long long*>(ws + mb);
+    o.exps = reinterpret_cast<int*>(ws + ex);
+    const bool rows = o.sr == 1;  // as absmax_kernel chooses
+    o.ax = rows ? (R + 255) / 256 : (R + 4 * AM_WROWS - 1) / (4 * AM_WROWS);
+    o.ay = rows ? (g.k + AM_RKC - 1) / AM_RKC : (g.k + AM_KK - 1) / AM_KK;
+  };
+  strides_a(g.ta, g.lda, a.sr, a.sk);
+  strides_b(g.tb, g.ldb, b.sr, b.sk);
+  set(a, g.A, g.m, L.Mpad, L.offA, QBM, L.offMA, L.offEA);
+  set(b, g.B, g.n, L.Npad, L.offB, bn, L.offMB, L.offEB);
 }
 
-// Clears this call's non-finite flag (a kernel, not a memset node, so that the
-// call can be captured into a graph).
-void clear_call_flag(int* call_flag, hipStream_t st) {
-  hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, st, reinterpret_cast<unsigned long long*>(call_flag),
-                     (int64_t)1);
+// The split phase's launches: clear both operands' row maxima (and this call's
+// non-finite flag, where the caller reads it: the words are neighbours), absmax,
+// split.  Kernels, not memset nodes, so that the call can be captured into a graph.
+// (One launch per operand and step, seven in all, took a 2500 x 1900 x 3001 INT8
+// problem 427 us; these three 406.)
+template <typename D, typename SplitKernel>
+void launch_split(const GemmArgs& g, const Layout& L, char* ws, int* flag, int* sticky, hipStream_t st, SplitKernel split) {
+  SplitOperand<double, D> a, b;
+  split_operands(g, L, ws, QBN, a, b);
+  const int64_t words = (int64_t)((flag ? L.offFlag + 8 : L.offEA) - L.offMA) / 8;
+  hipLaunchKernelGGL(zero_u64_kernel, dim3((unsigned)std::min<int64_t>((words + 255) / 256, 1024)), dim3(256), 0, st,
+                     reinterpret_cast<unsigned long long*>(ws + L.offMA), words);
+  hipLaunchKernelGGL(absmax_kernel<D>, dim3((unsigned)(a.ax * a.ay + b.ax * b.ay)), dim3(256), 0, st, a, b, g.k);
+  hipLaunchKernelGGL(split, dim3((unsigned)((L.Mpad + L.Npad) / 64), (unsigned)(L.Kpad / 64)), dim3(256), 0, st, a, b, g.k,
+                     L.Kpad, flag ? flag : sticky, sticky);
 }
 
 // elt as in make_layout: the kernel addresses planes in 16-bit units, so an
@@ -855,23 +902,14 @@ PairArgs pair_args(const GemmArgs& g, const Layout& L, const uint16_t* pA, const
 }
 
 template <int S>
-hipError_t run_ozaki(const GemmArgs& g, const Layout& L, char* ws, int* sticky, hipStream_t st) {
-  int64_t sr, sk;
-  int* flag = reinterpret_cast<int*>(ws + L.offFlag);
-  auto* mbA = reinterpret_cast<unsigned long long*>(ws + L.offMA);
-  auto* mbB = reinterpret_cast<unsigned long long*>(ws + L.offMB);
+hipError_t run_ozaki(const GemmArgs& g, const Layout& L, char* ws, bool want_flag, int* sticky, hipStream_t st) {
+  int* flag = want_flag ? reinterpret_cast<int*>(ws + L.offFlag) : nullptr;
   auto* eA = reinterpret_cast<int*>(ws + L.offEA);
   auto* eB = reinterpret_cast<int*>(ws + L.offEB);
   auto* pA = reinterpret_cast<uint16_t*>(ws + L.offA);
   auto* pB = reinterpret_cast<uint16_t*>(ws + L.offB);
   timing_begin(st, "ozaki_split");
-  clear_call_flag(flag, st);
-  strides_a(g.ta, g.lda, sr, sk);
-  launch_split_f64<S>(static_cast<const double*>(g.A), sr, sk, g.m, g.k, L.Mpad, L.Kpad, QBM, mbA, eA, pA, flag, sticky,
-                      st);
-  strides_b(g.tb, g.ldb, sr, sk);
-  launch_split_f64<S>(static_cast<const double*>(g.B), sr, sk, g.n, g.k, L.Npad, L.Kpad, QBN, mbB, eB, pB, flag, sticky,
-                      st);
+  launch_split<uint16_t>(g, L, ws, flag, sticky, st, split_f64_kernel<S>);
   timing_end(st, "ozaki_split");
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -883,34 +921,14 @@ hipError_t run_ozaki(const GemmArgs& g, const Layout& L, char* ws, int* sticky, 
 }
 
 template <int S>
-void launch_split_f64_i8(const double* P, int64_t sr, int64_t sk, int64_t R, int64_t K, int64_t Rpad, int64_t Kpad,
-                         int RB, unsigned long long* mb, int* ex, uint8_t* planes, int* call_flag, int* sticky,
-                         hipStream_t st) {
-  hipLaunchKernelGGL(zero_u64_kernel, dim3((unsigned)std::min<int64_t>((Rpad + 255) / 256, 1024)), dim3(256), 0, st,
-                     mb, Rpad);
-  launch_absmax(P, sr, sk, R, K, mb, st);
-  hipLaunchKernelGGL(split_f64_i8_kernel<S>, dim3((unsigned)(Rpad / 64), (unsigned)(Kpad / 64)), dim3(256), 0, st, P,
-                     sr, sk, R, K, mb, ex, planes, Rpad * Kpad, Kpad, RB, call_flag, sticky);
-}
-
-template <int S>
-hipError_t run_ozaki_i8(const GemmArgs& g, const Layout& L, char* ws, int* sticky, hipStream_t st) {
-  int64_t sr, sk;
-  int* flag = reinterpret_cast<int*>(ws + L.offFlag);
-  auto* mbA = reinterpret_cast<unsigned long long*>(ws + L.offMA);
-  auto* mbB = reinterpret_cast<unsigned long long*>(ws + L.offMB);
+hipError_t run_ozaki_i8(const GemmArgs& g, const Layout& L, char* ws, bool want_flag, int* sticky, hipStream_t st) {
+  int* flag = want_flag ? reinterpret_cast<int*>(ws + L.offFlag) : nullptr;
   auto* eA = reinterpret_cast<int*>(ws + L.offEA);
   auto* eB = reinterpret_cast<int*>(ws + L.offEB);
   auto* pA = reinterpret_cast<uint8_t*>(ws + L.offA);
   auto* pB = reinterpret_cast<uint8_t*>(ws + L.offB);
   timing_begin(st, "ozaki_i8_split");
-  clear_call_flag(flag, st);
-  strides_a(g.ta, g.lda, sr, sk);
-  launch_split_f64_i8<S>(static_cast<const double*>(g.A), sr, sk, g.m, g.k, L.Mpad, L.Kpad, QBM, mbA, eA, pA, flag,
-                         sticky, st);
-  strides_b(g.tb, g.ldb, sr, sk);
-  launch_split_f64_i8<S>(static_cast<const double*>(g.B), sr, sk, g.n, g.k, L.Npad, L.Kpad, QBN, mbB, eB, pB, flag,
-                         sticky, st);
+  launch_split<uint8_t>(g, L, ws, flag, sticky, st, split_f64_i8_kernel<S>);
   timing_end(st, "ozaki_i8_split");
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -933,34 +951,34 @@ size_t emulated_flag_offset(int64_t m, int64_t n, int64_t k, int s, bool i8) {
 
 size_t ozaki_i8_workspace_bytes(int64_t m, int64_t n, int64_t k, int s) { return make_layout(m, n, k, s, 1).total; }
 
-hipError_t launch_dgemm_ozaki_i8(const GemmArgs& g, int s, void* ws, int* sticky, hipStream_t st) {
+hipError_t launch_dgemm_ozaki_i8(const GemmArgs& g, int s, void* ws, bool want_flag, int* sticky, hipStream_t st) {
   const Layout L = make_layout(g.m, g.n, g.k, s, 1);
   char* w = static_cast<char*>(ws);
   switch (s) {
-    case 1: return run_ozaki_i8<1>(g, L, w, sticky, st);
-    case 2: return run_ozaki_i8<2>(g, L, w, sticky, st);
-    case 3: return run_ozaki_i8<3>(g, L, w, sticky, st);
-    case 4: return run_ozaki_i8<4>(g, L, w, sticky, st);
-    case 5: return run_ozaki_i8<5>(g, L, w, sticky, st);
-    case 6: return run_ozaki_i8<6>(g, L, w, sticky, st);
-    case 7: return run_ozaki_i8<7>(g, L, w, sticky, st);
-    case 8: return run_ozaki_i8<8>(g, L, w, sticky, st);
+    case 1: return run_ozaki_i8<1>(g, L, w, want_flag, sticky, st);
+    case 2: return run_ozaki_i8<2>(g, L, w, want_flag, sticky, st);
+    case 3: return run_ozaki_i8<3>(g, L, w, want_flag, sticky, st);
+    case 4: return run_ozaki_i8<4>(g, L, w, want_flag, sticky, st);
+    case 5: return run_ozaki_i8<5>(g, L, w, want_flag, sticky, st);
+    case 6: return run_ozaki_i8<6>(g, L, w, want_flag, sticky, st);
+    case 7: return run_ozaki_i8<7>(g, L, w, want_flag, sticky, st);
+    case 8: return run_ozaki_i8<8>(g, L, w, want_flag, sticky, st);
     default: return hipErrorInvalidValue;
   }
 }
 
-hipError_t launch_dgemm_ozaki(const GemmArgs& g, int s, void* ws, int* sticky, hipStream_t st) {
+hipError_t launch_dgemm_ozaki(const GemmArgs& g, int s, void* ws, bool want_flag, int* sticky, hipStream_t st) {
   const Layout L = make_layout(g.m, g.n, g.k, s);
   char* w = static_cast<char*>(ws);
   switch (s) {
-    case 1: return run_ozaki<1>(g, L, w, sticky, st);
-    case 2: return run_ozaki<2>(g, L, w, sticky, st);
-    case 3: return run_ozaki<3>(g, L, w, sticky, st);
-    case 4: return run_ozaki<4>(g, L, w, sticky, st);
-    case 5: return run_ozaki<5>(g, L, w, sticky, st);
-    case 6: return run_ozaki<6>(g, L, w, sticky, st);
-    case 7: return run_ozaki<7>(g, L, w, sticky, st);
-    case 8: return run_ozaki<8>(g, L, w, sticky, st);
+    case 1: return run_ozaki<1>(g, L, w, want_flag, sticky, st);
+    case 2: return run_ozaki<2>(g, L, w, want_flag, sticky, st);
+    case 3: return run_ozaki<3>(g, L, w, want_flag, sticky, st);
+    case 4: return run_ozaki<4>(g, L, w, want_flag, sticky, st);
+    case 5: return run_ozaki<5>(g, L, w, want_flag, sticky, st);
+    case 6: return run_ozaki<6>(g, L, w, want_flag, sticky, st);
+    case 7: return run_ozaki<7>(g, L, w, want_flag, sticky, st);
+    case 8: return run_ozaki<8>(g, L, w, want_flag, sticky, st);
     default: return hipErrorInvalidValue;
   }
 }
@@ -990,22 +1008,20 @@ void launch_x3_pairs(const PairArgs& p, int nprod, hipStream_t st) {
   else hipLaunchKernelGGL((slice_pair_gemm_kernel<1, 3, 6, X3_WB, BN>), grid, block, 0, st, p);
 }
 
-hipError_t launch_sgemm_bf16x3(const GemmArgs& g, int nprod, void* ws, int* sticky, hipStream_t st) {
+hipError_t launch_sgemm_bf16x3(const GemmArgs& g, int nprod, void* ws, bool want_flag, int* sticky, hipStream_t st) {
   const int bn = x3_bn(g.m, g.n);
   const Layout L = make_layout(g.m, g.n, g.k, 3, 2, bn);
   char* w = static_cast<char*>(ws);
   auto* pA = reinterpret_cast<uint16_t*>(w + L.offA);
   auto* pB = reinterpret_cast<uint16_t*>(w + L.offB);
   int* flag = reinterpret_cast<int*>(w + L.offFlag);
-  int64_t sr, sk;
+  SplitOperand<float, uint16_t> a, b;
+  split_operands(g, L, w, bn, a, b);
   timing_begin(st, "bf16x3_split");
-  clear_call_flag(flag, st);
-  strides_a(g.ta, g.lda, sr, sk);
-  hipLaunchKernelGGL(split_f32_kernel, dim3((unsigned)(L.Mpad / 64), (unsigned)(L.Kpad / 64)), dim3(256), 0, st,
-                     static_cast<const float*>(g.A), sr, sk, g.m, g.k, pA, L.Mpad * L.Kpad, L.Kpad, QBM, flag, sticky);
-  strides_b(g.tb, g.ldb, sr, sk);
-  hipLaunchKernelGGL(split_f32_kernel, dim3((unsigned)(L.Npad / 64), (unsigned)(L.Kpad / 64)), dim3(256), 0, st,
-                     static_cast<const float*>(g.B), sr, sk, g.n, g.k, pB, L.Npad * L.Kpad, L.Kpad, bn, flag, sticky);
+  if (want_flag)
+    hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, st, reinterpret_cast<unsigned long long*>(flag), (int64_t)1);
+  hipLaunchKernelGGL(split_f32_kernel, dim3((unsigned)((L.Mpad + L.Npad) / 64), (unsigned)(L.Kpad / 64)), dim3(256), 0, st, a,
+                     b, g.k, L.Kpad, want_flag ? flag : sticky, sticky);
   timing_end(st, "bf16x3_split");
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
