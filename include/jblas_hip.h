@@ -332,10 +332,10 @@ int jb_grouped_choices(int method, int64_t count, const jb_gemm_desc* descs, int
 /* For C = alpha*op(A)*op(B) + beta*C_in and upstream gradient dC (m x n):
  *   dA (shape of A) = alpha * dC * op(B)^T   (transA 'N')  or  alpha * op(B) * dC^T ('T')
  *   dB (shape of B) = alpha * op(A)^T * dC   (transB 'N')  or  alpha * dC^T * op(A) ('T')
- * Adjoint GEMMs with m*n >= 256 tiles of 128x128 (and k >= 256) run on the
- * single-problem kernels, one after the other on the stream (asynchronously);
- * smaller ones share one one-shot grouped launch (transposed-layout loaders),
- * which synchronises `stream` like jb_gemm_grouped_dev.
+ * Both run on the single-problem kernels, one after the other on the stream,
+ * asynchronously.  Those with fewer than m*n = 256 tiles of 128x128 (or k < 256) are
+ * split along k as a grouped launch of them would be (jb_grouped_choices), and are not
+ * available while `stream` is being captured (JB_ERR_STATE).
  * dA or dB may be NULL to skip it.  method: JB_F64_NATIVE, JB_F32_NATIVE, JB_F32_BF16X3. */
 int jb_gemm_pullback_dev(int method, char transA, char transB, int64_t m, int64_t n, int64_t k,
                          double alpha, const void* A, int64_t lda, const void* B, int64_t ldb,

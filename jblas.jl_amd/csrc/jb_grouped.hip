@@ -1527,29 +1527,45 @@ static int pullback_descs(char ta, char tb, int64_t m, int64_t n, int64_t k, dou
   return JB_OK;
 }
 
-// The adjoint GEMMs of one large product fill the GPU on their own: those run
-// on the single-problem kernels (128x128 tiles, stream-ordered one after the
-// other); smaller ones share one grouped launch.
+// A large adjoint product fills the GPU on its own; the others (at most two) are split
+// along k exactly as a grouped launch of them would be (plan_choices), for the chains
+// and the bits of that launch.
 static bool pullback_big(const jb_gemm_desc& d) {
   return (double)d.m * (double)d.n >= 256.0 * 128.0 * 128.0 && d.k >= 256;
 }
 
+// Every adjoint runs on the single-problem kernels, one after the other on `s`,
+// without synchronising.  (The small ones shared a one-shot grouped launch before: its
+// lists' allocation and upload, its streams and its synchronisation took 150 us for the
+// two products of a 512 x 384 x 256 layer, which take 25 us here.)
 static int pullback_run_locked(int method, const std::vector<jb_gemm_desc>& d, hipStream_t s) {
   std::vector<jb_gemm_desc> small;
+  for (const jb_gemm_desc& x : d)
+    if (x.m > 0 && x.n > 0 && !pullback_big(x)) small.push_back(x);
+  std::vector<GProb> probs;
+  double flops;
+  int rc = small.empty() ? JB_OK : plan_choices(method, (int64_t)small.size(), small.data(), Forced(), probs, &flops);
+  if (rc) return rc;
+  if (!small.empty() && (rc = refuse_capture(s, "the pullback of a small product"))) return rc;
+  auto choice = probs.begin();
   for (const jb_gemm_desc& x : d) {
-    if (!pullback_big(x)) {
-      small.push_back(x);
-      continue;
-    }
+    if (x.m == 0 || x.n == 0) continue;
     GemmArgs g;
-    int rc = validate_gemm(x.transA, x.transB, x.m, x.n, x.k, x.alpha == 0.0, x.A, x.lda, x.B, x.ldb, x.C, x.ldc, &g);
-    if (rc) return rc;
+    if ((rc = validate_gemm(x.transA, x.transB, x.m, x.n, x.k, x.alpha == 0.0, x.A, x.lda, x.B, x.ldb, x.C, x.ldc, &g)))
+      return rc;
     g.alpha = x.alpha;
     g.beta = x.beta;
-    if ((rc = single_gemm_dev_locked(method, g, s))) return rc;
+    int how = method;
+    bool report = true;
+    if (!pullback_big(x)) {
+      const GProb& c = *choice++;
+      if (c.splitk > 1) g.kchunk = c.kchunk;
+      if (c.cfg == CFG_SMALL && method == JB_F32_BF16X3) how = JB_F32_NATIVE;  // its FP32 chain
+      report = false;
+    }
+    if ((rc = single_gemm_dev_locked(how, g, s, report))) return rc;
   }
-  if (small.empty()) return JB_OK;
-  return run_grouped_once(method, (int64_t)small.size(), small.data(), Forced(), s);
+  return JB_OK;
 }
 
 static int pullback_validate(int method, char ta, char tb, int64_t m, int64_t n, int64_t k, const void* A, int64_t lda,

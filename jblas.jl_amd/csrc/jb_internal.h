@@ -17,7 +17,14 @@ struct GemmArgs {
   int64_t ldb;
   void* C;
   int64_t ldc;
+  // Split-K (adjoints of small products): k per split, a multiple of 32 (0: one
+  // chain over all of k), device memory for the splits' results and zeroed per-tile
+  // counters (gemm_mfma_split_need / bf16x3_split_need), which the call leaves zeroed.
+  int64_t kchunk = 0;
+  void* part = nullptr;
+  int* counters = nullptr;
 };
+int gemm_splits(const GemmArgs& g);
 
 // ---- FP64 -----------------------------------------------------------------
 // Native FP64 MFMA GEMM; its chains are the jmul! recurrence bit for bit.
@@ -58,7 +65,10 @@ size_t bf16x3_flag_offset(int64_t m, int64_t n, int64_t k);
 // ---- FP32 -----------------------------------------------------------------
 // Native FP32 MFMA GEMM; its chains are the jmul! recurrence in Float32 bit for bit.
 hipError_t launch_sgemm_mfma(const GemmArgs& g, hipStream_t s);
-size_t bf16x3_workspace_bytes(int64_t m, int64_t n, int64_t k);
+// Device memory a split-K product on launch_dgemm_mfma (elt 8) / launch_sgemm_mfma (elt 4) needs.
+void gemm_mfma_split_need(const GemmArgs& g, size_t elt, size_t* part_bytes, int64_t* counters);
+void bf16x3_split_need(const GemmArgs& g, size_t* part_bytes, int64_t* counters);
+size_t bf16x3_workspace_bytes(int64_t m, int64_t n, int64_t k, int splits = 1);
 // Non-finite inputs become NaN slices (every product they enter is NaN) and set
 // the two flags as in launch_dgemm_ozaki.
 hipError_t launch_sgemm_bf16x3(const GemmArgs& g, int nprod, void* ws, bool want_flag, int* sticky, hipStream_t s);

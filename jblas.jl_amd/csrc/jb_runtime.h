@@ -17,6 +17,8 @@ struct Buffer {
   void release();
 };
 
+constexpr int64_t SPLITK_COUNTERS = 1 << 16;
+
 struct Runtime {
   std::mutex mu;  // serialises every entry point
   bool inited = false;
@@ -29,6 +31,7 @@ struct Runtime {
   bool ws_pending = false;
   bool ws_in_graph = false;      // a graph captured a call that uses `ws`
   std::vector<void*> retired;    // workspaces that captured graphs may use (freed by jb_finalize)
+  int* counters = nullptr;       // split-K arrival counters, all zero between launches (the user holds `ws`)
   int* sticky = nullptr;         // set by any emulated call that met Inf/NaN; cleared by jb_nonfinite_check
 };
 
@@ -48,8 +51,12 @@ int ws_release(hipStream_t s);
 int run_staged(const GemmArgs& g, size_t elt, bool read_c, const std::function<int(const GemmArgs&, hipStream_t)>& dev);
 
 // One GEMM of a grouped method (JB_F64_NATIVE, JB_F32_NATIVE, JB_F32_BF16X3
-// with six products) on the single-problem kernels.
-int single_gemm_dev_locked(int method, const GemmArgs& g, hipStream_t s);
+// with six products) on the single-problem kernels, split along k if g.kchunk says so.
+// report: whether a non-finite operand raises the sticky flag.
+int single_gemm_dev_locked(int method, const GemmArgs& g, hipStream_t s, bool report = true);
+
+// JB_ERR_STATE while `s` is being captured into a graph.
+int refuse_capture(hipStream_t s, const char* what);
 
 // grouped / autotuner (jb_grouped.hip)
 void grouped_release_all();

@@ -173,6 +173,18 @@ int init_locked(int device) {
     }
     if ((e = hipMemset(r.sticky, 0, 256)) != hipSuccess) return hip_fail(e, "clear the non-finite flag");
   }
+  if (r.counters == nullptr) {
+    if ((e = hipMalloc(&r.counters, SPLITK_COUNTERS * sizeof(int))) != hipSuccess) {
+      r.counters = nullptr;
+      return fail(JB_ERR_ALLOC, "split-K counter allocation failed: %s", hipGetErrorString(e));
+    }
+    if ((e = hipMemset(r.counters, 0, SPLITK_COUNTERS * sizeof(int))) != hipSuccess) {
+      hipFree(r.counters);
+      r.counters = nullptr;
+      return hip_fail(e, "clear the split-K counters");
+    }
+    hipDeviceSynchronize();  // the fill is asynchronous; callers' streams do not wait for it
+  }
   r.device = device;
   r.inited = true;
   log_line("init device %d: %s %s, %d CUs, %.2f GHz, LDS %d B/CU, L2 %lld B, HBM %lld B", device, d.name, d.arch,
@@ -214,6 +226,10 @@ void Buffer::release() {
 static bool capturing(hipStream_t s) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
+int refuse_capture(hipStream_t s, const char* what) {
+  return capturing(s) ? fail(JB_ERR_STATE, "%s is not available during graph capture", what) : JB_OK;
 }
 
 // Stream-ordered use of the shared workspace: a call waits for the previous
@@ -327,6 +343,10 @@ void finalize_locked() {
   r.retired.clear();
   r.ws_in_graph = false;
   r.staging.release();
+  if (r.counters) {
+    hipFree(r.counters);
+    r.counters = nullptr;
+  }
   if (r.sticky) {
     hipFree(r.sticky);
     r.sticky = nullptr;
@@ -832,12 +852,40 @@ static int sgemm_dev_locked(const GemmArgs& g, int method, int nprod, hipStream_
 }
 
 // One problem on the single-problem kernels of a grouped method (the caller
-// holds the lock and has validated `g`).
-extern "C++" int jb::single_gemm_dev_locked(int method, const GemmArgs& g, hipStream_t s) {
-  if (method == JB_F64_NATIVE) return dgemm_dev_locked(g, false, s);
-  if (method == JB_F32_NATIVE) return sgemm_dev_locked(g, JB_F32_NATIVE, 0, s);
-  if (method == JB_F32_BF16X3) return sgemm_dev_locked(g, JB_F32_BF16X3, 6, s);
-  return fail(-1, "unknown method %d", method);
+// holds the lock and has validated `g`).  A split problem's partial results live in
+// the workspace, after the 3xBF16 planes; its user order also keeps the counters
+// to one launch at a time.
+extern "C++" int jb::single_gemm_dev_locked(int method, const GemmArgs& g, hipStream_t s, bool report) {
+  const bool x3 = method == JB_F32_BF16X3, f64 = method == JB_F64_NATIVE;
+  if (!x3 && !f64 && method != JB_F32_NATIVE) return fail(-1, "unknown method %d", method);
+  if (gemm_splits(g) == 1 && (report || !x3))
+    return f64 ? dgemm_dev_locked(g, false, s) : sgemm_dev_locked(g, method, 6, s);
+  if (g.m == 0 || g.n == 0 || g.k == 0 || g.alpha == 0.0) {
+    GemmArgs h = g;
+    h.kchunk = 0;
+    return f64 ? dgemm_dev_locked(h, false, s) : sgemm_dev_locked(h, JB_F32_NATIVE, 0, s);
+  }
+  GemmArgs h = g;
+  const size_t planes = x3 ? bf16x3_workspace_bytes(g.m, g.n, g.k, gemm_splits(g)) : 0;
+  size_t part = 0;
+  int64_t counters = 0;
+  if (gemm_splits(g) > 1) {
+    if (x3) bf16x3_split_need(g, &part, &counters);
+    else gemm_mfma_split_need(g, f64 ? 8 : 4, &part, &counters);
+    // (problems are split only while they have fewer tiles than the device holds workgroups)
+    if (counters > SPLITK_COUNTERS) return fail(JB_ERR_UNSUPPORTED, "split product of %lld tiles", (long long)counters);
+  }
+  void* ws = nullptr;
+  int rc = ws_acquire(planes + part, s, &ws);
+  if (rc) return rc;
+  h.part = static_cast<char*>(ws) + planes;
+  h.counters = rt().counters;
+  // (word 1 of the sticky buffer: a flag nobody reads)
+  const hipError_t e = x3    ? launch_sgemm_bf16x3(h, 6, ws, false, rt().sticky + (report ? 0 : 1), s)
+                       : f64 ? launch_dgemm_mfma(h, s)
+                             : launch_sgemm_mfma(h, s);
+  rc = ws_release(s);
+  return e == hipSuccess ? rc : hip_fail(e, "split-K gemm launch");
 }
 
 int jb_sgemm_dev(char transA, char transB, int64_t m, int64_t n, int64_t k, float alpha, const float* A, int64_t lda,

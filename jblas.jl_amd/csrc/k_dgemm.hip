@@ -19,21 +19,63 @@ namespace jb {
 namespace {
 
 // ---------------------------------------------------------------------------
-// (1) MFMA GEMM: one block per tile of C (jb_ring.h).
+// (1) MFMA GEMM: one block per tile of C (jb_ring.h) and, for the adjoints of a
+//     small product, per chunk of k.
 // ---------------------------------------------------------------------------
+
+// Split-K: each block stores its chunk's results, thread by thread, to its slab; the
+// last block of the tile to arrive sums the slabs in split order into acc and
+// returns true.  The counters are zero between launches: the last block clears its own.
+template <typename T, typename Tile>
+__device__ __forceinline__ bool splitk_sum(typename Tile::Acc& acc, T* part, int* counters, int id, char* lds) {
+  constexpr int EL = Tile::WIM * Tile::WIN * 4;
+  gptr<T> slab = as_global(part) + (int64_t)id * gridDim.y * (EL * Tile::NTH) + threadIdx.x;
+  auto at = [&](int q, int i, int j, int r) { return ((int64_t)q * EL + (i * Tile::WIN + j) * 4 + r) * Tile::NTH; };
+#pragma unroll
+  for (int i = 0; i < Tile::WIM; ++i)
+#pragma unroll
+    for (int j = 0; j < Tile::WIN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) slab[at(blockIdx.y, i, j, r)] = acc[i][j][r];
+  int* flag = reinterpret_cast<int*>(lds);
+  __threadfence();
+  __syncthreads();  // (every wave is done with the ring)
+  if (threadIdx.x == 0) *flag = atomicAdd(counters + id, 1);
+  __syncthreads();
+  if (*flag != (int)gridDim.y - 1) return false;
+  __threadfence();
+  if (threadIdx.x == 0) counters[id] = 0;
+#pragma unroll
+  for (int i = 0; i < Tile::WIM; ++i)
+#pragma unroll
+    for (int j = 0; j < Tile::WIN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = slab[at(0, i, j, r)];
+  for (int q = 1; q < (int)gridDim.y; ++q)
+#pragma unroll
+    for (int i = 0; i < Tile::WIM; ++i)
+#pragma unroll
+      for (int j = 0; j < Tile::WIN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][j][r] += slab[at(q, i, j, r)];
+  return true;
+}
+
 template <typename T, bool TA, bool TB, bool VEC, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int NSLOT,
           int MINW>
 __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
     int64_t M, int64_t N, int64_t K, T alpha, const T* __restrict__ A, int64_t lda, const T* __restrict__ B, int64_t ldb,
-    T beta, T* __restrict__ C, int64_t ldc, int tiles_m, int tiles_n, int acc_from_c) {
+    T beta, T* __restrict__ C, int64_t ldc, int tiles_m, int tiles_n, int acc_from_c, int64_t kchunk, T* __restrict__ part,
+    int* __restrict__ counters) {
   typedef RingTile<T, TA, TB, VEC, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT> Tile;
   constexpr int WIM = Tile::WIM, WIN = Tile::WIN;
   __shared__ __attribute__((aligned(1024))) char ring[Tile::SMEM];
 
   const int nblocks = tiles_m * tiles_n;
+  const int id = xcd_remap(blockIdx.x, nblocks, 8);
   int tm, tn;
-  tile_coords(xcd_remap(blockIdx.x, nblocks, 8), tiles_m, tiles_n, 8, tm, tn);
-  const int64_t m0 = (int64_t)tm * BTM, n0 = (int64_t)tn * BTN;
+  tile_coords(id, tiles_m, tiles_n, 8, tm, tn);
+  const int64_t m0 = (int64_t)tm * BTM, n0 = (int64_t)tn * BTN, kb = blockIdx.y * kchunk;
   Tile tile(ring, threadIdx.x);
 
   // Chains start from -0.0: the first MFMA step fma(a, x, -0.0) is then exactly
@@ -62,9 +104,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
         }
     }
   }
-  tile.begin(as_global(A) + (TA ? m0 * lda : m0), lda, as_global(B) + (TB ? n0 : n0 * ldb), ldb, M - m0, N - n0, K);
+  tile.begin(as_global(A) + (TA ? kb + m0 * lda : m0 + kb * lda), lda, as_global(B) + (TB ? n0 + kb * ldb : kb + n0 * ldb),
+             ldb, M - m0, N - n0, min(K - kb, kchunk));
   tile.run(acc);
-
+  if (gridDim.y > 1 && !splitk_sum<T, Tile>(acc, part, counters, id, ring)) return;
   tile.store(acc, C + m0 + n0 * ldc, ldc, M - m0, N - n0, alpha, beta);
 }
 
@@ -190,6 +233,8 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 }  // namespace
 
+int gemm_splits(const GemmArgs& g) { return g.kchunk > 0 ? (int)std::max<int64_t>(1, (g.k + g.kchunk - 1) / g.kchunk) : 1; }
+
 template <typename T, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int NSLOT, int MINW>
 static hipError_t launch_gemm_mfma_bt(const GemmArgs& g, hipStream_t s, int acc_from_c) {
   const int tiles_m = (int)((g.m + BTM - 1) / BTM), tiles_n = (int)((g.n + BTN - 1) / BTN);
@@ -202,11 +247,13 @@ static hipError_t launch_gemm_mfma_bt(const GemmArgs& g, hipStream_t s, int acc_
   auto B = static_cast<const T*>(g.B);
   auto C = static_cast<T*>(g.C);
   const T alpha = (T)g.alpha, beta = (T)g.beta;
+  const int splits = gemm_splits(g);
+  const int64_t kchunk = splits > 1 ? g.kchunk : g.k;
   const char* tname = sizeof(T) == 8 ? "dgemm_mfma" : "sgemm_mfma";
 #define JB_LAUNCH_V(TA, TB, V)                                                                                          \
-  hipLaunchKernelGGL((gemm_mfma_kernel<T, TA, TB, V, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT, MINW>), dim3(nblocks),        \
+  hipLaunchKernelGGL((gemm_mfma_kernel<T, TA, TB, V, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT, MINW>), dim3(nblocks, splits), \
                      dim3(64 * WGM * WGN), 0, s, g.m, g.n, g.k, alpha, A, g.lda, B, g.ldb, beta, C, g.ldc, tiles_m,     \
-                     tiles_n, acc_from_c)
+                     tiles_n, acc_from_c, kchunk, static_cast<T*>(g.part), g.counters)
 #define JB_LAUNCH(TA, TB)                      \
   do {                                         \
     if (vec) JB_LAUNCH_V(TA, TB, !WIDE);     \
@@ -245,33 +292,51 @@ template <> struct Ring<float, 32, 32> { static constexpr auto run = launch_gemm
 // 124 / 37.6 / 36.7 / 36.9, 1536^3 178 / 146 / 119 / 119, 3072^3 1023 / 811 / 876 /
 // 943, 4096^3 1826 / 1961 / 2038 / 2209; FP32 800x840x900 60 / 20.3 / 20.4 / 18.8,
 // 3072^3 519 / 426 / 475 / 526, 4096^3 922 / 986 / 1074 / 1216.
+enum TileId { T128, T64, T64X32, T32, TWIDE };
 template <typename T>
-static hipError_t launch_gemm_mfma(const GemmArgs& g, hipStream_t s, int acc_from_c = 0) {
+static TileId pick_tile(const GemmArgs& g) {
   constexpr bool F64 = sizeof(T) == 8;
   // A load's offset inside a stage spans up to 128 rows of ld elements (k contiguous) or 32 k of them (rows
   // contiguous).  Past 32 bits (from 2^22 or 2^24 doubles on) the 64x32 tile with 64-bit addresses takes the problem.
   const int64_t lim = ((int64_t)1 << 32) / (int64_t)sizeof(T);
-  if (g.lda >= lim / (g.ta ? 128 : 32) || g.ldb >= lim / (g.tb ? 32 : 128))
-    return launch_gemm_mfma_bt<T, true, 64, 32, 2, 2, F64 ? 16 : 32, 3, 2>(g, s, acc_from_c);
+  if (g.lda >= lim / (g.ta ? 128 : 32) || g.ldb >= lim / (g.tb ? 32 : 128)) return TWIDE;
   // testing: pin one variant ("128", "64", "64x32", "32")
   const char* force = getenv("JB_GEMM_TILE");
   if (force && *force) {
-    if (!strcmp(force, "128")) return Ring<T, 128, 128>::run(g, s, acc_from_c);
-    if (!strcmp(force, "64")) return Ring<T, 64, 64>::run(g, s, acc_from_c);
-    if (!strcmp(force, "64x32")) return Ring<T, 64, 32>::run(g, s, acc_from_c);
-    if (!strcmp(force, "32")) return Ring<T, 32, 32>::run(g, s, acc_from_c);
+    if (!strcmp(force, "128")) return T128;
+    if (!strcmp(force, "64")) return T64;
+    if (!strcmp(force, "64x32")) return T64X32;
+    if (!strcmp(force, "32")) return T32;
   }
-  const int64_t cus = std::max(runtime_compute_units(), 1);
+  const int64_t cus = std::max(runtime_compute_units(), 1), splits = gemm_splits(g);
   auto cost = [&](int bm, int bn, double rate, double alone) {
-    const int64_t tiles = ((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn);
-    const int64_t rounds = (tiles + cus - 1) / cus;
+    const int64_t blocks = ((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * splits;
+    const int64_t rounds = (blocks + cus - 1) / cus;
     return (double)(rounds * bm * bn) / (rounds == 1 ? rate * alone : rate);
   };
   const double c128 = cost(128, 128, 1.0, 0.95), c64 = cost(64, 64, F64 ? 0.96 : 0.91, 0.90);
   const double c64x32 = cost(64, 32, F64 ? 0.885 : 0.83, 1.0), c32 = cost(32, 32, F64 ? 0.81 : 0.74, 1.0);
-  if (c128 <= std::min(c64, std::min(c64x32, c32))) return Ring<T, 128, 128>::run(g, s, acc_from_c);
-  if (c64 <= std::min(c64x32, c32)) return Ring<T, 64, 64>::run(g, s, acc_from_c);
-  return c64x32 < c32 ? Ring<T, 64, 32>::run(g, s, acc_from_c) : Ring<T, 32, 32>::run(g, s, acc_from_c);
+  if (c128 <= std::min(c64, std::min(c64x32, c32))) return T128;
+  if (c64 <= std::min(c64x32, c32)) return T64;
+  return c64x32 < c32 ? T64X32 : T32;
+}
+
+template <typename T>
+static hipError_t launch_gemm_mfma(const GemmArgs& g, hipStream_t s, int acc_from_c = 0) {
+  switch (pick_tile<T>(g)) {
+    case T128: return Ring<T, 128, 128>::run(g, s, acc_from_c);
+    case T64: return Ring<T, 64, 64>::run(g, s, acc_from_c);
+    case T64X32: return Ring<T, 64, 32>::run(g, s, acc_from_c);
+    case T32: return Ring<T, 32, 32>::run(g, s, acc_from_c);
+    default: return launch_gemm_mfma_bt<T, true, 64, 32, 2, 2, sizeof(T) == 8 ? 16 : 32, 3, 2>(g, s, acc_from_c);
+  }
+}
+
+void gemm_mfma_split_need(const GemmArgs& g, size_t elt, size_t* part_bytes, int64_t* counters) {
+  static const int BM[] = {128, 64, 64, 32, 64}, BN[] = {128, 64, 32, 32, 32};
+  const TileId t = elt == 8 ? pick_tile<double>(g) : pick_tile<float>(g);
+  *counters = ((g.m + BM[t] - 1) / BM[t]) * ((g.n + BN[t] - 1) / BN[t]);
+  *part_bytes = (size_t)*counters * gemm_splits(g) * BM[t] * BN[t] * elt;
 }
 
 hipError_t launch_dgemm_mfma(const GemmArgs& g, hipStream_t s) { return launch_gemm_mfma<double>(g, s); }

@@ -490,6 +490,10 @@ struct PairArgs {
   void* C;
   int64_t ldc;
   int tiles_m, tiles_n;
+  // split-K (3xBF16): k stages per split, the splits' results and per-tile counters
+  int split_stages;
+  float* part;
+  int* counters;
 };
 
 __device__ __forceinline__ void two_sum(double a, double b, double& s, double& e) {
@@ -565,8 +569,10 @@ __global__ __launch_bounds__((64 * (QBM / (32 * WB)) * (BN / 32)), 1) void slice
   // registers) plus the lane's offset, added last.  Adding the lane offset
   // first put a 64-bit vector add (and selects) in front of every load; this
   // form took the s = 6 kernel from 19.9 to 19.0 ms at 8192^3.
-  const uint16_t* gA = p.pa + (int64_t)tm * QBM * p.Kpad;
-  const uint16_t* gB = p.pb + (int64_t)tn * BN * p.Kpad;
+  // (3xBF16 split-K: this block's stages start at st0)
+  const int64_t st0 = MODE == 1 ? (int64_t)blockIdx.y * p.split_stages : 0;
+  const uint16_t* gA = p.pa + (int64_t)tm * QBM * p.Kpad + st0 * (QBM * QBK);
+  const uint16_t* gB = p.pb + (int64_t)tn * BN * p.Kpad + st0 * (BN * QBK);
   // Piece i of this wave's share of stage ks (pieces j = wave + NWAVES*i; A:
   // plane t, 4 pieces of 1 KB; B: plane t, BN/32 pieces) -> LDS slot `slot`.
   auto issue_piece = [&](int ks, int slot, int i) JB_INLINE {
@@ -636,7 +642,7 @@ __global__ __launch_bounds__((64 * (QBM / (32 * WB)) * (BN / 32)), 1) void slice
   // pass).  Per chunk end the flushes stay in increasing level order.
   auto fast = [&](const int L) { return MODE == 0 && S <= 6 && kc_stages(L) == 2; };  // (S > 6 would spill)
 
-  const int nst = (int)(p.Kpad / QBK);
+  const int nst = MODE == 1 ? (int)min<int64_t>(p.Kpad / QBK - st0, p.split_stages) : (int)(p.Kpad / QBK);
   // The prefetch is unconditional: past the last stage it loads the last stage
   // again, into the slot of a stage every wave is done with, so every stage has
   // the same loads in flight and the stage code has no branch around its loads
@@ -774,6 +780,37 @@ __global__ __launch_bounds__((64 * (QBM / (32 * WB)) * (BN / 32)), 1) void slice
       }
     }
   } else {
+    float res[WB][16];
+#pragma unroll
+    for (int b = 0; b < WB; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) res[b][e] = acc[0][b][e] + acc[1][b][e];
+    if (gridDim.y > 1) {
+      // Each block stores its chunk's results, thread by thread, to its slab; the tile's last block to arrive sums
+      // the slabs in split order.  The counters are zero between launches: that block clears its own.
+      constexpr int NTH = 64 * NWAVES;
+      gptr<float> slab = as_global(p.part) + (int64_t)tile * gridDim.y * (QBM * BN) + tid;
+#pragma unroll
+      for (int b = 0; b < WB; ++b)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) slab[(int64_t)blockIdx.y * (QBM * BN) + (b * 16 + e) * NTH] = res[b][e];
+      int* flag = reinterpret_cast<int*>(ring);
+      __threadfence();
+      __syncthreads();  // (every wave is done with the ring)
+      if (tid == 0) *flag = atomicAdd(p.counters + tile, 1);
+      __syncthreads();
+      if (*flag != (int)gridDim.y - 1) return;
+      __threadfence();
+      if (tid == 0) p.counters[tile] = 0;
+      for (int q = 0; q < (int)gridDim.y; ++q)
+#pragma unroll
+        for (int b = 0; b < WB; ++b)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const float v = slab[(int64_t)q * (QBM * BN) + (b * 16 + e) * NTH];
+            res[b][e] = q == 0 ? v : res[b][e] + v;
+          }
+    }
     gptr<float> C = as_global(static_cast<float*>(eC));
     const float alpha = (float)ealpha, beta = (float)ebeta;
 #pragma unroll
@@ -784,7 +821,7 @@ __global__ __launch_bounds__((64 * (QBM / (32 * WB)) * (BN / 32)), 1) void slice
       for (int e = 0; e < 16; ++e) {
         const int64_t n = n0 + wn0 + 8 * (e / 4) + 4 * hl + (e % 4);
         if (n < eN) {
-          float c = alpha * (acc[0][b][e] + acc[1][b][e]);
+          float c = alpha * res[b][e];
           if (beta != 0.0f) c = fmaf(beta, C[m + n * eldc], c);
           C[m + n * eldc] = c;
         }
@@ -898,6 +935,9 @@ PairArgs pair_args(const GemmArgs& g, const Layout& L, const uint16_t* pA, const
   p.ldc = g.ldc;
   p.tiles_m = (int)(L.Mpad / QBM);
   p.tiles_n = (int)(L.Npad / bn);
+  p.split_stages = (int)(p.Kpad / QBK);
+  p.part = static_cast<float*>(g.part);
+  p.counters = g.counters;
   return p;
 }
 
@@ -989,19 +1029,25 @@ hipError_t launch_dgemm_ozaki(const GemmArgs& g, int s, void* ws, bool want_flag
 // waves, two workgroups per CU).  At 8192^3: 277 -> 305 TF/s with 3 products,
 // 197 -> 207 with 6; 4096 x 2048 x 4096 with 6: 165 -> 171; 2048^3 (128 tiles
 // of 128 x 256): 149 -> 119, hence the 128-wide tile there.
-int x3_bn(int64_t m, int64_t n) {
+int x3_bn(int64_t m, int64_t n, int splits = 1) {
+  if (splits > 1) return 128;
   const int64_t t256 = ((m + QBM - 1) / QBM) * ((n + 255) / 256);
   return t256 >= 2 * (int64_t)std::max(runtime_compute_units(), 1) ? 256 : 128;
 }
 
-size_t bf16x3_workspace_bytes(int64_t m, int64_t n, int64_t k) {
-  return make_layout(m, n, k, 3, 2, x3_bn(m, n)).total;
+size_t bf16x3_workspace_bytes(int64_t m, int64_t n, int64_t k, int splits) {
+  return make_layout(m, n, k, 3, 2, x3_bn(m, n, splits)).total;
 }
 size_t bf16x3_flag_offset(int64_t m, int64_t n, int64_t k) { return make_layout(m, n, k, 3, 2, x3_bn(m, n)).offFlag; }
 
+void bf16x3_split_need(const GemmArgs& g, size_t* part_bytes, int64_t* counters) {
+  *counters = ((g.m + QBM - 1) / QBM) * ((g.n + 127) / 128);
+  *part_bytes = (size_t)*counters * gemm_splits(g) * QBM * 128 * sizeof(float);
+}
+
 template <int BN>
-void launch_x3_pairs(const PairArgs& p, int nprod, hipStream_t st) {
-  const dim3 grid(p.tiles_m * p.tiles_n);
+void launch_x3_pairs(const PairArgs& p, int nprod, int splits, hipStream_t st) {
+  const dim3 grid(p.tiles_m * p.tiles_n, splits);
   const dim3 block(64 * (QBM / (32 * X3_WB)) * (BN / 32));
   if (nprod == 3) hipLaunchKernelGGL((slice_pair_gemm_kernel<1, 3, 3, X3_WB, BN>), grid, block, 0, st, p);
   else if (nprod == 6) hipLaunchKernelGGL((slice_pair_gemm_kernel<1, 3, 4, X3_WB, BN>), grid, block, 0, st, p);
@@ -1009,7 +1055,7 @@ void launch_x3_pairs(const PairArgs& p, int nprod, hipStream_t st) {
 }
 
 hipError_t launch_sgemm_bf16x3(const GemmArgs& g, int nprod, void* ws, bool want_flag, int* sticky, hipStream_t st) {
-  const int bn = x3_bn(g.m, g.n);
+  const int bn = x3_bn(g.m, g.n, gemm_splits(g));
   const Layout L = make_layout(g.m, g.n, g.k, 3, 2, bn);
   char* w = static_cast<char*>(ws);
   auto* pA = reinterpret_cast<uint16_t*>(w + L.offA);
@@ -1025,10 +1071,11 @@ hipError_t launch_sgemm_bf16x3(const GemmArgs& g, int nprod, void* ws, bool want
   timing_end(st, "bf16x3_split");
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const PairArgs p = pair_args(g, L, pA, pB, nullptr, nullptr, 2, bn);
+  PairArgs p = pair_args(g, L, pA, pB, nullptr, nullptr, 2, bn);
+  if (gemm_splits(g) > 1) p.split_stages = (int)(g.kchunk / QBK);
   timing_begin(st, "bf16x3_gemm");
-  if (bn == 256) launch_x3_pairs<256>(p, nprod, st);
-  else launch_x3_pairs<128>(p, nprod, st);
+  if (bn == 256) launch_x3_pairs<256>(p, nprod, 1, st);
+  else launch_x3_pairs<128>(p, nprod, gemm_splits(g), st);
   timing_end(st, "bf16x3_gemm");
   return hipGetLastError();
 }

@@ -6,8 +6,8 @@ For Y = alpha*op(A)*op(B) + beta*C and an upstream cotangent dY:
   dB    = alpha * op(A)^T * dY            (tB = 'N';  alpha * dY^T * op(A) for 'T')
   dC    = beta * dY
   dalpha = <dY, op(A)*op(B)>,  dbeta = <dY, C>
-dA and dB come from the library's pullback entry point: both adjoint GEMMs in
-one grouped launch with the transposed-layout loaders.  The reference has no
+dA and dB come from the library's pullback entry point, which runs the two adjoint
+GEMMs one after the other on the stream.  The reference has no
 differentiation (ChainRulesCore is absent from its Project.toml).
 """
 from __future__ import annotations
@@ -34,7 +34,7 @@ def _fwd_method(dtype, method):
 
 
 def pullback_(tA: str, tB: str, alpha: float, A, B, dY, dA=None, dB=None, *, method=None, stream=None):
-    """dA, dB (either may be None) in one grouped launch; returns (dA, dB)."""
+    """dA, dB (either may be None), stream-ordered; returns (dA, dB)."""
     a, b, dy = _Operand(A, False, "A"), _Operand(B, False, "B"), _Operand(dY, False, "dY")
     m, k = (a.rows, a.cols) if tA.upper() == "N" else (a.cols, a.rows)
     n = b.cols if tB.upper() == "N" else b.rows
@@ -93,7 +93,7 @@ def pullback_grouped_(problems: Sequence[tuple], *, method=None, stream=None) ->
 
 class GemmFunction(torch.autograd.Function):
     """torch autograd binding: Y = A @ B through the library, backward through
-    the pullback entry point (one grouped launch for dA and dB)."""
+    the pullback entry point (dA and dB, one after the other)."""
 
     @staticmethod
     def forward(ctx, A, B, method=None):
