@@ -341,6 +341,14 @@ int jb_gemm_pullback_dev(int method, char transA, char transB, int64_t m, int64_
                          double alpha, const void* A, int64_t lda, const void* B, int64_t ldb,
                          const void* dC, int64_t lddc, void* dA, int64_t ldda, void* dB,
                          int64_t lddb, void* stream);
+/* The same for a cotangent stored either way: dC is op(dC) = dC ('N', m x n) or its
+ * transpose ('T': the memory is n x m), and the gradients are those of op(A) (dA, m x k)
+ * and op(B) (dB, k x n) whatever transA and transB.  Row-major A, B and dC enter as 'T'
+ * operands without a copy. */
+int jb_gemm_adjoint_dev(int method, char transA, char transB, char transC, int64_t m, int64_t n,
+                        int64_t k, double alpha, const void* A, int64_t lda, const void* B,
+                        int64_t ldb, const void* dC, int64_t lddc, void* dA, int64_t ldda,
+                        void* dB, int64_t lddb, void* stream);
 int jb_gemm_pullback(int method, char transA, char transB, int64_t m, int64_t n, int64_t k,
                      double alpha, const void* A, int64_t lda, const void* B, int64_t ldb,
                      const void* dC, int64_t lddc, void* dA, int64_t ldda, void* dB,

@@ -1604,6 +1604,41 @@ int jb_gemm_pullback_dev(int method, char transA, char transB, int64_t m, int64_
   return pullback_run_locked(method, d, (hipStream_t)stream);
 }
 
+int jb_gemm_adjoint_dev(int method, char transA, char transB, char transC, int64_t m, int64_t n, int64_t k, double alpha,
+                        const void* A, int64_t lda, const void* B, int64_t ldb, const void* dC, int64_t lddc, void* dA,
+                        int64_t ldda, void* dB, int64_t lddb, void* stream) {
+  const bool tc = !(transC == 'N' || transC == 'n');
+  if (!(transC == 'N' || transC == 'n' || transC == 'T' || transC == 't' || transC == 'C' || transC == 'c'))
+    return fail(-4, "bad transC");
+  // the gradients are those of op(A) and op(B): checked as the outputs of an 'N', 'N' product
+  int rc = pullback_validate(method, transA, transB, m, n, k, A, lda, B, ldb, dC, tc ? std::max<int64_t>(1, m) : lddc,
+                             nullptr, 1, nullptr, 1);
+  if (rc) return rc < -3 ? rc - 1 : rc;
+  if (dB && m > 0 && !A) return fail(-9, "A is NULL");
+  if (dA && n > 0 && !B) return fail(-11, "B is NULL");
+  if (tc && lddc < std::max<int64_t>(1, n)) return fail(-14, "lddc too small");
+  if (dA && ldda < std::max<int64_t>(1, m)) return fail(-16, "ldda too small");
+  if (dB && lddb < std::max<int64_t>(1, k)) return fail(-18, "lddb too small");
+  std::vector<jb_gemm_desc> d;
+  pullback_descs('N', 'N', m, n, k, alpha, A, lda, B, ldb, dC, lddc, dA, ldda, dB, lddb, d);
+  for (jb_gemm_desc& x : d) {
+    // dA = alpha*op(dC)*op(B)^T, dB = alpha*op(A)^T*op(dC)
+    const bool tA = !(transA == 'N' || transA == 'n'), tB = !(transB == 'N' || transB == 'n');
+    if (x.C == dA) {
+      x.transA = tc ? 'T' : 'N';
+      x.transB = tB ? 'N' : 'T';
+    } else {
+      x.transA = tA ? 'N' : 'T';
+      x.transB = tc ? 'T' : 'N';
+    }
+  }
+  if (d.empty()) return JB_OK;
+  if ((rc = validate_descs(method, (int64_t)d.size(), d.data()))) return rc;
+  std::lock_guard<std::mutex> lk(rt().mu);
+  if ((rc = ensure_init())) return rc;
+  return pullback_run_locked(method, d, (hipStream_t)stream);
+}
+
 int jb_gemm_pullback(int method, char transA, char transB, int64_t m, int64_t n, int64_t k, double alpha,
                      const void* A, int64_t lda, const void* B, int64_t ldb, const void* dC, int64_t lddc, void* dA,
                      int64_t ldda, void* dB, int64_t lddb) {

@@ -107,6 +107,8 @@ SIGNATURES = {
     "jb_grouped_choices": (_int, [_int, _i64, C.c_void_p, C.POINTER(_int), C.POINTER(_int), C.POINTER(_i64)]),
     "jb_gemm_pullback_dev": (_int, [_int, _ch, _ch, _i64, _i64, _i64, _dbl, _p, _i64, _p, _i64, _p, _i64, _p, _i64,
                                     _p, _i64, _p]),
+    "jb_gemm_adjoint_dev": (_int, [_int, _ch, _ch, _ch, _i64, _i64, _i64, _dbl, _p, _i64, _p, _i64, _p, _i64, _p, _i64,
+                                   _p, _i64, _p]),
     "jb_gemm_pullback": (_int, [_int, _ch, _ch, _i64, _i64, _i64, _dbl, _p, _i64, _p, _i64, _p, _i64, _p, _i64,
                                 _p, _i64]),
     "jb_fill_uniform_dev": (_int, [C.c_uint64, _i64, _p, _p]),
