@@ -75,7 +75,7 @@ __device__ __forceinline__ void put_result(const GProb& P, int tm, int tn, int s
   } else {
     const int tile = tm * P.tiles_n + tn;
     gptr<T> slab = as_global(static_cast<T*>(P.part)) + ((int64_t)tile * P.splitk + split) * (BM * BN);
-    slab[i + j * BM] = v;
+    agent_store(slab + i + j * BM, v);
   }
 }
 
@@ -85,25 +85,33 @@ template <typename T, int BM, int NTH>
 __device__ void splitk_combine(const GProb& P, int tm, int tn, int BN, int* counters, int* sflag) {
   if (P.splitk == 1) return;
   const int tile = tm * P.tiles_n + tn;
-  __threadfence();
+  drain_stores();
   __syncthreads();
   if (threadIdx.x == 0) *sflag = atomicAdd(counters + P.counter_base + tile, 1);
   __syncthreads();
   if (*sflag != P.splitk - 1) return;  // not the last split of this tile
-  __threadfence();
   gptr<const T> slab = as_global(static_cast<const T*>(P.part)) + ((int64_t)tile * P.splitk) * (BM * BN);
   gptr<T> C = as_global(static_cast<T*>(P.C));
   const T alpha = (T)P.alpha, beta = (T)P.beta;
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  for (int e = threadIdx.x; e < BM * BN; e += NTH) {
-    const int i = e % BM, j = e / BM;
-    const int64_t m = m0 + i, n = n0 + j;
-    if (m < P.m && n < P.n) {
-      T s = slab[e];
-      for (int q = 1; q < P.splitk; ++q) s += slab[(int64_t)q * (BM * BN) + e];
-      T c = alpha * s;
-      if (beta != T(0)) c = fma(beta, C[m + n * P.ldc], c);
-      C[m + n * P.ldc] = c;
+  constexpr int U = 4;  // loads in flight per thread; tiles have a multiple of 32 columns
+  static_assert(BM * 32 % (U * NTH) == 0, "whole groups of loads");
+  for (int e = threadIdx.x; e < BM * BN; e += U * NTH) {
+    T s[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) s[u] = agent_load<T>(slab + e + u * NTH);
+    for (int q = 1; q < P.splitk; ++q)
+#pragma unroll
+      for (int u = 0; u < U; ++u) s[u] += agent_load<T>(slab + (int64_t)q * (BM * BN) + e + u * NTH);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = (e + u * NTH) % BM, j = (e + u * NTH) / BM;
+      const int64_t m = m0 + i, n = n0 + j;
+      if (m < P.m && n < P.n) {
+        T c = alpha * s[u];
+        if (beta != T(0)) c = fma(beta, C[m + n * P.ldc], c);
+        C[m + n * P.ldc] = c;
+      }
     }
   }
 }

@@ -99,6 +99,22 @@ void timing_end(hipStream_t s, const char* kernel);
 template <typename T> using gptr = __attribute__((address_space(1))) T*;
 template <typename T> __device__ __forceinline__ gptr<T> as_global(T* p) { return (gptr<T>)p; }
 
+// Split-K partial results pass between workgroups on different XCDs, whose L2s are not
+// coherent.  Device-scope stores and loads of the elements themselves (write-through,
+// read past the L2), the stores drained before the tile's arrival counter is raised,
+// take the place of device-scope fences: a fence writes the whole L2 back, and every
+// wave of every split issued one (256 x 384 x 512 FP32 in two splits: 25.9 us, 8.1 so;
+// 1024 uneven FP64 products of a plan 2405, 2380).
+template <typename T> __device__ __forceinline__ void agent_store(gptr<T> p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T> __device__ __forceinline__ T agent_load(gptr<const T> p) {
+  return __hip_atomic_load((gptr<T>)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void drain_stores() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // XCD-aware block swizzle: hardware places workgroup w on XCD (w % nxcd).
 // Returns a tile id such that each XCD owns a contiguous range of tile ids.
 __device__ __forceinline__ int xcd_remap(int w, int nblocks, int nxcd) {

@@ -36,28 +36,27 @@ __device__ __forceinline__ bool splitk_sum(typename Tile::Acc& acc, T* part, int
 #pragma unroll
     for (int j = 0; j < Tile::WIN; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) slab[at(blockIdx.y, i, j, r)] = acc[i][j][r];
+      for (int r = 0; r < 4; ++r) agent_store(slab + at(blockIdx.y, i, j, r), acc[i][j][r]);
   int* flag = reinterpret_cast<int*>(lds);
-  __threadfence();
+  drain_stores();
   __syncthreads();  // (every wave is done with the ring)
   if (threadIdx.x == 0) *flag = atomicAdd(counters + id, 1);
   __syncthreads();
   if (*flag != (int)gridDim.y - 1) return false;
-  __threadfence();
   if (threadIdx.x == 0) counters[id] = 0;
 #pragma unroll
   for (int i = 0; i < Tile::WIM; ++i)
 #pragma unroll
     for (int j = 0; j < Tile::WIN; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[i][j][r] = slab[at(0, i, j, r)];
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = agent_load<T>(slab + at(0, i, j, r));
   for (int q = 1; q < (int)gridDim.y; ++q)
 #pragma unroll
     for (int i = 0; i < Tile::WIM; ++i)
 #pragma unroll
       for (int j = 0; j < Tile::WIN; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[i][j][r] += slab[at(q, i, j, r)];
+        for (int r = 0; r < 4; ++r) acc[i][j][r] += agent_load<T>(slab + at(q, i, j, r));
   return true;
 }
 

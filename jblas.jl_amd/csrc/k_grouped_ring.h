@@ -52,7 +52,7 @@ __device__ __forceinline__ void ring_part(const GProb& P, const GItem& w, int64_
 #pragma unroll
       for (int j = 0; j < WIN; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) slab[tile.row(i) + (coff + tile.col(j, r)) * BM] = acc[i][j][r];
+        for (int r = 0; r < 4; ++r) agent_store<T>(slab + tile.row(i) + (coff + tile.col(j, r)) * BM, acc[i][j][r]);
   }
 }
 

@@ -793,21 +793,20 @@ __global__ __launch_bounds__((64 * (QBM / (32 * WB)) * (BN / 32)), 1) void slice
 #pragma unroll
       for (int b = 0; b < WB; ++b)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) slab[(int64_t)blockIdx.y * (QBM * BN) + (b * 16 + e) * NTH] = res[b][e];
+        for (int e = 0; e < 16; ++e) agent_store(slab + (int64_t)blockIdx.y * (QBM * BN) + (b * 16 + e) * NTH, res[b][e]);
       int* flag = reinterpret_cast<int*>(ring);
-      __threadfence();
+      drain_stores();
       __syncthreads();  // (every wave is done with the ring)
       if (tid == 0) *flag = atomicAdd(p.counters + tile, 1);
       __syncthreads();
       if (*flag != (int)gridDim.y - 1) return;
-      __threadfence();
       if (tid == 0) p.counters[tile] = 0;
       for (int q = 0; q < (int)gridDim.y; ++q)
 #pragma unroll
         for (int b = 0; b < WB; ++b)
 #pragma unroll
           for (int e = 0; e < 16; ++e) {
-            const float v = slab[(int64_t)q * (QBM * BN) + (b * 16 + e) * NTH];
+            const float v = agent_load<float>(slab + (int64_t)q * (QBM * BN) + (b * 16 + e) * NTH);
             res[b][e] = q == 0 ? v : res[b][e] + v;
           }
     }
