@@ -37,8 +37,11 @@ namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f16v __attribute__((ext_vector_type(16)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+#define JB_INLINE __attribute__((always_inline))  // lambdas of the kernels: never outlined
 
 // The thread index as an opaque value, read once per work item: offsets derived
 // from it are then formed inside the work loop of the persistent kernel rather
@@ -84,46 +87,6 @@ struct GRun4 {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         v[q][e] = (gr < Rtot && gk + e < Kend) ? (RC ? P[gr + (gk + e) * ld] : P[gk + e + gr * ld]) : 0.0f;
-    }
-  }
-  // Stages whose k range lies inside the operand: the lane part of each run's
-  // address is formed once per work item (lane_base), with the row clamped
-  // into the operand (a row past its end reads the last row and is zeroed);
-  // a stage then adds only the wave-uniform k0 (times ld for rows-contiguous
-  // operands), so a load costs one 64-bit add instead of a guarded 64-bit
-  // multiply-add chain per element.  A k-contiguous run is one 16-byte load
-  // when `vec` (16-byte aligned base, ld a multiple of 4).
-  gptr<const float> lp[NR];
-  bool rok[NR];
-  __device__ __forceinline__ void lane_base(gptr<const float> P, int64_t ld, int64_t r0, int64_t Rtot) {
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      const int64_t r = r0 + row(q);
-      rok[q] = r < Rtot;
-      const int64_t rc = rok[q] ? r : Rtot - 1;
-      lp[q] = RC ? P + rc + (int64_t)(4 * krun(q)) * ld : P + rc * ld + 4 * krun(q);
-    }
-  }
-  // rows_in: every row of the tile lies inside the operand (no zeroing)
-  __device__ __forceinline__ void load_kfull(int64_t ld, int64_t k0, bool vec, bool rows_in) {
-    if (!RC && vec) {
-#pragma unroll
-      for (int q = 0; q < NR; ++q) {
-        const V4 x = *(gptr<const V4>)(lp[q] + k0);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[q][e] = x[e];
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < NR; ++q)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[q][e] = RC ? lp[q][(k0 + e) * ld] : lp[q][k0 + e];
-    }
-    if (!rows_in) {
-#pragma unroll
-      for (int q = 0; q < NR; ++q)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[q][e] = rok[q] ? v[q][e] : 0.0f;
     }
   }
   // x = hi + mid + lo + rest: each plane is x rounded to BF16 (nearest even,
@@ -262,25 +225,208 @@ __device__ void bf16x3_tile(const GProb& P, int tm, int tn, int split, char* sme
   splitk_combine<float, BM, GNT>(P, tm, tn, BN, counters, sflag);
 }
 
+// One operand's stages of the 128-row/column 3xBF16 tiles, in the run map of GRun4: raw
+// FP32 runs of four k in registers, loaded through a buffer descriptor (the stage's base
+// in scalar registers, one lane offset per run), then split plane by plane.  Rows past
+// the operand read its last row: they meet only rows or columns outside C.
+template <int R, bool RC, bool VEC, int NTH>
+struct XRuns {
+  static constexpr int BK = 32, NR = R * BK / (4 * NTH);
+  static_assert(R * BK == 4 * NTH * NR && (!RC || NTH % R == 0), "run map");
+  typedef float V4 __attribute__((ext_vector_type(4)));
+  V4 v[NR];
+  uint32_t vo[NR];  // bytes from the stage's base
+  uint32_t wo[NR];  // LDS bytes of the run in plane 0
+  __device__ __forceinline__ static int row(int t, int q) { return RC ? t % R : t / (BK / 4) + (4 * NTH / BK) * q; }
+  __device__ __forceinline__ static int krun(int t, int q) { return RC ? t / R + (NTH / R) * q : t % (BK / 4); }
+  __device__ __forceinline__ void begin(int t, int64_t ld, int64_t rows) {
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      const int r = row(t, q), k = krun(t, q);
+      const uint32_t rc = (uint32_t)(r < rows ? r : rows - 1);
+      vo[q] = 4 * (RC ? rc + 4 * k * (uint32_t)ld : rc * (uint32_t)ld + 4 * k);
+      wo[q] = 2 * (r * BK + 8 * bf_chunk(r, k >> 1) + 4 * (k & 1));
+    }
+  }
+  // run q of the full stage at `base`
+  __device__ __forceinline__ void load(int q, gptr<const float> base, int64_t ld) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, -1, 0x00027000);
+    if constexpr (!RC && VEC) {
+      v[q] = __builtin_bit_cast(V4, __builtin_amdgcn_raw_buffer_load_b128(rs, vo[q], 0, 0));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[q][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, vo[q], RC ? 4 * e * (uint32_t)ld : 4 * e, 0));
+    }
+#endif
+  }
+  // run q of the stage at `base` that has nk < 32 k left, the rest zero
+  __device__ __forceinline__ void load_tail(int t, int q, gptr<const float> base, int64_t ld, int nk) {
+    const int k = 4 * krun(t, q);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[q][e] = k + e < nk ? *(gptr<const float>)((gptr<const char>)base + vo[q] + (RC ? 4 * (int64_t)e * ld : 4 * e)) : 0.0f;
+  }
+  // plane p of run q (in order 0, 1, 2): v becomes what the planes so far leave (GRun4::store3)
+  __device__ __forceinline__ void plane(int q, int p, char* S) {
+    V4& x = v[q];
+    float y[4] = {x[0], x[1], x[2], x[3]};
+    if (p == 0) {
+      const float BMAX = __uint_as_float(0x7F7F0000u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = __builtin_amdgcn_fmed3f(x[e], -BMAX, BMAX);
+    }
+    uint32_t w0 = __builtin_bit_cast(uint32_t, bf2{(__bf16)y[0], (__bf16)y[1]});
+    uint32_t w1 = __builtin_bit_cast(uint32_t, bf2{(__bf16)y[2], (__bf16)y[3]});
+    *reinterpret_cast<uint2*>(S + wo[q] + p * (R * BK * 2)) = uint2{w0, w1};
+    if (p < 2) {
+      asm("" : "+v"(w0), "+v"(w1));
+      x[0] -= __uint_as_float(w0 << 16);
+      x[1] -= __uint_as_float(w0 & 0xffff0000u);
+      x[2] -= __uint_as_float(w1 << 16);
+      x[3] -= __uint_as_float(w1 & 0xffff0000u);
+    }
+  }
+};
+
 // 3xBF16 tile of the 128-row/column shapes (128x128, 128x64, 64x128): WM x WN
 // waves of (BM/WM) x (BN/WN), each a grid of 32x32 blocks of
 // v_mfma_f32_32x32x16_bf16 (one 16-byte fragment per lane feeds twice the
 // products of a 16x16x32 fragment, so the LDS reads per product halve).  The
-// staging and the LDS image are those of bf16x3_tile ([plane][row][32 k],
-// chunks swizzled by bf_chunk); a 32x32x16 fragment of k-step h is chunk
-// 2h + lane/32 of row lane%32.  Same 6 products and two accumulators.  The
-// in-register split costs VALU work per staged element, so the larger tiles
-// (fewer staged elements per product) run more MFMAs per VALU instruction.
+// LDS image is that of bf16x3_tile ([plane][row][32 k], chunks swizzled by
+// bf_chunk); a 32x32x16 fragment of k-step h is chunk 2h + lane/32 of row lane%32.
+// Same 6 products and two accumulators.  Bound: the split's vector instructions
+// beside the products (150 to 220 a stage and wave, 24 MFMAs of 32 cycles).  So a
+// stage is one basic block in which the next stage's split runs between the MFMAs,
+// a plane of a run at a time, and each run is reloaded as soon as it is split: all
+// waves of a SIMD otherwise did their MFMAs together and then their splits together.
+// 64 products of 1024^3, 128x128 tile: 164 TF/s (987 of BF16 products); 1024 uneven
+// products in one plan 1465 us, 1378 so.
+template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool VEC>
+__device__ __forceinline__ void x3_large_loop(const GProb& P, int64_t m0, int64_t n0, int64_t kb, int64_t ke, char* smem,
+                                              f16v (&acc)[2][BM / WM / 32][BN / WN / 32]) {
+  constexpr int NTH = 64 * WM * WN, BK = 32;
+  constexpr int IB = BM / WM / 32, JB = BN / WN / 32, NB = IB * JB;  // 32x32 blocks per wave
+  constexpr int AB = 3 * BM * BK * 2, BUF = AB + 3 * BN * BK * 2;    // bytes of A's planes, of a stage
+  typedef XRuns<BM, !TA, VEC, NTH> RA;
+  typedef XRuns<BN, TB, VEC, NTH> RB;
+  const int tid = work_item_tid();
+  const int lane = tid % 64, wave = tid / 64;
+  const int l32 = lane % 32, hl = lane / 32;
+  const int64_t lda = P.lda, ldb = P.ldb;
+  gptr<const float> A = as_global(static_cast<const float*>(P.A)) + (TA ? kb + m0 * lda : m0 + kb * lda);
+  gptr<const float> B = as_global(static_cast<const float*>(P.B)) + (TB ? n0 + kb * ldb : kb + n0 * ldb);
+  const int64_t sa = TA ? BK : BK * lda, sb = TB ? BK * ldb : BK;  // from stage to stage
+  RA ra;
+  RB rb;
+  ra.begin(tid, lda, P.m - m0);
+  rb.begin(tid, ldb, P.n - n0);
+  const int nkt = (int)((ke - kb + BK - 1) / BK), nfull = (int)((ke - kb) / BK), tail = (int)((ke - kb) % BK);
+  auto load_stage = [&](int kt) JB_INLINE {
+#pragma unroll
+    for (int q = 0; q < RA::NR; ++q)
+      if (kt < nfull) ra.load(q, A + kt * sa, lda);
+      else ra.load_tail(tid, q, A + kt * sa, lda, tail);
+#pragma unroll
+    for (int q = 0; q < RB::NR; ++q)
+      if (kt < nfull) rb.load(q, B + kt * sb, ldb);
+      else rb.load_tail(tid, q, B + kt * sb, ldb, tail);
+  };
+  // fragment addresses: the two k-steps' chunks differ by an exclusive or with 2
+  const int ar = (wave % WM) * (BM / WM) + l32, br = (wave / WM) * (BN / WN) + l32;
+  const uint32_t fa[2] = {2u * (ar * BK + 8 * bf_chunk(ar, hl)), 2u * (ar * BK + 8 * bf_chunk(ar, 2 + hl))};
+  const uint32_t fb[2] = {AB + 2u * (br * BK + 8 * bf_chunk(br, hl)), AB + 2u * (br * BK + 8 * bf_chunk(br, 2 + hl))};
+  bf8 a[2][3][IB], b[2][3][JB];
+  // fragment f of k-step h, in the order the products need them: planes 0 of A and B first
+  constexpr int NF = 3 * (IB + JB);
+  auto frag = [&](const int h, const int f, const char* S) JB_INLINE {
+    const int p = f / (IB + JB), i = f % (IB + JB);
+    if (i < IB) a[h][p][i] = *reinterpret_cast<const bf8*>(S + fa[h] + (p * BM + 32 * i) * BK * 2);
+    else b[h][p][i - IB] = *reinterpret_cast<const bf8*>(S + fb[h] + (p * BN + 32 * (i - IB)) * BK * 2);
+  };
+  // product x of 6 of every block: X = op(B) plane (p -> n), Y = op(A) plane (q -> m)
+  auto mfma = [&](const int h, const int x, const int blk) JB_INLINE {
+    constexpr int PB[6] = {0, 1, 0, 2, 1, 0}, PA[6] = {0, 0, 1, 0, 1, 2};
+    const int i = blk / JB, j = blk % JB, l = x > 0;
+    acc[l][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[h][PB[x]][j], a[h][PA[x]][i], acc[l][i][j], 0, 0, 0);
+  };
+  constexpr int NM = 12 * NB, NP = 3 * (RA::NR + RB::NR);  // MFMAs and split pieces of a stage
+  // one stage; split: stage kt + 1 from the runs to the other buffer; reload: stage kt + 2 into the runs
+  auto stage = [&](const int kt, auto split, auto reload) JB_INLINE {
+    const char* S = smem + (kt & 1) * BUF;
+    char* D = smem + (~kt & 1) * BUF;
+    gptr<const float> An = A + (kt + 2) * sa, Bn = B + (kt + 2) * sb;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) frag(0, f, S);
+#pragma unroll
+    for (int x = 0; x < NM; ++x) {
+      __builtin_amdgcn_sched_barrier(0);
+      const int h = x / (6 * NB);
+      mfma(h, x % (6 * NB) / NB, x % NB);
+      if (x < NF) frag(1, x, S);
+      if constexpr (NM / 2 < NF) {
+        if (x == NM / 2 - 1)
+#pragma unroll
+          for (int f = NM / 2; f < NF; ++f) frag(1, f, S);
+      }
+      if constexpr (decltype(split)::value) {
+#pragma unroll
+        for (int y = x * NP / NM; y < (x + 1) * NP / NM; ++y) {
+          const int q = y / 3, p = y % 3;
+          if (q < RA::NR) {
+            ra.plane(q, p, D);
+            if (decltype(reload)::value && p == 2) ra.load(q, An, lda);
+          } else {
+            rb.plane(q - RA::NR, p, D + AB);
+            if (decltype(reload)::value && p == 2) rb.load(q - RA::NR, Bn, ldb);
+          }
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (decltype(split)::value) __syncthreads();
+  };
+  __syncthreads();  // LDS may still be read by the previous work item
+  load_stage(0);
+#pragma unroll
+  for (int y = 0; y < NP; ++y)
+    if (y / 3 < RA::NR) ra.plane(y / 3, y % 3, smem);
+    else rb.plane(y / 3 - RA::NR, y % 3, smem + AB);
+  typedef std::integral_constant<bool, true> Yes;
+  typedef std::integral_constant<bool, false> No;
+  int kt = 0;
+  if (nfull > 2) {
+    // (the loads in the loop's own order: its waits count them)
+#pragma unroll
+    for (int q = 0; q < RA::NR; ++q) ra.load(q, A + sa, lda);
+#pragma unroll
+    for (int q = 0; q < RB::NR; ++q) rb.load(q, B + sb, ldb);
+    __syncthreads();
+#pragma unroll 1
+    for (; kt + 2 < nfull; ++kt) stage(kt, Yes(), Yes());
+    if (kt + 2 < nkt) {
+      stage(kt, Yes(), No());
+      load_stage(kt + 2);
+      ++kt;
+    }
+  } else {
+    if (nkt > 1) load_stage(1);
+    __syncthreads();
+  }
+#pragma unroll 1
+  for (; kt + 1 < nkt; ++kt) {
+    stage(kt, Yes(), No());
+    if (kt + 2 < nkt) load_stage(kt + 2);
+  }
+  stage(kt, No(), No());
+}
+
 template <int BM, int BN, int WM, int WN, bool TA, bool TB>
 __device__ void x3_large_tile(const GProb& P, int tm, int tn, int split, char* smem, int* counters, int* sflag) {
   constexpr int NTH = 64 * WM * WN;
-  constexpr int BK = 32;
-  constexpr int RS = BK;
-  constexpr int IB = BM / WM / 32, JB = BN / WN / 32;  // 32x32 blocks per wave along m, n
+  constexpr int IB = BM / WM / 32, JB = BN / WN / 32;
   static_assert(IB >= 1 && JB >= 1 && IB * WM * 32 == BM && JB * WN * 32 == BN, "wave grid");
-  constexpr int BUF = 3 * (BM + BN) * RS;
-  typedef float f16v __attribute__((ext_vector_type(16)));
-  uint16_t* const S0 = reinterpret_cast<uint16_t*>(smem);
   const int tid = work_item_tid();
   const int lane = tid % 64, wave = tid / 64;
   const int wm0 = (wave % WM) * (BM / WM), wn0 = (wave / WM) * (BN / WN);
@@ -288,26 +434,6 @@ __device__ void x3_large_tile(const GProb& P, int tm, int tn, int split, char* s
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
   const int64_t kb = (int64_t)split * P.kchunk;
   const int64_t ke = min(P.k, kb + P.kchunk);
-  gptr<const float> A = as_global(static_cast<const float*>(P.A));
-  gptr<const float> B = as_global(static_cast<const float*>(P.B));
-  GRun4<BM, BK, !TA, NTH> la(tid);
-  GRun4<BN, BK, TB, NTH> lb(tid);
-  // stages inside the operand along k take load_kfull: k-contiguous operands in
-  // 16-byte vectors where the base is 16-byte aligned and ld a multiple of 4
-  const bool fa = m0 + BM <= P.m, fb = n0 + BN <= P.n;
-  const bool va = ((reinterpret_cast<uintptr_t>(P.A) & 15) == 0) && P.lda % 4 == 0;
-  const bool vb = ((reinterpret_cast<uintptr_t>(P.B) & 15) == 0) && P.ldb % 4 == 0;
-  la.lane_base(A, P.lda, m0, P.m);
-  lb.lane_base(B, P.ldb, n0, P.n);
-  auto load_stage = [&](int64_t k0) {
-    if (k0 + BK <= ke) {
-      la.load_kfull(P.lda, k0, va, fa);
-      lb.load_kfull(P.ldb, k0, vb, fb);
-    } else {
-      la.load(A, P.lda, m0, k0, P.m, ke);
-      lb.load(B, P.ldb, n0, k0, P.n, ke);
-    }
-  };
   f16v acc[2][IB][JB];
 #pragma unroll
   for (int l = 0; l < 2; ++l)
@@ -317,55 +443,13 @@ __device__ void x3_large_tile(const GProb& P, int tm, int tn, int split, char* s
       for (int j = 0; j < JB; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[l][i][j][e] = 0.0f;
-  const int nkt = (int)((ke - kb + BK - 1) / BK);
-  // two LDS stages, one barrier per stage, as in bf16x3_tile
-  if (nkt > 0) {
-    __syncthreads();  // LDS may still be read by the previous work item
-    load_stage(kb);
-    la.store3(S0);
-    lb.store3(S0 + 3 * BM * RS);
-    if (nkt > 1) load_stage(kb + BK);
-    __syncthreads();
-  }
-  for (int kt = 0; kt < nkt; ++kt) {
-    const uint16_t* As = S0 + (kt & 1) * BUF;
-    const uint16_t* Bs = As + 3 * BM * RS;
-#pragma unroll
-    for (int h = 0; h < BK / 16; ++h) {
-      bf8 a[3][IB], b[3][JB];
-#pragma unroll
-      for (int p = 0; p < 3; ++p) {
-#pragma unroll
-        for (int i = 0; i < IB; ++i) {
-          const int r = wm0 + 32 * i + l32;
-          a[p][i] = __builtin_bit_cast(bf8, *reinterpret_cast<const u4*>(As + (p * BM + r) * RS + 8 * bf_chunk(r, 2 * h + hl)));
-        }
-#pragma unroll
-        for (int j = 0; j < JB; ++j) {
-          const int r = wn0 + 32 * j + l32;
-          b[p][j] = __builtin_bit_cast(bf8, *reinterpret_cast<const u4*>(Bs + (p * BN + r) * RS + 8 * bf_chunk(r, 2 * h + hl)));
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < IB; ++i)
-#pragma unroll
-        for (int j = 0; j < JB; ++j) {
-          // X = op(B) plane (p -> n), Y = op(A) plane (q -> m)
-          acc[0][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[0][j], a[0][i], acc[0][i][j], 0, 0, 0);
-          acc[1][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[1][j], a[0][i], acc[1][i][j], 0, 0, 0);
-          acc[1][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[0][j], a[1][i], acc[1][i][j], 0, 0, 0);
-          acc[1][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[2][j], a[0][i], acc[1][i][j], 0, 0, 0);
-          acc[1][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[1][j], a[1][i], acc[1][i][j], 0, 0, 0);
-          acc[1][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[0][j], a[2][i], acc[1][i][j], 0, 0, 0);
-        }
-    }
-    if (kt + 1 < nkt) {
-      uint16_t* nxt = S0 + ((kt + 1) & 1) * BUF;  // last read in stage kt-1, before the previous barrier
-      la.store3(nxt);
-      lb.store3(nxt + 3 * BM * RS);
-      if (kt + 2 < nkt) load_stage(kb + (int64_t)(kt + 2) * BK);
-    }
-    __syncthreads();
+  if (kb < ke) {
+    // k-contiguous operands come in 16-byte vectors where every one has its base 16-byte
+    // aligned and ld a multiple of 4
+    const bool va = !TA || ((reinterpret_cast<uintptr_t>(P.A) & 15) == 0 && P.lda % 4 == 0);
+    const bool vb = TB || ((reinterpret_cast<uintptr_t>(P.B) & 15) == 0 && P.ldb % 4 == 0);
+    if ((!TA && TB) || (va && vb)) x3_large_loop<BM, BN, WM, WN, TA, TB, true>(P, m0, n0, kb, ke, smem, acc);
+    else x3_large_loop<BM, BN, WM, WN, TA, TB, false>(P, m0, n0, kb, ke, smem, acc);
   }
   // item e of lane l in block (i, j): row wm0 + 32 i + l%32, column wn0 + 32 j + 8 (e/4) + 4 (l/32) + e%4
 #pragma unroll
@@ -775,7 +859,7 @@ GroupedKernel launch_kernel(int kind, int L) {
 // Byte offsets inside an operand stage (up to 128 rows or 32 k of ld elements) past 32 bits.
 bool wide_ld(int kind, const GProb& g) {
   const int64_t lim = ((int64_t)1 << 32) / (128 * (kind == 0 ? 8 : 4));
-  return kind != 2 && std::max(g.lda, g.ldb) >= lim;
+  return (kind != 2 || large_cfg(g.cfg)) && std::max(g.lda, g.ldb) >= lim;
 }
 
 // The ring tile (k_grouped_ring.h) of a native problem, and the extent of the work
@@ -1537,7 +1621,7 @@ static bool pullback_big(const jb_gemm_desc& d) {
 // Every adjoint runs on the single-problem kernels, one after the other on `s`,
 // without synchronising.  (The small ones shared a one-shot grouped launch before: its
 // lists' allocation and upload, its streams and its synchronisation took 150 us for the
-// two products of a 512 x 384 x 256 layer, which take 25 us here.)
+// two products of a 512 x 384 x 256 layer, which take 15 us here.)
 static int pullback_run_locked(int method, const std::vector<jb_gemm_desc>& d, hipStream_t s) {
   std::vector<jb_gemm_desc> small;
   for (const jb_gemm_desc& x : d)
