@@ -45,15 +45,27 @@ struct GroupedKernel {
   int threads;
 };
 // The persistent kernels of the native methods' MFMA tiles (k_grouped_ring.h) for
-// transpose combination 2 ta + tb: `which` tile, with 16-byte (vec) or 4-byte
-// operand loads, or, for leading dimensions past 32-bit offsets, 64x64 tiles.
-GroupedKernelFn grouped_ring_f64_vec(int which, int combo);
+// transpose combination 2 ta + tb: `which` tile, or, for leading dimensions past
+// 32-bit offsets, 64x64 tiles.
 GroupedKernelFn grouped_ring_f64(int which, int combo);
 GroupedKernelFn grouped_ring_f64_wide_ld(int combo);
-GroupedKernelFn grouped_ring_f32(int which, int combo, bool vec);
+GroupedKernelFn grouped_ring_f32(int which, int combo);
 GroupedKernelFn grouped_ring_f32_wide_ld(int combo);
+// Those of the 3xBF16 method (k_grouped_x3.hip): 128x128, 128x64, 64x128, 64x64 items.
+GroupedKernel grouped_x3(int which, int combo);
+GroupedKernelFn grouped_x3_wide_ld(int combo);
 
 namespace {
+
+// The thread index as an opaque value, read once per work item: offsets derived
+// from it are then formed inside the work loop of the persistent kernel rather
+// than hoisted out of it and held in registers for all eight tile variants at
+// once (which exhausts the register file).
+__device__ __forceinline__ int work_item_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
 
 // Result element (i, j) of tile (tm, tn): with one split it goes straight to
 // C through the alpha/beta epilogue, otherwise to this split's partial slab.
@@ -94,8 +106,9 @@ __device__ void splitk_combine(const GProb& P, int tm, int tn, int BN, int* coun
   gptr<T> C = as_global(static_cast<T*>(P.C));
   const T alpha = (T)P.alpha, beta = (T)P.beta;
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  constexpr int U = 4;  // loads in flight per thread; tiles have a multiple of 32 columns
-  static_assert(BM * 32 % (U * NTH) == 0, "whole groups of loads");
+  // loads in flight per thread (64- and 128-row tiles have a multiple of 64 columns, the 32-row one 32)
+  constexpr int U = BM == 32 ? 4 : 16;
+  static_assert(BM * (BM == 32 ? 32 : 64) % (U * NTH) == 0, "whole groups of loads");
   for (int e = threadIdx.x; e < BM * BN; e += U * NTH) {
     T s[U];
 #pragma unroll

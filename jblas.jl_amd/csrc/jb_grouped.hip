@@ -9,10 +9,9 @@
 //   * work items (problem, output tile, k-split) sorted by decreasing cost
 //     are pulled from a device counter by a grid of CU-filling workgroups,
 //     so uneven problems load-balance;
-//   * the native methods' MFMA tiles run in persistent kernels per tile shape,
-//     transpose combination and load width (k_grouped_ring.h), the 3xBF16
-//     128-row/column tiles per shape and combination, the other 3xBF16 tiles and
-//     the small problems in one more; a plan's kernels run concurrently;
+//   * the MFMA tiles run in persistent kernels per tile shape and transpose
+//     combination (k_grouped_ring.h, k_grouped_x3.hip), the small problems in one
+//     more; a plan's kernels run concurrently;
 //   * split-K partials go to a workspace slot per (tile, split); the last
 //     split to finish (per-tile arrival counter) sums them in split order,
 //     so results are deterministic;
@@ -34,434 +33,6 @@
 
 namespace jb {
 namespace {
-
-typedef double d4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef float f16v __attribute__((ext_vector_type(16)));
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-
-#define JB_INLINE __attribute__((always_inline))  // lambdas of the kernels: never outlined
-
-// The thread index as an opaque value, read once per work item: offsets derived
-// from it are then formed inside the work loop of the persistent kernel rather
-// than hoisted out of it and held in registers for all eight tile variants at
-// once (which exhausts the register file).
-__device__ __forceinline__ int work_item_tid() {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t;
-}
-
-typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-
-// LDS rows of the 3xBF16 tile hold BK = 32 BF16 (64 bytes, four 16-byte chunks,
-// no padding); chunk c of row r is stored at chunk c ^ ((r >> 2) & 3), so the 16
-// rows that one 16-byte fragment read covers (same c) hit 16 distinct 4-bank
-// groups of the 64-bank LDS.
-__device__ __forceinline__ int bf_chunk(int r, int c) { return c ^ ((r >> 2) & 3); }
-
-// FP32 operand staging of the 3xBF16 tile in runs of four consecutive k of one
-// row (R x BK tile, NR runs per thread, NTH threads), split into hi/mid/lo BF16
-// planes ([plane][row][BK], chunks swizzled) with one 8-byte LDS store per plane
-// and run.
-//   RC (rows contiguous): run q of thread t is row t % R, k-run t / R + (NTH / R) q
-//   otherwise:            row t / (BK / 4) + (4 NTH / BK) q, k-run t % (BK / 4)
-// Lanes with consecutive t take consecutive addresses of the contiguous index.
-template <int R, int BK, bool RC, int NTH = GNT>
-struct GRun4 {
-  static constexpr int NR = R * BK / (4 * NTH);
-  static_assert(NR >= 1 && R * BK == 4 * NTH * NR, "tile must split into whole runs per thread");
-  static_assert(RC ? (NTH % R == 0 && (NTH / R) * NR == BK / 4) : ((4 * NTH / BK) * NR == R), "run map");
-  typedef float V4 __attribute__((ext_vector_type(4)));
-  float v[NR][4];
-  int tid;
-  __device__ explicit GRun4(int t) : tid(t) {}
-  __device__ __forceinline__ int row(int q) const { return RC ? tid % R : tid / (BK / 4) + (4 * NTH / BK) * q; }
-  __device__ __forceinline__ int krun(int q) const { return RC ? tid / R + (NTH / R) * q : tid % (BK / 4); }
-  __device__ __forceinline__ void load(gptr<const float> P, int64_t ld, int64_t r0, int64_t k0, int64_t Rtot,
-                                       int64_t Kend) {
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      const int64_t gr = r0 + row(q), gk = k0 + 4 * krun(q);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[q][e] = (gr < Rtot && gk + e < Kend) ? (RC ? P[gr + (gk + e) * ld] : P[gk + e + gr * ld]) : 0.0f;
-    }
-  }
-  // x = hi + mid + lo + rest: each plane is x rounded to BF16 (nearest even,
-  // v_cvt_pk_bf16_f32), subtracted exactly before the next plane.
-  __device__ __forceinline__ void store3(uint16_t* S) const {
-    static_assert(BK == 32, "four 16-byte chunks per LDS row");
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      float x[4] = {v[q][0], v[q][1], v[q][2], v[q][3]};
-      const int r = row(q), kr = krun(q);
-      uint16_t* dst = S + r * BK + 8 * bf_chunk(r, kr >> 1) + 4 * (kr & 1);
-      // |x| within half a BF16 ulp of FLT_MAX rounds to Inf: the first plane
-      // rounds x clamped to the largest finite BF16, which for such an x is
-      // its truncation (the residual then has at most 16 significant bits and
-      // the split stays exact, as in the single-problem split) and for every
-      // other finite x changes nothing.  An Inf or NaN x still leaves a NaN
-      // residual, so every product it enters is NaN.
-      const float BMAX = __uint_as_float(0x7F7F0000u);
-#pragma unroll
-      for (int p = 0; p < 3; ++p) {
-        float y[4] = {x[0], x[1], x[2], x[3]};
-        if (p == 0) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) y[e] = __builtin_amdgcn_fmed3f(x[e], -BMAX, BMAX);
-        }
-        uint32_t w0 = __builtin_bit_cast(uint32_t, bf2{(__bf16)y[0], (__bf16)y[1]});
-        uint32_t w1 = __builtin_bit_cast(uint32_t, bf2{(__bf16)y[2], (__bf16)y[3]});
-        *reinterpret_cast<uint2*>(dst + p * R * BK) = uint2{w0, w1};
-        if (p < 2) {
-          // the packed BF16 values back in FP32 (low half shifted up, high half
-          // masked): one packed conversion per two elements and plane.  Written
-          // as (float) of each BF16, or with w0, w1 visible to the compiler, it
-          // converted each low element a second time on its own; the empty asm
-          // hides where w0 and w1 came from.
-          asm("" : "+v"(w0), "+v"(w1));
-          x[0] -= __uint_as_float(w0 << 16);
-          x[1] -= __uint_as_float(w0 & 0xffff0000u);
-          x[2] -= __uint_as_float(w1 << 16);
-          x[3] -= __uint_as_float(w1 & 0xffff0000u);
-        }
-      }
-    }
-  }
-};
-
-// 3xBF16 tile for FP32 operands: the staged FP32 tile is split into hi/mid/lo
-// BF16 planes in LDS ([plane][row][32 k]); v_mfma_f32_16x16x32_bf16 computes the
-// 6 products t+u <= 4, level 2 in one accumulator and the rest in another.
-template <int BM, int BN, bool TA, bool TB>
-__device__ void bf16x3_tile(const GProb& P, int tm, int tn, int split, char* smem, int* counters, int* sflag) {
-  constexpr int BK = 32;
-  constexpr int RS = BK;  // bf16 per LDS row
-  constexpr int IM = BM / 32, JN = BN / 32;
-  constexpr int BUF = 3 * (BM + BN) * RS;  // one stage: A planes [3][BM][RS], then B planes [3][BN][RS]
-  uint16_t* const S0 = reinterpret_cast<uint16_t*>(smem);
-  const int tid = work_item_tid();
-  const int lane = tid % 64, wave = tid / 64;
-  const int wm0 = (wave % 2) * (BM / 2), wn0 = (wave / 2) * (BN / 2);
-  const int g = lane / 16, l16 = lane % 16;
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  const int64_t kb = (int64_t)split * P.kchunk;
-  const int64_t ke = min(P.k, kb + P.kchunk);
-  gptr<const float> A = as_global(static_cast<const float*>(P.A));
-  gptr<const float> B = as_global(static_cast<const float*>(P.B));
-  GRun4<BM, BK, !TA> la(tid);
-  GRun4<BN, BK, TB> lb(tid);
-  f4 acc[2][IM][JN];
-#pragma unroll
-  for (int l = 0; l < 2; ++l)
-#pragma unroll
-    for (int i = 0; i < IM; ++i)
-#pragma unroll
-      for (int j = 0; j < JN; ++j) acc[l][i][j] = f4{0, 0, 0, 0};
-  const int nkt = (int)((ke - kb + BK - 1) / BK);
-  // Two LDS stages.  Stage kt+1 is split into the other buffer after stage
-  // kt's products are issued, and stage kt+2 is then loaded into the freed
-  // registers, so a load has a whole stage to arrive; one barrier per stage.
-  if (nkt > 0) {
-    __syncthreads();  // LDS may still be read by the previous work item
-    la.load(A, P.lda, m0, kb, P.m, ke);
-    lb.load(B, P.ldb, n0, kb, P.n, ke);
-    la.store3(S0);
-    lb.store3(S0 + 3 * BM * RS);
-    if (nkt > 1) {
-      la.load(A, P.lda, m0, kb + BK, P.m, ke);
-      lb.load(B, P.ldb, n0, kb + BK, P.n, ke);
-    }
-    __syncthreads();
-  }
-  for (int kt = 0; kt < nkt; ++kt) {
-    const uint16_t* As = S0 + (kt & 1) * BUF;
-    const uint16_t* Bs = As + 3 * BM * RS;
-    bf8 a[3][IM], b[3][JN];
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-#pragma unroll
-      for (int i = 0; i < IM; ++i)
-        a[p][i] = __builtin_bit_cast(bf8, *reinterpret_cast<const u4*>(As + (p * BM + wm0 + 16 * i + l16) * RS +
-                                                                          8 * bf_chunk(l16, g)));
-#pragma unroll
-      for (int j = 0; j < JN; ++j)
-        b[p][j] = __builtin_bit_cast(bf8, *reinterpret_cast<const u4*>(Bs + (p * BN + wn0 + 16 * j + l16) * RS +
-                                                                          8 * bf_chunk(l16, g)));
-    }
-#pragma unroll
-    for (int i = 0; i < IM; ++i)
-#pragma unroll
-      for (int j = 0; j < JN; ++j) {
-        // X = op(B) plane (p -> n), Y = op(A) plane (q -> m)
-        acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[0][j], a[0][i], acc[0][i][j], 0, 0, 0);
-        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[1][j], a[0][i], acc[1][i][j], 0, 0, 0);
-        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[0][j], a[1][i], acc[1][i][j], 0, 0, 0);
-        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[2][j], a[0][i], acc[1][i][j], 0, 0, 0);
-        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[1][j], a[1][i], acc[1][i][j], 0, 0, 0);
-        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[0][j], a[2][i], acc[1][i][j], 0, 0, 0);
-      }
-    if (kt + 1 < nkt) {
-      uint16_t* nxt = S0 + ((kt + 1) & 1) * BUF;  // last read in stage kt-1, before the previous barrier
-      la.store3(nxt);
-      lb.store3(nxt + 3 * BM * RS);
-      if (kt + 2 < nkt) {
-        la.load(A, P.lda, m0, kb + (int64_t)(kt + 2) * BK, P.m, ke);
-        lb.load(B, P.ldb, n0, kb + (int64_t)(kt + 2) * BK, P.n, ke);
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < IM; ++i)
-#pragma unroll
-    for (int j = 0; j < JN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        put_result<float, BM, BN>(P, tm, tn, split, wm0 + 16 * i + l16, wn0 + 16 * j + 4 * g + r,
-                                  acc[0][i][j][r] + acc[1][i][j][r]);
-  splitk_combine<float, BM, GNT>(P, tm, tn, BN, counters, sflag);
-}
-
-// One operand's stages of the 128-row/column 3xBF16 tiles, in the run map of GRun4: raw
-// FP32 runs of four k in registers, loaded through a buffer descriptor (the stage's base
-// in scalar registers, one lane offset per run), then split plane by plane.  Rows past
-// the operand read its last row: they meet only rows or columns outside C.
-template <int R, bool RC, bool VEC, int NTH>
-struct XRuns {
-  static constexpr int BK = 32, NR = R * BK / (4 * NTH);
-  static_assert(R * BK == 4 * NTH * NR && (!RC || NTH % R == 0), "run map");
-  typedef float V4 __attribute__((ext_vector_type(4)));
-  V4 v[NR];
-  uint32_t vo[NR];  // bytes from the stage's base
-  uint32_t wo[NR];  // LDS bytes of the run in plane 0
-  __device__ __forceinline__ static int row(int t, int q) { return RC ? t % R : t / (BK / 4) + (4 * NTH / BK) * q; }
-  __device__ __forceinline__ static int krun(int t, int q) { return RC ? t / R + (NTH / R) * q : t % (BK / 4); }
-  __device__ __forceinline__ void begin(int t, int64_t ld, int64_t rows) {
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      const int r = row(t, q), k = krun(t, q);
-      const uint32_t rc = (uint32_t)(r < rows ? r : rows - 1);
-      vo[q] = 4 * (RC ? rc + 4 * k * (uint32_t)ld : rc * (uint32_t)ld + 4 * k);
-      wo[q] = 2 * (r * BK + 8 * bf_chunk(r, k >> 1) + 4 * (k & 1));
-    }
-  }
-  // run q of the full stage at `base`
-  __device__ __forceinline__ void load(int q, gptr<const float> base, int64_t ld) {
-#ifdef __HIP_DEVICE_COMPILE__
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, -1, 0x00027000);
-    if constexpr (!RC && VEC) {
-      v[q] = __builtin_bit_cast(V4, __builtin_amdgcn_raw_buffer_load_b128(rs, vo[q], 0, 0));
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[q][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, vo[q], RC ? 4 * e * (uint32_t)ld : 4 * e, 0));
-    }
-#endif
-  }
-  // run q of the stage at `base` that has nk < 32 k left, the rest zero
-  __device__ __forceinline__ void load_tail(int t, int q, gptr<const float> base, int64_t ld, int nk) {
-    const int k = 4 * krun(t, q);
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      v[q][e] = k + e < nk ? *(gptr<const float>)((gptr<const char>)base + vo[q] + (RC ? 4 * (int64_t)e * ld : 4 * e)) : 0.0f;
-  }
-  // plane p of run q (in order 0, 1, 2): v becomes what the planes so far leave (GRun4::store3)
-  __device__ __forceinline__ void plane(int q, int p, char* S) {
-    V4& x = v[q];
-    float y[4] = {x[0], x[1], x[2], x[3]};
-    if (p == 0) {
-      const float BMAX = __uint_as_float(0x7F7F0000u);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) y[e] = __builtin_amdgcn_fmed3f(x[e], -BMAX, BMAX);
-    }
-    uint32_t w0 = __builtin_bit_cast(uint32_t, bf2{(__bf16)y[0], (__bf16)y[1]});
-    uint32_t w1 = __builtin_bit_cast(uint32_t, bf2{(__bf16)y[2], (__bf16)y[3]});
-    *reinterpret_cast<uint2*>(S + wo[q] + p * (R * BK * 2)) = uint2{w0, w1};
-    if (p < 2) {
-      asm("" : "+v"(w0), "+v"(w1));
-      x[0] -= __uint_as_float(w0 << 16);
-      x[1] -= __uint_as_float(w0 & 0xffff0000u);
-      x[2] -= __uint_as_float(w1 << 16);
-      x[3] -= __uint_as_float(w1 & 0xffff0000u);
-    }
-  }
-};
-
-// 3xBF16 tile of the 128-row/column shapes (128x128, 128x64, 64x128): WM x WN
-// waves of (BM/WM) x (BN/WN), each a grid of 32x32 blocks of
-// v_mfma_f32_32x32x16_bf16 (one 16-byte fragment per lane feeds twice the
-// products of a 16x16x32 fragment, so the LDS reads per product halve).  The
-// LDS image is that of bf16x3_tile ([plane][row][32 k], chunks swizzled by
-// bf_chunk); a 32x32x16 fragment of k-step h is chunk 2h + lane/32 of row lane%32.
-// Same 6 products and two accumulators.  Bound: the split's vector instructions
-// beside the products (150 to 220 a stage and wave, 24 MFMAs of 32 cycles).  So a
-// stage is one basic block in which the next stage's split runs between the MFMAs,
-// a plane of a run at a time, and each run is reloaded as soon as it is split: all
-// waves of a SIMD otherwise did their MFMAs together and then their splits together.
-// 64 products of 1024^3, 128x128 tile: 164 TF/s (987 of BF16 products); 1024 uneven
-// products in one plan 1465 us, 1378 so.
-template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool VEC>
-__device__ __forceinline__ void x3_large_loop(const GProb& P, int64_t m0, int64_t n0, int64_t kb, int64_t ke, char* smem,
-                                              f16v (&acc)[2][BM / WM / 32][BN / WN / 32]) {
-  constexpr int NTH = 64 * WM * WN, BK = 32;
-  constexpr int IB = BM / WM / 32, JB = BN / WN / 32, NB = IB * JB;  // 32x32 blocks per wave
-  constexpr int AB = 3 * BM * BK * 2, BUF = AB + 3 * BN * BK * 2;    // bytes of A's planes, of a stage
-  typedef XRuns<BM, !TA, VEC, NTH> RA;
-  typedef XRuns<BN, TB, VEC, NTH> RB;
-  const int tid = work_item_tid();
-  const int lane = tid % 64, wave = tid / 64;
-  const int l32 = lane % 32, hl = lane / 32;
-  const int64_t lda = P.lda, ldb = P.ldb;
-  gptr<const float> A = as_global(static_cast<const float*>(P.A)) + (TA ? kb + m0 * lda : m0 + kb * lda);
-  gptr<const float> B = as_global(static_cast<const float*>(P.B)) + (TB ? n0 + kb * ldb : kb + n0 * ldb);
-  const int64_t sa = TA ? BK : BK * lda, sb = TB ? BK * ldb : BK;  // from stage to stage
-  RA ra;
-  RB rb;
-  ra.begin(tid, lda, P.m - m0);
-  rb.begin(tid, ldb, P.n - n0);
-  const int nkt = (int)((ke - kb + BK - 1) / BK), nfull = (int)((ke - kb) / BK), tail = (int)((ke - kb) % BK);
-  auto load_stage = [&](int kt) JB_INLINE {
-#pragma unroll
-    for (int q = 0; q < RA::NR; ++q)
-      if (kt < nfull) ra.load(q, A + kt * sa, lda);
-      else ra.load_tail(tid, q, A + kt * sa, lda, tail);
-#pragma unroll
-    for (int q = 0; q < RB::NR; ++q)
-      if (kt < nfull) rb.load(q, B + kt * sb, ldb);
-      else rb.load_tail(tid, q, B + kt * sb, ldb, tail);
-  };
-  // fragment addresses: the two k-steps' chunks differ by an exclusive or with 2
-  const int ar = (wave % WM) * (BM / WM) + l32, br = (wave / WM) * (BN / WN) + l32;
-  const uint32_t fa[2] = {2u * (ar * BK + 8 * bf_chunk(ar, hl)), 2u * (ar * BK + 8 * bf_chunk(ar, 2 + hl))};
-  const uint32_t fb[2] = {AB + 2u * (br * BK + 8 * bf_chunk(br, hl)), AB + 2u * (br * BK + 8 * bf_chunk(br, 2 + hl))};
-  bf8 a[2][3][IB], b[2][3][JB];
-  // fragment f of k-step h, in the order the products need them: planes 0 of A and B first
-  constexpr int NF = 3 * (IB + JB);
-  auto frag = [&](const int h, const int f, const char* S) JB_INLINE {
-    const int p = f / (IB + JB), i = f % (IB + JB);
-    if (i < IB) a[h][p][i] = *reinterpret_cast<const bf8*>(S + fa[h] + (p * BM + 32 * i) * BK * 2);
-    else b[h][p][i - IB] = *reinterpret_cast<const bf8*>(S + fb[h] + (p * BN + 32 * (i - IB)) * BK * 2);
-  };
-  // product x of 6 of every block: X = op(B) plane (p -> n), Y = op(A) plane (q -> m)
-  auto mfma = [&](const int h, const int x, const int blk) JB_INLINE {
-    constexpr int PB[6] = {0, 1, 0, 2, 1, 0}, PA[6] = {0, 0, 1, 0, 1, 2};
-    const int i = blk / JB, j = blk % JB, l = x > 0;
-    acc[l][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[h][PB[x]][j], a[h][PA[x]][i], acc[l][i][j], 0, 0, 0);
-  };
-  constexpr int NM = 12 * NB, NP = 3 * (RA::NR + RB::NR);  // MFMAs and split pieces of a stage
-  // one stage; split: stage kt + 1 from the runs to the other buffer; reload: stage kt + 2 into the runs
-  auto stage = [&](const int kt, auto split, auto reload) JB_INLINE {
-    const char* S = smem + (kt & 1) * BUF;
-    char* D = smem + (~kt & 1) * BUF;
-    gptr<const float> An = A + (kt + 2) * sa, Bn = B + (kt + 2) * sb;
-#pragma unroll
-    for (int f = 0; f < NF; ++f) frag(0, f, S);
-#pragma unroll
-    for (int x = 0; x < NM; ++x) {
-      __builtin_amdgcn_sched_barrier(0);
-      const int h = x / (6 * NB);
-      mfma(h, x % (6 * NB) / NB, x % NB);
-      if (x < NF) frag(1, x, S);
-      if constexpr (NM / 2 < NF) {
-        if (x == NM / 2 - 1)
-#pragma unroll
-          for (int f = NM / 2; f < NF; ++f) frag(1, f, S);
-      }
-      if constexpr (decltype(split)::value) {
-#pragma unroll
-        for (int y = x * NP / NM; y < (x + 1) * NP / NM; ++y) {
-          const int q = y / 3, p = y % 3;
-          if (q < RA::NR) {
-            ra.plane(q, p, D);
-            if (decltype(reload)::value && p == 2) ra.load(q, An, lda);
-          } else {
-            rb.plane(q - RA::NR, p, D + AB);
-            if (decltype(reload)::value && p == 2) rb.load(q - RA::NR, Bn, ldb);
-          }
-        }
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (decltype(split)::value) __syncthreads();
-  };
-  __syncthreads();  // LDS may still be read by the previous work item
-  load_stage(0);
-#pragma unroll
-  for (int y = 0; y < NP; ++y)
-    if (y / 3 < RA::NR) ra.plane(y / 3, y % 3, smem);
-    else rb.plane(y / 3 - RA::NR, y % 3, smem + AB);
-  typedef std::integral_constant<bool, true> Yes;
-  typedef std::integral_constant<bool, false> No;
-  int kt = 0;
-  if (nfull > 2) {
-    // (the loads in the loop's own order: its waits count them)
-#pragma unroll
-    for (int q = 0; q < RA::NR; ++q) ra.load(q, A + sa, lda);
-#pragma unroll
-    for (int q = 0; q < RB::NR; ++q) rb.load(q, B + sb, ldb);
-    __syncthreads();
-#pragma unroll 1
-    for (; kt + 2 < nfull; ++kt) stage(kt, Yes(), Yes());
-    if (kt + 2 < nkt) {
-      stage(kt, Yes(), No());
-      load_stage(kt + 2);
-      ++kt;
-    }
-  } else {
-    if (nkt > 1) load_stage(1);
-    __syncthreads();
-  }
-#pragma unroll 1
-  for (; kt + 1 < nkt; ++kt) {
-    stage(kt, Yes(), No());
-    if (kt + 2 < nkt) load_stage(kt + 2);
-  }
-  stage(kt, No(), No());
-}
-
-template <int BM, int BN, int WM, int WN, bool TA, bool TB>
-__device__ void x3_large_tile(const GProb& P, int tm, int tn, int split, char* smem, int* counters, int* sflag) {
-  constexpr int NTH = 64 * WM * WN;
-  constexpr int IB = BM / WM / 32, JB = BN / WN / 32;
-  static_assert(IB >= 1 && JB >= 1 && IB * WM * 32 == BM && JB * WN * 32 == BN, "wave grid");
-  const int tid = work_item_tid();
-  const int lane = tid % 64, wave = tid / 64;
-  const int wm0 = (wave % WM) * (BM / WM), wn0 = (wave / WM) * (BN / WN);
-  const int l32 = lane % 32, hl = lane / 32;
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  const int64_t kb = (int64_t)split * P.kchunk;
-  const int64_t ke = min(P.k, kb + P.kchunk);
-  f16v acc[2][IB][JB];
-#pragma unroll
-  for (int l = 0; l < 2; ++l)
-#pragma unroll
-    for (int i = 0; i < IB; ++i)
-#pragma unroll
-      for (int j = 0; j < JB; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[l][i][j][e] = 0.0f;
-  if (kb < ke) {
-    // k-contiguous operands come in 16-byte vectors where every one has its base 16-byte
-    // aligned and ld a multiple of 4
-    const bool va = !TA || ((reinterpret_cast<uintptr_t>(P.A) & 15) == 0 && P.lda % 4 == 0);
-    const bool vb = TB || ((reinterpret_cast<uintptr_t>(P.B) & 15) == 0 && P.ldb % 4 == 0);
-    if ((!TA && TB) || (va && vb)) x3_large_loop<BM, BN, WM, WN, TA, TB, true>(P, m0, n0, kb, ke, smem, acc);
-    else x3_large_loop<BM, BN, WM, WN, TA, TB, false>(P, m0, n0, kb, ke, smem, acc);
-  }
-  // item e of lane l in block (i, j): row wm0 + 32 i + l%32, column wn0 + 32 j + 8 (e/4) + 4 (l/32) + e%4
-#pragma unroll
-  for (int i = 0; i < IB; ++i)
-#pragma unroll
-    for (int j = 0; j < JB; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        put_result<float, BM, BN>(P, tm, tn, split, wm0 + 32 * i + l32, wn0 + 32 * j + 8 * (e / 4) + 4 * hl + e % 4,
-                                  acc[0][i][j][e] + acc[1][i][j][e]);
-  splitk_combine<float, BM, NTH>(P, tm, tn, BN, counters, sflag);
-}
 
 // Small problem (m, n, k <= 64) in one work item, the form of fastmul!
 // (src/kernels.jl:202-208, kernel_quote :42-201): no MFMA tile; lane = row of C
@@ -591,73 +162,23 @@ __device__ __forceinline__ void run_small(const GProb& P, int combo, char* smem)
   }
 }
 
-// The small items of the native methods (T = double or float), and the 3xBF16
-// method's 64x64, 32x32 and small items.
-template <int BM>
-__device__ __forceinline__ void run_x3_combo(const GProb& P, int combo, int tm, int tn, int split, char* smem,
-                                             int* counters, int* sflag) {
-  switch (combo) {
-    case 0: bf16x3_tile<BM, BM, false, false>(P, tm, tn, split, smem, counters, sflag); break;
-    case 1: bf16x3_tile<BM, BM, false, true>(P, tm, tn, split, smem, counters, sflag); break;
-    case 2: bf16x3_tile<BM, BM, true, false>(P, tm, tn, split, smem, counters, sflag); break;
-    default: bf16x3_tile<BM, BM, true, true>(P, tm, tn, split, smem, counters, sflag); break;
-  }
-}
-
-// KIND 0: FP64 native, 1: FP32 native (small items only), 2: FP32 3xBF16.
+// The small items.  KIND 0: FP64, 1: FP32.
 template <int KIND>
 __global__ __launch_bounds__(GNT, 2) void grouped_kernel(const GProb* __restrict__ probs, const GItem* __restrict__ items,
                                                          const int* __restrict__ qdesc, int* __restrict__ qnext,
-                                                         int* __restrict__ counters) {
+                                                         int* __restrict__) {
   constexpr int E = KIND == 0 ? 8 : 4;
-  constexpr int SMEM = (KIND == 2) ? (2 * 3 * (64 + 64) * 32 * 2) : 64 * (64 + 16 / E) * E;
-  __shared__ __attribute__((aligned(16))) char smem[SMEM];
-  static_assert(SMEM >= 64 * (64 + 16 / E) * E, "small path stages op(B) in LDS");
-  __shared__ int s_item, s_flag;
+  __shared__ __attribute__((aligned(16))) char smem[64 * (64 + 16 / E) * E];  // op(B)
+  __shared__ int s_item;
   int q = blockIdx.x % NXCD, tries = 0;
   for (;;) {
-    const int it = pop_item(qdesc, qnext, q, tries, &s_item);
+    const int it = pop_item(qdesc, qnext, q, tries, &s_item);  // its barriers: the previous item's op(B) is read
     if (it < 0) break;
-    const GItem w = items[it];
-    const GProb P = probs[w.prob];
-    const int combo = (P.ta ? 2 : 0) + (P.tb ? 1 : 0);
-    if (KIND == 2 && P.cfg != CFG_SMALL) {
-      const int tm = w.tile / P.tiles_n, tn = w.tile % P.tiles_n;
-      if (P.cfg == 0) run_x3_combo<64>(P, combo, tm, tn, w.split, smem, counters, &s_flag);
-      else run_x3_combo<32>(P, combo, tm, tn, w.split, smem, counters, &s_flag);
-    } else {
-      __syncthreads();  // the previous item's op(B) may still be read
-      run_small<KIND>(P, combo, smem);
-    }
+    const GProb P = probs[items[it].prob];
+    run_small<KIND>(P, (P.ta ? 2 : 0) + (P.tb ? 1 : 0), smem);
   }
 }
 
-// The 3xBF16 counterpart: items of one 128-row/column tile shape and transpose
-// combination.  LDS: two stages of three BF16 planes of (BM + BN) rows x 32 k.
-// 128x64 and 64x128: four waves of 64x32 / 32x64, 72 KB (two workgroups per
-// CU); 128x128: eight waves of 64x32, 96 KB (one workgroup of 8 waves per CU).
-template <int BM, int BN> struct X3Waves {
-  static constexpr int WM = 2, WN = (BM == 128 && BN == 128) ? 4 : 2;
-  static constexpr int NTH = 64 * WM * WN;
-  static constexpr int MINB = NTH > GNT ? 1 : 2;  // workgroups per CU for the register budget
-};
-template <int BM, int BN, bool TA, bool TB>
-__global__ __launch_bounds__((X3Waves<BM, BN>::NTH), (X3Waves<BM, BN>::MINB))
-void grouped_large_x3_kernel(const GProb* __restrict__ probs, const GItem* __restrict__ items,
-                             const int* __restrict__ qdesc, int* __restrict__ qnext, int* __restrict__ counters) {
-  constexpr int SMEM = 2 * 3 * (BM + BN) * 32 * 2;
-  __shared__ __attribute__((aligned(16))) char smem[SMEM];
-  __shared__ int s_item, s_flag;
-  int q = blockIdx.x % NXCD, tries = 0;
-  for (;;) {
-    const int it = pop_item(qdesc, qnext, q, tries, &s_item);
-    if (it < 0) break;
-    const GItem w = items[it];
-    const GProb P = probs[w.prob];
-    const int tm = w.tile / P.tiles_n, tn = w.tile % P.tiles_n;
-    x3_large_tile<BM, BN, X3Waves<BM, BN>::WM, X3Waves<BM, BN>::WN, TA, TB>(P, tm, tn, w.split, smem, counters, &s_flag);
-  }
-}
 
 __global__ void zero_i32_kernel(int* p, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
@@ -701,17 +222,30 @@ std::string bucket_key(int method, int64_t m, int64_t n, int64_t k) {
 // otherwise, for FP64, the tile with the least padded area per unit of
 // measured throughput (TILE_RATE: each tile's FP64 rate on groups of
 // 1024 x 1024 problems with k = 256 and 1024, relative to the 128x128 tile);
-// for 3xBF16 the 64x128 tile (its split in registers makes every tile shape
-// cost about the same per staged element: on the 1024-problem log-uniform set
-// the 64x128 tile for every problem ran 7 % (NN) to 24 % (TN) faster than the
-// 64x64 / 32x32 rule and within 2 % of the best single shape per transpose
-// combination except NT, where 128x128 is 7.6 % faster -- a choice the tuner
-// can make); for native FP32 the 64x64 tile from max(m, n) >= 96, else 32x32.
+// for 3xBF16 the 64x128 tile (plan_choices refines it for large groups);
+// for native FP32 the 64x64 tile from max(m, n) >= 96, else 32x32.
 // Split-K is not chosen per problem: plan_build splits the longest work items
 // when the whole group has fewer work items than the device holds workgroups
 // (the blocking decision that depends on the device, blocking_structure's role
 // in src/memory_management.jl:78-140).
-constexpr double TILE_RATE[NCFG] = {0.90, 0.65, 0.0, 1.0, 1.0, 0.97};
+// (3xBF16: 170, 155, 156 and 143 TF/s on 1024^3 with the 128x128, 128x64, 64x128 and 64x64
+// tile, 127, 118, 119 and 109 with k = 256.)
+constexpr double TILE_RATE[2][NCFG] = {{0.90, 0.65, 0.0, 1.0, 1.0, 0.97}, {0.87, 0.0, 0.0, 1.0, 0.92, 0.94}};
+int tile_by_rate(int kind, int64_t m, int64_t n) {
+  int cfg = CFG_LARGE;
+  double best = 0;
+  for (int c : {CFG_LARGE, CFG_TALL, CFG_WIDE, 0, 1}) {
+    if (kind == 2 && c == 1) continue;  // (the 64x64 tile's kernel)
+    const double padded = (double)((m + CFG_BM[c] - 1) / CFG_BM[c] * CFG_BM[c]) *
+                          (double)((n + CFG_BN[c] - 1) / CFG_BN[c] * CFG_BN[c]);
+    const double t = padded / TILE_RATE[kind / 2][c];
+    if (c == CFG_LARGE || t < best) {
+      best = t;
+      cfg = c;
+    }
+  }
+  return cfg;
+}
 void default_choice(int kind, int64_t m, int64_t n, int64_t k, int& cfg, int& splitk) {
   splitk = 1;
   if (m <= SMALL_MAX && n <= SMALL_MAX && k <= SMALL_MAX) {
@@ -722,20 +256,8 @@ void default_choice(int kind, int64_t m, int64_t n, int64_t k, int& cfg, int& sp
     cfg = std::max(m, n) >= 96 ? 0 : 1;
     return;
   }
-  if (kind == 2) {
-    cfg = CFG_WIDE;
-    return;
-  }
-  double best = 0;
-  for (int c : {CFG_LARGE, CFG_TALL, CFG_WIDE, 0, 1}) {
-    const double padded = (double)((m + CFG_BM[c] - 1) / CFG_BM[c] * CFG_BM[c]) *
-                          (double)((n + CFG_BN[c] - 1) / CFG_BN[c] * CFG_BN[c]);
-    const double t = padded / TILE_RATE[c];
-    if (c == CFG_LARGE || t < best) {
-      best = t;
-      cfg = c;
-    }
-  }
+  if (kind == 2) cfg = CFG_WIDE;
+  else cfg = tile_by_rate(kind, m, n);
 }
 
 // A choice taken from a bucket (table, tuner trial, forced) may name the small
@@ -768,12 +290,10 @@ bool choose(int method, int64_t m, int64_t n, int64_t k, int& cfg, int& splitk) 
 // ---------------------------------------------------------------------------
 // plans
 // ---------------------------------------------------------------------------
-// Persistent launches of a plan, by kernel.  Native methods: for each ring tile
-// (ring_of) and transpose combination one with 16-byte and one with 4-byte
-// operand loads, then one per combination for leading dimensions past 32-bit
-// offsets.  3xBF16: one per 128-row/column tile shape and combination (L < 12).
-// Last, one for the other items.
-constexpr int L_WIDE = 3 * 4 * 2, L_OTHER = L_WIDE + 4, NLAUNCH = L_OTHER + 1;
+// Persistent launches of a plan, by kernel: for each tile (ring_of; 3xBF16: grouped_x3)
+// one per transpose combination, then one per combination for leading dimensions past
+// 32-bit offsets, then one for the small items.
+constexpr int L_WIDE = 4 * 4, L_OTHER = L_WIDE + 4, NLAUNCH = L_OTHER + 1;
 
 // forced choice for the autotuner's trial launches: cfg >= 0 forces one choice
 // on every problem; otherwise `over` (bucket -> choice) is consulted before the table
@@ -840,45 +360,33 @@ size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // The kernel of launch L (see NLAUNCH) of a plan of method kind `kind`.
 GroupedKernel launch_kernel(int kind, int L) {
-  static const GroupedKernelFn x3[12] = {
-      grouped_large_x3_kernel<128, 128, false, false>, grouped_large_x3_kernel<128, 128, false, true>,
-      grouped_large_x3_kernel<128, 128, true, false>,  grouped_large_x3_kernel<128, 128, true, true>,
-      grouped_large_x3_kernel<128, 64, false, false>,  grouped_large_x3_kernel<128, 64, false, true>,
-      grouped_large_x3_kernel<128, 64, true, false>,   grouped_large_x3_kernel<128, 64, true, true>,
-      grouped_large_x3_kernel<64, 128, false, false>,  grouped_large_x3_kernel<64, 128, false, true>,
-      grouped_large_x3_kernel<64, 128, true, false>,   grouped_large_x3_kernel<64, 128, true, true>};
-  if (L == L_OTHER) return {kind == 0 ? grouped_kernel<0> : kind == 1 ? grouped_kernel<1> : grouped_kernel<2>, GNT};
-  if (kind == 2) return {x3[L], L < 4 ? X3Waves<128, 128>::NTH : GNT};
+  if (L == L_OTHER) return {kind == 0 ? grouped_kernel<0> : grouped_kernel<1>, GNT};
+  if (kind == 2) return L >= L_WIDE ? GroupedKernel{grouped_x3_wide_ld(L - L_WIDE), GNT} : grouped_x3(L / 4, L % 4);
   if (L >= L_WIDE) return {kind == 0 ? grouped_ring_f64_wide_ld(L - L_WIDE) : grouped_ring_f32_wide_ld(L - L_WIDE), GNT};
-  const int which = L / 8, combo = L / 2 % 4;
-  const bool vec = L % 2 == 0;
-  if (kind == 1) return {grouped_ring_f32(which, combo, vec), GNT};
-  return {vec ? grouped_ring_f64_vec(which, combo) : grouped_ring_f64(which, combo), GNT};
+  return {kind == 1 ? grouped_ring_f32(L / 4, L % 4) : grouped_ring_f64(L / 4, L % 4), GNT};
 }
 
 // Byte offsets inside an operand stage (up to 128 rows or 32 k of ld elements) past 32 bits.
 bool wide_ld(int kind, const GProb& g) {
   const int64_t lim = ((int64_t)1 << 32) / (128 * (kind == 0 ? 8 : 4));
-  return (kind != 2 || large_cfg(g.cfg)) && std::max(g.lda, g.ldb) >= lim;
+  return std::max(g.lda, g.ldb) >= lim;
 }
 
 // The ring tile (k_grouped_ring.h) of a native problem, and the extent of the work
-// items its tiles run in: FP64 64x64 and 32x32 tiles share 128x64 items.
+// items its tiles run in: FP64 64x64 and 32x32 tiles share 128x64 items, 3xBF16 ones 64x64.
 int ring_of(int kind, int cfg) { return kind == 1 ? (cfg == 1 ? 2 : 0) : (cfg == CFG_WIDE ? 1 : 0); }
-int item_rows(int kind, const GProb& g) { return kind == 0 && !wide_ld(kind, g) && g.cfg < 2 ? 128 : CFG_BM[g.cfg]; }
-int item_cols(int kind, const GProb& g) { return kind == 0 && !wide_ld(kind, g) && g.cfg < 2 ? 64 : CFG_BN[g.cfg]; }
+int item_rows(int kind, const GProb& g) {
+  return kind == 0 && !wide_ld(kind, g) && g.cfg < 2 ? 128 : kind == 2 && g.cfg < 2 ? 64 : CFG_BM[g.cfg];
+}
+int item_cols(int kind, const GProb& g) { return kind != 1 && !wide_ld(kind, g) && g.cfg < 2 ? 64 : CFG_BN[g.cfg]; }
 
 // The launch of problem g's items.
 int launch_of(int kind, const GProb& g) {
   const int combo = 2 * g.ta + g.tb;
-  if (g.cfg == CFG_SMALL || (kind == 2 && !large_cfg(g.cfg))) return L_OTHER;
-  if (kind == 2) return 4 * (g.cfg - CFG_LARGE) + combo;
+  if (g.cfg == CFG_SMALL) return L_OTHER;
   if (wide_ld(kind, g)) return L_WIDE + combo;
-  const int vw = kind == 0 ? 2 : 4;
-  const bool vec = ((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.B)) & 15) == 0 &&
-                   g.lda % vw == 0 && g.ldb % vw == 0 && (g.ta ? g.k : g.m) % vw == 0 &&
-                   (g.tb ? g.n : g.k) % vw == 0;
-  return 8 * ring_of(kind, g.cfg) + 2 * combo + (vec ? 0 : 1);
+  if (kind == 2) return 4 * (g.cfg < 2 ? 3 : g.cfg - CFG_LARGE) + combo;
+  return 4 * ring_of(kind, g.cfg) + combo;
 }
 
 // Relative duration of one work item of problem g (MFMA work of one k-split of
@@ -916,13 +424,23 @@ hipError_t grouped_occupancy(int kind, int L, int* occ) {
 // the MFMA tiles' residency: shorter chains also round less, and these depths are
 // the ones the methods' accuracy was measured with.
 constexpr int FILL[3][2] = {{4, 2}, {8, 8}, {3, 2}};
+// 3xBF16: 64x128 tiles per compute unit from which on each problem takes the tile with the
+// least padding.  That is up to four kernels, whose longest items start one kernel after
+// the other: 1024 products (17000 tiles) 1378 us with 64x128 tiles, 1253 so; 350 products
+// (8524) 525 and 512; 119 (2940) 194 and 218; 53 (1492) 126 and 163.
+constexpr int X3_MANY = 32;
+// An item longer than this many times a workgroup's share of the group (two per compute
+// unit) is split further: it alone would bound the group.  78 FP64 products 431 us without,
+// 348 at 1.0 (at 2.0 they are not split); 16 and 31 products in 3xBF16 111 and 99 us
+// without, 95.5 and 91 at 2.0, 99 and 101 at 1.0 (26 products 135 at both ends, 143).
+constexpr double LONGEST[3] = {1.0, 1.0, 2.0};
 
 // Tile and split of every problem with m, n > 0 (in order), the plan's first
 // two passes: the table / tuner / static choice per problem, then the device
 // fill: while the group has fewer tiles than FILL workgroups per compute unit (the
 // 128-row/column tiles and the others counted apart), the split of its statically
-// chosen problem with the longest tiles doubles, down to 256 k per split.  Last,
-// each split's k range is fixed.  flops: sum of 2 m n k.
+// chosen problem with the longest tiles doubles, down to 256 k per split; then items
+// that would bound the group are split (LONGEST).  Last, each split's k range is fixed.  flops: sum of 2 m n k.
 int plan_choices(int method, int64_t count, const jb_gemm_desc* d, const Forced& forced, std::vector<GProb>& probs,
                  double* flops) {
   const int kind = kind_of(method);
@@ -973,6 +491,12 @@ int plan_choices(int method, int64_t count, const jb_gemm_desc* d, const Forced&
   auto tiles = [](const GProb& g) {
     return (g.m + CFG_BM[g.cfg] - 1) / CFG_BM[g.cfg] * ((g.n + CFG_BN[g.cfg] - 1) / CFG_BN[g.cfg]);
   };
+  if (kind == 2) {
+    int64_t all = 0;
+    for (auto& g : probs) all += tiles(g) * std::max(g.splitk, 1);
+    for (size_t i = 0; i < probs.size(); ++i)
+      if (dflt[i] && all >= X3_MANY * cus && !wide_ld(kind, probs[i])) probs[i].cfg = tile_by_rate(kind, probs[i].m, probs[i].n);
+  }
   int64_t items[2] = {0, 0};
   for (auto& g : probs) items[large_cfg(g.cfg)] += tiles(g) * std::max(g.splitk, 1);
   for (;;) {
@@ -992,6 +516,15 @@ int plan_choices(int method, int64_t count, const jb_gemm_desc* d, const Forced&
     GProb& g = probs[best];
     items[large_cfg(g.cfg)] += tiles(g) * g.splitk;
     g.splitk *= 2;
+  }
+  // items that would bound the group
+  auto cost = [](const GProb& g) { return (double)CFG_BM[g.cfg] * CFG_BN[g.cfg] * ((double)g.k / g.splitk + 128.0); };
+  double total = 0;
+  for (auto& g : probs) total += (double)tiles(g) * g.splitk * cost(g);
+  for (size_t i = 0; i < probs.size(); ++i) {
+    GProb& g = probs[i];
+    while (dflt[i] && g.splitk < 64 && g.k / (2 * g.splitk) >= 256 && cost(g) > LONGEST[kind] * total / (2.0 * cus))
+      g.splitk *= 2;
   }
   // k per split: a multiple of 32, and no split comes out empty
   for (auto& g : probs) {

@@ -99,6 +99,13 @@ void timing_end(hipStream_t s, const char* kernel);
 template <typename T> using gptr = __attribute__((address_space(1))) T*;
 template <typename T> __device__ __forceinline__ gptr<T> as_global(T* p) { return (gptr<T>)p; }
 
+// Record count of a buffer descriptor from base up to end > base, at most 2^32 - 1 (two
+// halves, so that it stays in scalar registers: a 64-bit minimum is a vector compare).
+template <typename T> __device__ __forceinline__ uint32_t buffer_records(gptr<const T> base, gptr<const T> end) {
+  const uint64_t bytes = (uint64_t)(end - base) * sizeof(T);
+  return (uint32_t)(bytes >> 32) ? 0xffffffffu : (uint32_t)bytes;
+}
+
 // Split-K partial results pass between workgroups on different XCDs, whose L2s are not
 // coherent.  Device-scope stores and loads of the elements themselves (write-through,
 // read past the L2), the stores drained before the tile's arrival counter is raised,

@@ -34,7 +34,7 @@ typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 //     offset, no arithmetic), the stages are unrolled over the ring (constant LDS
 //     offsets), and the next fragments are read behind the first MFMA row of a group.
 //     FP64, register-staged form -> this: 1024^3 TN 44.2 -> 35.2 us, 4096^3 64 -> 74
-//     TF/s, 2999x1777x2111 on odd leading dimensions 462 -> 382 us; FP32 8192^3 130
+//     TF/s, 2999x1777x2111 on odd leading dimensions 462 -> 359 us; FP32 8192^3 130
 //     -> 152 of 157 TF/s.
 //
 //     LDS images (no padding: the loads write 64 consecutive pieces):
@@ -44,13 +44,18 @@ typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 //     The XORs spread the 16 rows and 4 k of one fragment read over all 64
 //     banks; the loads apply them to the global address of each lane.
 //
-//     VEC: 16 bytes per lane (16-byte aligned bases, leading dimensions and the
-//     contiguous extent multiples of the vector); otherwise 4 bytes per lane,
-//     which serves any size and leading dimension through the same LDS image.
-//     Rows past the operand read its last row again (those results are not
-//     stored).  A last stage shorter than BK reads clamped k, and the
-//     fragments replace it: -0.0 from A and +0.0 from B, whose product -0 leaves
-//     every chain value unchanged.
+//     16 bytes per lane, whatever the sizes and leading dimensions: a buffer load needs
+//     4-byte alignment only.  A vector that starts inside the contiguous extent may end
+//     past it: in the next column's elements, or, at the end of the operand, past the
+//     descriptor's record count, where the load returns zeros (checked per 4 bytes).
+//     What it brings there is not used: rows past the operand feed results that are
+//     not stored (vectors wholly past it read its last one again), and a last stage
+//     shorter than BK, whose later vectors read clamped k, has its fragments past the
+//     last k replaced: -0.0 from A and +0.0 from B, whose product -0 leaves every chain
+//     value unchanged.  (Odd sizes took 4-byte loads before:
+//     2999x1777x2111 FP64 on odd leading dimensions 382 us, 359 so; 209 uneven FP32
+//     products of odd sizes in one plan 430 and 410.)
+//     WIDE: 4 bytes per lane and 64-bit addresses, every element clamped on its own.
 // ---------------------------------------------------------------------------
 template <typename T> struct Mfma;
 template <> struct Mfma<double> {
@@ -73,23 +78,22 @@ template <> struct Mfma<float> {
 constexpr int SCHED_ALU = 6;
 #define JB_LDS __attribute__((address_space(3)))
 
-// One wave's load of 64 x LB bytes into LDS at dst, lane l's from base + so + vo (base and so wave-uniform).
-template <int LB>
-__device__ __forceinline__ void ring_load(gptr<const void> base, uint32_t vo, uint32_t so, char* dst) {
+// One wave's load of 64 x 16 bytes into LDS at dst, lane l's from base + so + vo (base and so wave-uniform);
+// zeros from `records` bytes after base on.
+__device__ __forceinline__ void ring_load(gptr<const void> base, uint32_t records, uint32_t vo, uint32_t so, char* dst) {
 #ifdef __HIP_DEVICE_COMPILE__  // the descriptor type exists on the device only
-  __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(const void*)base, 0, 0xffffffffu, 0x00027000);
-  if constexpr (LB == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (JB_LDS void*)dst, 16, vo, so, 0, 0);
-  else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (JB_LDS void*)dst, 4, vo, so, 0, 0);
+  __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(const void*)base, 0, records, 0x00027000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (JB_LDS void*)dst, 16, vo, so, 0, 0);
 #endif
 }
 
 // One operand (R rows of op(A) or columns of op(B)) of the kernel below.
 //   RC: element (r, k) at P[r + k*ld], else at P[k + r*ld].
 //   WIDE: a lane's byte offset inside a stage may exceed 32 bits.
-template <typename T, int R, int BK, bool RC, bool VEC, int NW, bool WIDE>
+template <typename T, int R, int BK, bool RC, int NW, bool WIDE>
 struct RingOperand {
   static constexpr int EB = sizeof(T);
-  static constexpr int LB = VEC ? 16 : 4;                  // bytes per lane of one load
+  static constexpr int LB = WIDE ? 4 : 16;                 // bytes per lane of one load
   static constexpr int PB = 64 * LB;                       // bytes per load (one wave)
   static constexpr int BYTES = R * BK * EB;                // one stage
   static constexpr int NP = BYTES / PB / NW;               // loads per wave and stage
@@ -138,9 +142,10 @@ struct RingOperand {
   }
   // Load i of this wave's share of the stage at k0 into LDS at `dst` (the operand's part of a slot).  P: the operand
   // at the tile's first row.  TAIL: the last stage, shorter than BK, k clamped to kmax (last vector start).
-  template <bool TAIL>
-  __device__ __forceinline__ void issue(gptr<const T> P, int64_t ld, int64_t k0, int64_t kmax, int wave, int lane,
-                                        char* dst, int i) const {
+  // INNER: not the last stage, whose vectors may end past the operand's last element (before `end`).
+  template <bool TAIL, bool INNER>
+  __device__ __forceinline__ void issue(gptr<const T> P, gptr<const T> end, int64_t ld, int64_t k0, int64_t kmax, int wave,
+                                        int lane, char* dst, int i) const {
     const int p = wave + NW * i;
     const int kleft = TAIL ? (int)(kmax - k0) : BK;
     const int kp = RC ? (TAIL ? min(p * KPL / LPK, kleft) : p * KPL / LPK) : 0;  // uniform: first k-row of the load
@@ -155,14 +160,16 @@ struct RingOperand {
         o -= (Off)max(k - kleft, 0) * EB;
       }
     }
-    if constexpr (WIDE) put((gptr<const char>)(P + (RC ? (k0 + kp) * ld : k0)) + o, dst + p * PB);
-    // A buffer load adds the stage's base (descriptor), the load's offset (scalar)
-    // and the lane's by itself: no vector address arithmetic is left in the loop.
-    else ring_load<LB>(P + (RC ? k0 * ld : k0), o, (uint32_t)kp * (uint32_t)ld * EB, dst + p * PB);
-  }
-  static __device__ __forceinline__ void put(gptr<const char> src, char* dst) {
-    if constexpr (VEC) __builtin_amdgcn_global_load_lds((gptr<const void>)src, (JB_LDS void*)dst, 16, 0, 0);
-    else __builtin_amdgcn_global_load_lds((gptr<const void>)src, (JB_LDS void*)dst, 4, 0, 0);
+    if constexpr (WIDE) {
+      gptr<const char> src = (gptr<const char>)(P + (RC ? (k0 + kp) * ld : k0)) + o;
+      __builtin_amdgcn_global_load_lds((gptr<const void>)src, (JB_LDS void*)(dst + p * PB), 4, 0, 0);
+    } else {
+      // A buffer load adds the stage's base (descriptor), the load's offset (scalar)
+      // and the lane's by itself: no vector address arithmetic is left in the loop.
+      gptr<const T> base = P + (RC ? k0 * ld : k0);
+      const uint32_t records = INNER ? 0xffffffffu : buffer_records(base, end);
+      ring_load(base, records, o, (uint32_t)kp * (uint32_t)ld * EB, dst + p * PB);
+    }
   }
 };
 
@@ -173,19 +180,19 @@ __device__ __forceinline__ void wait_ring() {
   __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
 }
 
-template <typename T, bool TA, bool TB, bool VEC, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int NSLOT_>
+template <typename T, bool TA, bool TB, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int NSLOT_>
 struct RingTile {
   static constexpr int NW = WGM * WGN;  // waves
   static constexpr int NTH = 64 * NW;
-  typedef RingOperand<T, BTM, BK, !TA, VEC, NW, WIDE> OA;
-  typedef RingOperand<T, BTN, BK, TB, VEC, NW, WIDE> OB;
+  typedef RingOperand<T, BTM, BK, !TA, NW, WIDE> OA;
+  typedef RingOperand<T, BTN, BK, TB, NW, WIDE> OB;
   static constexpr int WIM = BTM / WGM / 16, WIN = BTN / WGN / 16;  // 16 x 16 MFMA blocks per wave along m, n
   static constexpr int STAGE_B = OA::BYTES + OB::BYTES;
   static constexpr int NLD = OA::NP + OB::NP;  // loads per wave and stage
   // the loads a wait leaves in flight fit its counter
   static constexpr int NSLOT = (NSLOT_ - 2) * NLD < 64 ? NSLOT_ : 63 / NLD + 2;
   static constexpr int SMEM = NSLOT * STAGE_B;
-  static constexpr int VW = VEC ? 16 / (int)sizeof(T) : 1;
+  static constexpr int VW = WIDE ? 1 : 16 / (int)sizeof(T);
   static constexpr int NT4 = BK / 4;  // MFMA k-groups per stage
   static_assert(NT4 % 2 == 0, "the fragment buffers alternate over whole stages");
   typedef typename Mfma<T>::acc_t acc_t;
@@ -193,7 +200,7 @@ struct RingTile {
 
   char* ring;
   int lane, wave, wm, wn, g, l16;
-  gptr<const T> At, Bt;
+  gptr<const T> At, Bt, aend, bend;
   int64_t lda, ldb, K, kamax, kbmax;
   int ramax, rbmax, nst, nfull;
   OA oa;
@@ -213,13 +220,13 @@ struct RingTile {
   __device__ __forceinline__ int row(int i) const { return 16 * (i * WGM + wm) + l16; }
   __device__ __forceinline__ int col(int j, int r) const { return 16 * (j * WGN + wn) + Mfma<T>::prow(r, g); }
 
-  // load i of stage st; tail: the last stage, shorter than BK
-  template <typename Tail>
-  __device__ __forceinline__ void issue(int st, int slot, int i, Tail) const {
+  // load i of stage st; tail: the last stage, shorter than BK; inner: not the last stage
+  template <typename Tail, typename Inner = std::false_type>
+  __device__ __forceinline__ void issue(int st, int slot, int i, Tail, Inner = Inner()) const {
     char* dst = ring + slot * STAGE_B;
     const int64_t k0 = (int64_t)st * BK;
-    if (i < OA::NP) oa.template issue<Tail::value>(At, lda, k0, kamax, wave, lane, dst, i);
-    else ob.template issue<Tail::value>(Bt, ldb, k0, kbmax, wave, lane, dst + OA::BYTES, i - OA::NP);
+    if (i < OA::NP) oa.template issue<Tail::value, Inner::value>(At, aend, lda, k0, kamax, wave, lane, dst, i);
+    else ob.template issue<Tail::value, Inner::value>(Bt, bend, ldb, k0, kbmax, wave, lane, dst + OA::BYTES, i - OA::NP);
   }
 
   // Takes a product: A_, B_ at the tile's first row and column and its first k; rows, cols: what is left of C
@@ -232,10 +239,13 @@ struct RingTile {
     lda = lda_;
     ldb = ldb_;
     K = K_;
-    ramax = (int)min<int64_t>(rows - (TA ? 1 : VW), BTM);
-    rbmax = (int)min<int64_t>(cols - (TB ? VW : 1), BTN);
-    kamax = K - (TA ? VW : 1);
-    kbmax = K - (TB ? 1 : VW);
+    // the last vector starts, and the ends of the operands' last elements
+    ramax = (int)min<int64_t>(TA ? rows - 1 : (rows - 1) / VW * VW, BTM);
+    rbmax = (int)min<int64_t>(TB ? (cols - 1) / VW * VW : cols - 1, BTN);
+    kamax = TA ? (K - 1) / VW * VW : K - 1;
+    kbmax = TB ? K - 1 : (K - 1) / VW * VW;
+    aend = At + (TA ? (rows - 1) * lda + K : (K - 1) * lda + rows);
+    bend = Bt + (TB ? (K - 1) * ldb + cols : (cols - 1) * ldb + K);
     nst = (int)((K + BK - 1) / BK);
     nfull = (int)(K / BK);
     oa.init(lda, ramax, wave, lane);
@@ -278,7 +288,7 @@ struct RingTile {
   // MFMA group the block meets once: stage st + 1 has landed and every wave has
   // read all of stage st, so its slot takes stage st + NSLOT and the next stage's
   // first fragments are read while that group's MFMAs run.
-  // Tail: the short last stage.  Steady: stage st + NSLOT is a whole stage.
+  // Tail: the short last stage.  Steady: stage st + NSLOT is a whole stage and not the last.
   template <int WI, int WJ, typename Tail, typename Steady>
   __device__ __forceinline__ void stage(Acc& acc, int st, int slot, int nslot, Tail, Steady steady) {
     constexpr bool TAIL = Tail::value, STEADY = Steady::value;
@@ -309,7 +319,7 @@ struct RingTile {
           constexpr int PI = (NLD + WI - 1) / WI;
 #pragma unroll
           for (int q = PI * i; q < PI * (i + 1) && q < NLD; ++q) {
-            if (STEADY) issue(st + NSLOT, slot, q, std::false_type());
+            if (STEADY) issue(st + NSLOT, slot, q, std::false_type(), std::true_type());
             else if (!TAIL && st + NSLOT < nfull) issue(st + NSLOT, slot, q, std::false_type());
             else if (!TAIL && st + NSLOT < nst) issue(st + NSLOT, slot, q, std::true_type());
           }
@@ -338,7 +348,7 @@ struct RingTile {
     frags<WI, WJ>(0, 0, a[0], b[0]);
     int st = 0;
     // unrolled over the ring, so that every LDS address is a constant offset from a few lane registers
-    for (; st + 2 * NSLOT - 1 < nfull; st += NSLOT)
+    for (; st + 2 * NSLOT - 1 < min(nfull, nst - 1); st += NSLOT)
 #pragma unroll
       for (int d = 0; d < NSLOT; ++d)
         stage<WI, WJ>(acc, st + d, d, d + 1 == NSLOT ? 0 : d + 1, std::false_type(), std::true_type());

@@ -60,13 +60,13 @@ __device__ __forceinline__ bool splitk_sum(typename Tile::Acc& acc, T* part, int
   return true;
 }
 
-template <typename T, bool TA, bool TB, bool VEC, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int NSLOT,
+template <typename T, bool TA, bool TB, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int NSLOT,
           int MINW>
 __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
     int64_t M, int64_t N, int64_t K, T alpha, const T* __restrict__ A, int64_t lda, const T* __restrict__ B, int64_t ldb,
     T beta, T* __restrict__ C, int64_t ldc, int tiles_m, int tiles_n, int acc_from_c, int64_t kchunk, T* __restrict__ part,
     int* __restrict__ counters) {
-  typedef RingTile<T, TA, TB, VEC, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT> Tile;
+  typedef RingTile<T, TA, TB, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT> Tile;
   constexpr int WIM = Tile::WIM, WIN = Tile::WIN;
   __shared__ __attribute__((aligned(1024))) char ring[Tile::SMEM];
 
@@ -228,7 +228,6 @@ __global__ void scale_kernel(int64_t m, int64_t n, T beta, T* __restrict__ C, in
   }
 }
 
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace
 
@@ -238,10 +237,6 @@ template <typename T, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int
 static hipError_t launch_gemm_mfma_bt(const GemmArgs& g, hipStream_t s, int acc_from_c) {
   const int tiles_m = (int)((g.m + BTM - 1) / BTM), tiles_n = (int)((g.n + BTN - 1) / BTN);
   const int nblocks = tiles_m * tiles_n;
-  // 16-byte loads: aligned bases, and leading dimensions and contiguous extents of whole vectors
-  constexpr int VW = 16 / sizeof(T);
-  const bool vec = !WIDE && aligned16(g.A) && aligned16(g.B) && g.lda % VW == 0 && g.ldb % VW == 0 &&
-                   (g.ta ? g.k : g.m) % VW == 0 && (g.tb ? g.n : g.k) % VW == 0;
   auto A = static_cast<const T*>(g.A);
   auto B = static_cast<const T*>(g.B);
   auto C = static_cast<T*>(g.C);
@@ -249,21 +244,15 @@ static hipError_t launch_gemm_mfma_bt(const GemmArgs& g, hipStream_t s, int acc_
   const int splits = gemm_splits(g);
   const int64_t kchunk = splits > 1 ? g.kchunk : g.k;
   const char* tname = sizeof(T) == 8 ? "dgemm_mfma" : "sgemm_mfma";
-#define JB_LAUNCH_V(TA, TB, V)                                                                                          \
-  hipLaunchKernelGGL((gemm_mfma_kernel<T, TA, TB, V, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT, MINW>), dim3(nblocks, splits), \
-                     dim3(64 * WGM * WGN), 0, s, g.m, g.n, g.k, alpha, A, g.lda, B, g.ldb, beta, C, g.ldc, tiles_m,     \
+#define JB_LAUNCH(TA, TB)                                                                                             \
+  hipLaunchKernelGGL((gemm_mfma_kernel<T, TA, TB, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT, MINW>), dim3(nblocks, splits), \
+                     dim3(64 * WGM * WGN), 0, s, g.m, g.n, g.k, alpha, A, g.lda, B, g.ldb, beta, C, g.ldc, tiles_m,   \
                      tiles_n, acc_from_c, kchunk, static_cast<T*>(g.part), g.counters)
-#define JB_LAUNCH(TA, TB)                      \
-  do {                                         \
-    if (vec) JB_LAUNCH_V(TA, TB, !WIDE);     \
-    else JB_LAUNCH_V(TA, TB, false);         \
-  } while (0)
   timing_begin(s, tname);
   if (!g.ta && !g.tb) JB_LAUNCH(false, false);
   else if (!g.ta && g.tb) JB_LAUNCH(false, true);
   else if (g.ta && !g.tb) JB_LAUNCH(true, false);
   else JB_LAUNCH(true, true);
-#undef JB_LAUNCH_V
 #undef JB_LAUNCH
   timing_end(s, tname);
   return hipGetLastError();

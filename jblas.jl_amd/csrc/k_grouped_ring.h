@@ -24,9 +24,8 @@ __device__ __forceinline__ void ring_part(const GProb& P, const GItem& w, int64_
   for (int i = 0; i < WIM; ++i)
 #pragma unroll
     for (int j = 0; j < WIN; ++j) acc[i][j] = typename Tile::acc_t{T(-0.0), T(-0.0), T(-0.0), T(-0.0)};
-  // padding is skipped down to 32 x 32 blocks of the tile (with 4-byte loads to its halves: fewer loops to compile)
-  constexpr int SI = Tile::VW > 1 ? 1 : (WIM + 1) / 2, SJ = Tile::VW > 1 ? 1 : (WIN + 1) / 2;
-  tile.template run_fringe<SI, SJ>(acc, P.m - ms, P.n - ns);
+  // padding is skipped down to 32 x 32 blocks of the tile
+  tile.template run_fringe<1, 1>(acc, P.m - ms, P.n - ns);
   if (P.splitk == 1) {
     T* C = static_cast<T*>(P.C) + ms + ns * P.ldc;
     if (P.k == 0) {  // no products (k == 0 or alpha == 0): C = beta*C, +0 for beta == 0
@@ -93,23 +92,23 @@ __global__ __launch_bounds__(Tile::NTH, MINW) void grouped_ring_kernel(const GPr
 }
 
 enum { RING_TALL = 0, RING_WIDE = 1, RING_SMALL = 2 };
-template <typename T, bool TA, bool TB, bool VEC>
+template <typename T, bool TA, bool TB>
 GroupedKernelFn ring_kernel_of(int which) {
   if constexpr (sizeof(T) == 8) {
-    if (which == RING_TALL) return grouped_ring_kernel<RingTile<T, TA, TB, VEC, false, 128, 64, 2, 2, 16, 2>, T, TA, TB, 128, 64, 3>;
-    return grouped_ring_kernel<RingTile<T, TA, TB, VEC, false, 64, 128, 2, 2, 16, 2>, T, TA, TB, 64, 128, 3>;
+    if (which == RING_TALL) return grouped_ring_kernel<RingTile<T, TA, TB, false, 128, 64, 2, 2, 16, 2>, T, TA, TB, 128, 64, 3>;
+    return grouped_ring_kernel<RingTile<T, TA, TB, false, 64, 128, 2, 2, 16, 2>, T, TA, TB, 64, 128, 3>;
   } else {
-    if (which != RING_SMALL) return grouped_ring_kernel<RingTile<T, TA, TB, VEC, false, 64, 64, 2, 2, 32, 2>, T, TA, TB, 64, 64, 4>;
-    return grouped_ring_kernel<RingTile<T, TA, TB, VEC, false, 32, 32, 2, 2, 32, 3>, T, TA, TB, 32, 32, 4>;
+    if (which != RING_SMALL) return grouped_ring_kernel<RingTile<T, TA, TB, false, 64, 64, 2, 2, 32, 2>, T, TA, TB, 64, 64, 4>;
+    return grouped_ring_kernel<RingTile<T, TA, TB, false, 32, 32, 2, 2, 32, 3>, T, TA, TB, 32, 32, 4>;
   }
 }
-template <typename T, bool VEC>
+template <typename T>
 GroupedKernelFn ring_kernel_of(int which, int combo) {
   switch (combo) {
-    case 0: return ring_kernel_of<T, false, false, VEC>(which);
-    case 1: return ring_kernel_of<T, false, true, VEC>(which);
-    case 2: return ring_kernel_of<T, true, false, VEC>(which);
-    default: return ring_kernel_of<T, true, true, VEC>(which);
+    case 0: return ring_kernel_of<T, false, false>(which);
+    case 1: return ring_kernel_of<T, false, true>(which);
+    case 2: return ring_kernel_of<T, true, false>(which);
+    default: return ring_kernel_of<T, true, true>(which);
   }
 }
 // 64x64 items with 64-bit offsets
@@ -117,10 +116,10 @@ template <typename T>
 GroupedKernelFn ring_wide_ld_kernel(int combo) {
   constexpr int BK = sizeof(T) == 8 ? 16 : 32;
   switch (combo) {
-    case 0: return grouped_ring_kernel<RingTile<T, false, false, false, true, 64, 64, 2, 2, BK, 2>, T, false, false, 64, 64, 2>;
-    case 1: return grouped_ring_kernel<RingTile<T, false, true, false, true, 64, 64, 2, 2, BK, 2>, T, false, true, 64, 64, 2>;
-    case 2: return grouped_ring_kernel<RingTile<T, true, false, false, true, 64, 64, 2, 2, BK, 2>, T, true, false, 64, 64, 2>;
-    default: return grouped_ring_kernel<RingTile<T, true, true, false, true, 64, 64, 2, 2, BK, 2>, T, true, true, 64, 64, 2>;
+    case 0: return grouped_ring_kernel<RingTile<T, false, false, true, 64, 64, 2, 2, BK, 2>, T, false, false, 64, 64, 2>;
+    case 1: return grouped_ring_kernel<RingTile<T, false, true, true, 64, 64, 2, 2, BK, 2>, T, false, true, 64, 64, 2>;
+    case 2: return grouped_ring_kernel<RingTile<T, true, false, true, 64, 64, 2, 2, BK, 2>, T, true, false, 64, 64, 2>;
+    default: return grouped_ring_kernel<RingTile<T, true, true, true, 64, 64, 2, 2, BK, 2>, T, true, true, 64, 64, 2>;
   }
 }
 

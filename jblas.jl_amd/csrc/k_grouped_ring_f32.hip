@@ -2,8 +2,6 @@
 #include "k_grouped_ring.h"
 
 namespace jb {
-GroupedKernelFn grouped_ring_f32(int which, int combo, bool vec) {
-  return vec ? ring_kernel_of<float, true>(which, combo) : ring_kernel_of<float, false>(which, combo);
-}
+GroupedKernelFn grouped_ring_f32(int which, int combo) { return ring_kernel_of<float>(which, combo); }
 GroupedKernelFn grouped_ring_f32_wide_ld(int combo) { return ring_wide_ld_kernel<float>(combo); }
 }  // namespace jb
