@@ -490,6 +490,7 @@ struct PairArgs {
   void* C;
   int64_t ldc;
   int tiles_m, tiles_n;
+  int halves;  // last tiles run by two blocks each (half_tiles)
   // split-K (3xBF16): k stages per split, the splits' results and per-tile counters
   int split_stages;
   float* part;
@@ -546,8 +547,8 @@ __global__ __launch_bounds__((64 * (QBM / (32 * WB)) * (BN / 32)), 1) void slice
   constexpr int PD = NSLOT - 1;  // prefetch distance
   __shared__ __attribute__((aligned(1024))) char ring[NSLOT * STAGE_B];
 
-  const int nblocks = p.tiles_m * p.tiles_n;
-  const int tile = xcd_remap(blockIdx.x, nblocks, 8);
+  const int nwhole = p.tiles_m * p.tiles_n - p.halves, cut = (int)blockIdx.x - nwhole;
+  const int tile = cut < 0 ? xcd_remap(blockIdx.x, nwhole, 8) : nwhole + (cut < p.halves ? cut : cut - p.halves);
   int tm, tn;
   tile_coords(tile, p.tiles_m, p.tiles_n, OZ_GROUP, tm, tn);
   const int64_t m0 = (int64_t)tm * QBM, n0 = (int64_t)tn * BN;
@@ -650,6 +651,18 @@ __global__ __launch_bounds__((64 * (QBM / (32 * WB)) * (BN / 32)), 1) void slice
   // overlap).  The kernel waits for those loads before it ends.
 #pragma unroll
   for (int i = 0; i < PD; ++i) issue(min(i, nst - 1), i);
+  // A cut tile's block multiplies with half of its waves, one per SIMD (of two); the others
+  // only load.
+  if (cut >= 0 && (wave >= NWAVES / 2) != (cut >= p.halves)) {
+    for (int st = 0; st < nst; ++st) {
+      if (wave < NWL % NWAVES) wait_vmcnt<(PD - 1) * WL_MAX>();
+      else wait_vmcnt<(PD - 1) * WL_MIN>();
+      block_barrier();
+      issue(min(st + PD, nst - 1), (st + PD) % NSLOT);
+    }
+    wait_vmcnt<0>();
+    return;
+  }
   // chunk-end mask of the non-fast levels after stage st (bit l: level l's exact
   // chunk ends here and it is flushed), the stage loop's runtime form
   auto chunk_mask = [&](const int st) JB_INLINE {
@@ -914,6 +927,15 @@ void launch_split(const GemmArgs& g, const Layout& L, char* ws, int* flag, int* 
                      L.Kpad, flag ? flag : sticky, sticky);
 }
 
+// Tiles of the last round that run as two blocks each: where the tiles after the last
+// whole round over the compute units are at most half of them, so that the halves still
+// fit one round, which then takes about half as long
+// (2500 x 1900 x 3001, seven INT8 slices, 600 tiles: 406 us, 378 so).
+int half_tiles(int64_t tiles) {
+  const int64_t cus = std::max(runtime_compute_units(), 1), rest = tiles % cus;
+  return 2 * rest <= cus ? (int)rest : 0;
+}
+
 // elt as in make_layout: the kernel addresses planes in 16-bit units, so an
 // INT8 plane of Kpad k is a BF16-shaped plane of Kpad/2.
 PairArgs pair_args(const GemmArgs& g, const Layout& L, const uint16_t* pA, const uint16_t* pB, const int* eA,
@@ -934,6 +956,7 @@ PairArgs pair_args(const GemmArgs& g, const Layout& L, const uint16_t* pA, const
   p.ldc = g.ldc;
   p.tiles_m = (int)(L.Mpad / QBM);
   p.tiles_n = (int)(L.Npad / bn);
+  p.halves = gemm_splits(g) > 1 ? 0 : half_tiles((int64_t)p.tiles_m * p.tiles_n);
   p.split_stages = (int)(p.Kpad / QBK);
   p.part = static_cast<float*>(g.part);
   p.counters = g.counters;
@@ -954,7 +977,7 @@ hipError_t run_ozaki(const GemmArgs& g, const Layout& L, char* ws, bool want_fla
   if (e != hipSuccess) return e;
   const PairArgs p = pair_args(g, L, pA, pB, eA, eB);
   timing_begin(st, "slice_pair_gemm");
-  hipLaunchKernelGGL((slice_pair_gemm_kernel<0, S, S + 1, OZ_WB>), dim3(p.tiles_m * p.tiles_n), dim3(512 / OZ_WB), 0, st, p);
+  hipLaunchKernelGGL((slice_pair_gemm_kernel<0, S, S + 1, OZ_WB>), dim3(p.tiles_m * p.tiles_n + p.halves), dim3(512 / OZ_WB), 0, st, p);
   timing_end(st, "slice_pair_gemm");
   return hipGetLastError();
 }
@@ -974,7 +997,7 @@ hipError_t run_ozaki_i8(const GemmArgs& g, const Layout& L, char* ws, bool want_
   const PairArgs p = pair_args(g, L, reinterpret_cast<const uint16_t*>(pA), reinterpret_cast<const uint16_t*>(pB), eA,
                                eB, 1);
   timing_begin(st, "slice_pair_gemm_i8");
-  hipLaunchKernelGGL((slice_pair_gemm_kernel<2, S, S + 1, OZ_WB>), dim3(p.tiles_m * p.tiles_n), dim3(512 / OZ_WB), 0,
+  hipLaunchKernelGGL((slice_pair_gemm_kernel<2, S, S + 1, OZ_WB>), dim3(p.tiles_m * p.tiles_n + p.halves), dim3(512 / OZ_WB), 0,
                      st, p);
   timing_end(st, "slice_pair_gemm_i8");
   return hipGetLastError();
@@ -1046,7 +1069,7 @@ void bf16x3_split_need(const GemmArgs& g, size_t* part_bytes, int64_t* counters)
 
 template <int BN>
 void launch_x3_pairs(const PairArgs& p, int nprod, int splits, hipStream_t st) {
-  const dim3 grid(p.tiles_m * p.tiles_n, splits);
+  const dim3 grid(p.tiles_m * p.tiles_n + p.halves, splits);
   const dim3 block(64 * (QBM / (32 * X3_WB)) * (BN / 32));
   if (nprod == 3) hipLaunchKernelGGL((slice_pair_gemm_kernel<1, 3, 3, X3_WB, BN>), grid, block, 0, st, p);
   else if (nprod == 6) hipLaunchKernelGGL((slice_pair_gemm_kernel<1, 3, 4, X3_WB, BN>), grid, block, 0, st, p);
