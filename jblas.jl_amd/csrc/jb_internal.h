@@ -18,7 +18,7 @@ struct GemmArgs {
   void* C;
   int64_t ldc;
   // Split-K (adjoints of small products): k per split, a multiple of 32 (0: one
-  // chain over all of k), device memory for the splits' results and zeroed per-tile
+  // chain over all of k), device memory for the splits' results (else null) and zeroed per-tile
   // counters (gemm_mfma_split_need / bf16x3_split_need), which the call leaves zeroed.
   int64_t kchunk = 0;
   void* part = nullptr;

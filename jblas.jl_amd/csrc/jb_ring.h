@@ -142,9 +142,9 @@ struct RingOperand {
   }
   // Load i of this wave's share of the stage at k0 into LDS at `dst` (the operand's part of a slot).  P: the operand
   // at the tile's first row.  TAIL: the last stage, shorter than BK, k clamped to kmax (last vector start).
-  // INNER: not the last stage, whose vectors may end past the operand's last element (before `end`).
-  template <bool TAIL, bool INNER>
-  __device__ __forceinline__ void issue(gptr<const T> P, gptr<const T> end, int64_t ld, int64_t k0, int64_t kmax, int wave,
+  // records: bytes from the stage's base up to the operand's end.
+  template <bool TAIL>
+  __device__ __forceinline__ void issue(gptr<const T> P, uint32_t records, int64_t ld, int64_t k0, int64_t kmax, int wave,
                                         int lane, char* dst, int i) const {
     const int p = wave + NW * i;
     const int kleft = TAIL ? (int)(kmax - k0) : BK;
@@ -167,7 +167,6 @@ struct RingOperand {
       // A buffer load adds the stage's base (descriptor), the load's offset (scalar)
       // and the lane's by itself: no vector address arithmetic is left in the loop.
       gptr<const T> base = P + (RC ? k0 * ld : k0);
-      const uint32_t records = INNER ? 0xffffffffu : buffer_records(base, end);
       ring_load(base, records, o, (uint32_t)kp * (uint32_t)ld * EB, dst + p * PB);
     }
   }
@@ -200,7 +199,8 @@ struct RingTile {
 
   char* ring;
   int lane, wave, wm, wn, g, l16;
-  gptr<const T> At, Bt, aend, bend;
+  gptr<const T> At, Bt;
+  uint32_t arec, brec;  // bytes from the last stage's base to the operand's end (earlier stages' vectors end inside it)
   int64_t lda, ldb, K, kamax, kbmax;
   int ramax, rbmax, nst, nfull;
   OA oa;
@@ -220,13 +220,14 @@ struct RingTile {
   __device__ __forceinline__ int row(int i) const { return 16 * (i * WGM + wm) + l16; }
   __device__ __forceinline__ int col(int j, int r) const { return 16 * (j * WGN + wn) + Mfma<T>::prow(r, g); }
 
-  // load i of stage st; tail: the last stage, shorter than BK; inner: not the last stage
-  template <typename Tail, typename Inner = std::false_type>
-  __device__ __forceinline__ void issue(int st, int slot, int i, Tail, Inner = Inner()) const {
+  // load i of stage st; tail: the last stage, shorter than BK
+  template <typename Tail>
+  __device__ __forceinline__ void issue(int st, int slot, int i, Tail) const {
     char* dst = ring + slot * STAGE_B;
     const int64_t k0 = (int64_t)st * BK;
-    if (i < OA::NP) oa.template issue<Tail::value, Inner::value>(At, aend, lda, k0, kamax, wave, lane, dst, i);
-    else ob.template issue<Tail::value, Inner::value>(Bt, bend, ldb, k0, kbmax, wave, lane, dst + OA::BYTES, i - OA::NP);
+    const uint32_t records = st == nst - 1 ? (i < OA::NP ? arec : brec) : 0xffffffffu;
+    if (i < OA::NP) oa.template issue<Tail::value>(At, records, lda, k0, kamax, wave, lane, dst, i);
+    else ob.template issue<Tail::value>(Bt, records, ldb, k0, kbmax, wave, lane, dst + OA::BYTES, i - OA::NP);
   }
 
   // Takes a product: A_, B_ at the tile's first row and column and its first k; rows, cols: what is left of C
@@ -239,15 +240,16 @@ struct RingTile {
     lda = lda_;
     ldb = ldb_;
     K = K_;
-    // the last vector starts, and the ends of the operands' last elements
+    // the last vector starts
     ramax = (int)min<int64_t>(TA ? rows - 1 : (rows - 1) / VW * VW, BTM);
     rbmax = (int)min<int64_t>(TB ? (cols - 1) / VW * VW : cols - 1, BTN);
     kamax = TA ? (K - 1) / VW * VW : K - 1;
     kbmax = TB ? K - 1 : (K - 1) / VW * VW;
-    aend = At + (TA ? (rows - 1) * lda + K : (K - 1) * lda + rows);
-    bend = Bt + (TB ? (K - 1) * ldb + cols : (cols - 1) * ldb + K);
     nst = (int)((K + BK - 1) / BK);
     nfull = (int)(K / BK);
+    const int64_t kr = K - (int64_t)(nst - 1) * BK;  // k of the last stage
+    arec = records(TA ? (rows - 1) * lda + kr : (kr - 1) * lda + rows);
+    brec = records(TB ? (kr - 1) * ldb + cols : (cols - 1) * ldb + kr);
     oa.init(lda, ramax, wave, lane);
     ob.init(ldb, rbmax, wave, lane);
 #pragma unroll
@@ -257,6 +259,12 @@ struct RingTile {
         if (d < nfull) issue(d, d, i, std::false_type());
         else if (d < nst) issue(d, d, i, std::true_type());
       }
+  }
+
+  // (two halves: a 64-bit minimum is a vector compare, and a descriptor of vector registers a loop over the lanes)
+  static __device__ __forceinline__ uint32_t records(int64_t elements) {
+    const uint64_t bytes = (uint64_t)elements * sizeof(T);
+    return (uint32_t)(bytes >> 32) ? 0xffffffffu : (uint32_t)bytes;
   }
 
   template <int WI, int WJ>
@@ -288,7 +296,7 @@ struct RingTile {
   // MFMA group the block meets once: stage st + 1 has landed and every wave has
   // read all of stage st, so its slot takes stage st + NSLOT and the next stage's
   // first fragments are read while that group's MFMAs run.
-  // Tail: the short last stage.  Steady: stage st + NSLOT is a whole stage and not the last.
+  // Tail: the short last stage.  Steady: stage st + NSLOT is a whole stage.
   template <int WI, int WJ, typename Tail, typename Steady>
   __device__ __forceinline__ void stage(Acc& acc, int st, int slot, int nslot, Tail, Steady steady) {
     constexpr bool TAIL = Tail::value, STEADY = Steady::value;
@@ -319,7 +327,7 @@ struct RingTile {
           constexpr int PI = (NLD + WI - 1) / WI;
 #pragma unroll
           for (int q = PI * i; q < PI * (i + 1) && q < NLD; ++q) {
-            if (STEADY) issue(st + NSLOT, slot, q, std::false_type(), std::true_type());
+            if (STEADY) issue(st + NSLOT, slot, q, std::false_type());
             else if (!TAIL && st + NSLOT < nfull) issue(st + NSLOT, slot, q, std::false_type());
             else if (!TAIL && st + NSLOT < nst) issue(st + NSLOT, slot, q, std::true_type());
           }
@@ -348,7 +356,7 @@ struct RingTile {
     frags<WI, WJ>(0, 0, a[0], b[0]);
     int st = 0;
     // unrolled over the ring, so that every LDS address is a constant offset from a few lane registers
-    for (; st + 2 * NSLOT - 1 < min(nfull, nst - 1); st += NSLOT)
+    for (; st + 2 * NSLOT - 1 < nfull; st += NSLOT)
 #pragma unroll
       for (int d = 0; d < NSLOT; ++d)
         stage<WI, WJ>(acc, st + d, d, d + 1 == NSLOT ? 0 : d + 1, std::false_type(), std::true_type());

@@ -878,7 +878,7 @@ extern "C++" int jb::single_gemm_dev_locked(int method, const GemmArgs& g, hipSt
   void* ws = nullptr;
   int rc = ws_acquire(planes + part, s, &ws);
   if (rc) return rc;
-  h.part = static_cast<char*>(ws) + planes;
+  h.part = part ? static_cast<char*>(ws) + planes : nullptr;
   h.counters = rt().counters;
   // (word 1 of the sticky buffer: a flag nobody reads)
   const hipError_t e = x3    ? launch_sgemm_bf16x3(h, 6, ws, false, rt().sticky + (report ? 0 : 1), s)

@@ -106,7 +106,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
   tile.begin(as_global(A) + (TA ? kb + m0 * lda : m0 + kb * lda), lda, as_global(B) + (TB ? n0 + kb * ldb : kb + n0 * ldb),
              ldb, M - m0, N - n0, min(K - kb, kchunk));
   tile.run(acc);
-  if (gridDim.y > 1 && !splitk_sum<T, Tile>(acc, part, counters, id, ring)) return;
+  if (part && !splitk_sum<T, Tile>(acc, part, counters, id, ring)) return;
   tile.store(acc, C + m0 + n0 * ldc, ldc, M - m0, N - n0, alpha, beta);
 }
 

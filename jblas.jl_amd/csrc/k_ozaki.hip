@@ -798,7 +798,7 @@ __global__ __launch_bounds__((64 * (QBM / (32 * WB)) * (BN / 32)), 1) void slice
     for (int b = 0; b < WB; ++b)
 #pragma unroll
       for (int e = 0; e < 16; ++e) res[b][e] = acc[0][b][e] + acc[1][b][e];
-    if (gridDim.y > 1) {
+    if (p.part) {
       // Each block stores its chunk's results, thread by thread, to its slab; the tile's last block to arrive sums
       // the slabs in split order.  The counters are zero between launches: that block clears its own.
       constexpr int NTH = 64 * NWAVES;
