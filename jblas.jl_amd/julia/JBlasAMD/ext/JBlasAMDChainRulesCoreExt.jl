@@ -8,7 +8,7 @@ rrule of `gemm(tA, tB, α, A, B)` = α op(A) op(B):
   Ā = α C̄ op(B)ᵀ (tA = 'N') or α op(B) C̄ᵀ (tA = 'T')
   B̄ = α op(A)ᵀ C̄ (tB = 'N') or α C̄ᵀ op(A) (tB = 'T')
   ᾱ = ⟨C̄, op(A) op(B)⟩
-Ā and B̄ come from one grouped launch of the library's adjoint kernels.
+Ā and B̄ come from the library's pullback.
 """
 function ChainRulesCore.rrule(::typeof(gemm), tA::AbstractChar, tB::AbstractChar, α::Real,
                               A::StridedMatrix{T}, B::StridedMatrix{T}; kw...) where {T<:Union{Float32,Float64}}

@@ -271,7 +271,7 @@ end
     pullback!(tA, tB, α, A, B, dC, dA, dB; method)
 
 dA = α dC op(B)ᵀ (or its transpose for tA = 'T') and dB = α op(A)ᵀ dC (or
-transposed for tB = 'T'), both in one grouped launch (jb_gemm_pullback).
+transposed for tB = 'T'), one after the other (jb_gemm_pullback).
 Either of dA, dB may be `nothing`.
 """
 function pullback!(tA::AbstractChar, tB::AbstractChar, α::Real, A::StridedMatrix{T}, B::StridedMatrix{T},
