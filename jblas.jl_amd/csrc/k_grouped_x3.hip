@@ -88,18 +88,25 @@ struct XRuns {
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] = __builtin_amdgcn_fmed3f(x[e], -BMAX, BMAX);
     }
-    uint32_t w0 = __builtin_bit_cast(uint32_t, bf2{(__bf16)y[0], (__bf16)y[1]});
-    uint32_t w1 = __builtin_bit_cast(uint32_t, bf2{(__bf16)y[2], (__bf16)y[3]});
+    const uint32_t w0 = __builtin_bit_cast(uint32_t, bf2{(__bf16)y[0], (__bf16)y[1]});
+    const uint32_t w1 = __builtin_bit_cast(uint32_t, bf2{(__bf16)y[2], (__bf16)y[3]});
     *reinterpret_cast<uint2*>(S + wo[q] + p * (R * BK * 2)) = uint2{w0, w1};
     if (p < 2) {
-      // the packed BF16 values back in FP32 (low half shifted up, high half masked): one
-      // packed conversion per two elements.  With w0, w1 visible to the compiler it
-      // converted each low element a second time; the empty asm hides their origin.
-      asm("" : "+v"(w0), "+v"(w1));
-      x[0] -= __uint_as_float(w0 << 16);
-      x[1] -= __uint_as_float(w0 & 0xffff0000u);
-      x[2] -= __uint_as_float(w1 << 16);
-      x[3] -= __uint_as_float(w1 & 0xffff0000u);
+      // x minus its rounding as a dot product of the packed pair with (-1, 0) or (0, -1):
+      // one instruction in place of an unpacking shift or mask and a subtraction, with the
+      // same result for every input (checked on the device bit for bit, denormals, signed
+      // zeros, infinities and the largest values included; a NaN spreads to the other k of
+      // its pair, which feeds the same results).  The register constant: as an inline
+      // constant -1.0 stands for (0, -1).
+      uint32_t lo = 0x0000bf80u;
+      asm("" : "+s"(lo));
+      const bf2 first = __builtin_bit_cast(bf2, lo), second = __builtin_bit_cast(bf2, 0xbf800000u);
+#ifdef __HIP_DEVICE_COMPILE__
+      x[0] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, w0), first, x[0], false);
+      x[1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, w0), second, x[1], false);
+      x[2] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, w1), first, x[2], false);
+      x[3] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, w1), second, x[3], false);
+#endif
     }
   }
 };
