@@ -99,11 +99,10 @@ void timing_end(hipStream_t s, const char* kernel);
 template <typename T> using gptr = __attribute__((address_space(1))) T*;
 template <typename T> __device__ __forceinline__ gptr<T> as_global(T* p) { return (gptr<T>)p; }
 
-// Record count of a buffer descriptor from base up to end > base, at most 2^32 - 1 (two
-// halves, so that it stays in scalar registers: a 64-bit minimum is a vector compare).
-template <typename T> __device__ __forceinline__ uint32_t buffer_records(gptr<const T> base, gptr<const T> end) {
-  const uint64_t bytes = (uint64_t)(end - base) * sizeof(T);
-  return (uint32_t)(bytes >> 32) ? 0xffffffffu : (uint32_t)bytes;
+// Record count of a buffer descriptor over `elements` of T, at most 2^32 - 1.
+template <typename T> __device__ __forceinline__ uint32_t buffer_records(int64_t elements) {
+  const uint64_t bytes = (uint64_t)elements * sizeof(T);
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(bytes >> 32) ? 0xffffffffu : (uint32_t)bytes));
 }
 
 // Split-K partial results pass between workgroups on different XCDs, whose L2s are not

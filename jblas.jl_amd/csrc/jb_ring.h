@@ -248,8 +248,8 @@ struct RingTile {
     nst = (int)((K + BK - 1) / BK);
     nfull = (int)(K / BK);
     const int64_t kr = K - (int64_t)(nst - 1) * BK;  // k of the last stage
-    arec = records(TA ? (rows - 1) * lda + kr : (kr - 1) * lda + rows);
-    brec = records(TB ? (kr - 1) * ldb + cols : (cols - 1) * ldb + kr);
+    arec = buffer_records<T>(TA ? (rows - 1) * lda + kr : (kr - 1) * lda + rows);
+    brec = buffer_records<T>(TB ? (kr - 1) * ldb + cols : (cols - 1) * ldb + kr);
     oa.init(lda, ramax, wave, lane);
     ob.init(ldb, rbmax, wave, lane);
 #pragma unroll
@@ -259,12 +259,6 @@ struct RingTile {
         if (d < nfull) issue(d, d, i, std::false_type());
         else if (d < nst) issue(d, d, i, std::true_type());
       }
-  }
-
-  // (two halves: a 64-bit minimum is a vector compare, and a descriptor of vector registers a loop over the lanes)
-  static __device__ __forceinline__ uint32_t records(int64_t elements) {
-    const uint64_t bytes = (uint64_t)elements * sizeof(T);
-    return (uint32_t)(bytes >> 32) ? 0xffffffffu : (uint32_t)bytes;
   }
 
   template <int WI, int WJ>

@@ -45,9 +45,9 @@ struct XRuns {
     }
   }
   // Run q of the stage at `base`, with nk k left (the last stage may have fewer than 32).
-  // `end`: past the operand's last element, where the buffer load reads zeros (checked
-  // per 4 bytes), so a rows-contiguous operand is zero from k = nk on.
-  __device__ __forceinline__ void load(int t, int q, gptr<const float> base, gptr<const float> end, int64_t ld, int nk) {
+  // From `records` bytes on, past the operand's last element, the buffer load reads zeros
+  // (checked per 4 bytes), so a rows-contiguous operand is zero from k = nk on.
+  __device__ __forceinline__ void load(int t, int q, gptr<const float> base, uint32_t records, int64_t ld, int nk) {
     if constexpr (WIDE) {
       const int k = 4 * krun(t, q);
 #pragma unroll
@@ -56,7 +56,7 @@ struct XRuns {
     } else {
 #ifdef __HIP_DEVICE_COMPILE__
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)base, 0, buffer_records(base, end), 0x00027000);
+          (void*)base, 0, records, 0x00027000);
       if constexpr (!RC) {
         v[q] = __builtin_bit_cast(V4, __builtin_amdgcn_raw_buffer_load_b128(rs, vo[q], 0, 0));
       } else {
@@ -122,8 +122,10 @@ struct XRuns {
 // their splits together.  64 products of 1024^3, k-contiguous operands: 128x128 tile 158
 // TF/s so, 173 here (1040 of BF16 products), 64x64 23 (guarded element loads, split
 // after the MFMAs) and 143; 1021 x 1021 x 1023: 146 and 165 (128x128).  1024 uneven
-// products in one plan: 1465 us, 1378 with the 128-row/column tiles so, 1250 to 1320
-// with the 64x64 kernel and the choice of tiles by padding.
+// products in one plan: 1465 us, 1378 with the 128-row/column tiles so, 1326 with the
+// 64x64 kernel and the choice of tiles by padding, 1309 with the residuals by dot
+// products, 1203 with the record counts out of the loop (a 64-bit compare per load of a
+// stage: a vector instruction and a wait for its scalar result).
 template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool WIDE>
 __device__ __forceinline__ void x3_loop(const GProb& P, int64_t m0, int64_t n0, int64_t kb, int64_t ke, char* smem,
                                               f16v (&acc)[2][BM / WM / 32][BN / WN / 32]) {
@@ -144,11 +146,14 @@ __device__ __forceinline__ void x3_loop(const GProb& P, int64_t m0, int64_t n0, 
   ra.begin(tid, lda, P.m - m0);
   rb.begin(tid, ldb, P.n - n0);
   const int K = (int)(ke - kb), nkt = (K + BK - 1) / BK;
-  gptr<const float> Ae = A + (TA ? (P.m - m0 - 1) * lda + K : (K - 1) * lda + P.m - m0);
-  gptr<const float> Be = B + (TB ? (K - 1) * ldb + P.n - n0 : (P.n - n0 - 1) * ldb + K);
+  // bytes from the last stage's base to the operand's end (earlier stages' loads end inside it)
+  const int kl = K - (nkt - 1) * BK;
+  const uint32_t reca = buffer_records<float>(TA ? (P.m - m0 - 1) * lda + kl : (kl - 1) * lda + P.m - m0);
+  const uint32_t recb = buffer_records<float>(TB ? (kl - 1) * ldb + P.n - n0 : (P.n - n0 - 1) * ldb + kl);
   auto load = [&](int kt, int q) JB_INLINE {
-    if (q < RA::NR) ra.load(tid, q, A + kt * sa, Ae, lda, K - kt * BK);
-    else rb.load(tid, q - RA::NR, B + kt * sb, Be, ldb, K - kt * BK);
+    const bool last = kt == nkt - 1;
+    if (q < RA::NR) ra.load(tid, q, A + kt * sa, last ? reca : 0xffffffffu, lda, K - kt * BK);
+    else rb.load(tid, q - RA::NR, B + kt * sb, last ? recb : 0xffffffffu, ldb, K - kt * BK);
   };
   auto mask = [&](int kt, int q) JB_INLINE {
     if (q < RA::NR) ra.mask(tid, q, K - kt * BK);
