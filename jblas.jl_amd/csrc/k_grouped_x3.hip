@@ -259,6 +259,34 @@ __device__ void x3_tile(const GProb& P, int tm, int tn, int split, char* smem, i
         for (int e = 0; e < 16; ++e) acc[l][i][j][e] = 0.0f;
   if (kb < ke) x3_loop<BM, BN, WM, WN, TA, TB, WIDE>(P, m0, n0, kb, ke, smem, acc);
   // item e of lane l in block (i, j): row wm0 + 32 i + l%32, column wn0 + 32 j + 8 (e/4) + 4 (l/32) + e%4
+  if (!WIDE && P.splitk == 1 && kb < ke && (float)P.beta == 0.0f && P.ldc < (1 << 22)) {
+#ifdef __HIP_DEVICE_COMPILE__
+    // One multiply and one buffer store per element: columns in scalar offsets, rows in the
+    // lane's; columns past C lie past the record count, where stores are dropped.  (The
+    // general form below forms and checks an address per element: 1024 uneven products
+    // 1228 us, 1197 so; groups of 20 to 700 products 4.6 to 8.4 % faster.)
+    const int rows = (int)min<int64_t>(P.m - m0, BM), cols = (int)min<int64_t>(P.n - n0, BN);
+    const uint32_t ld = 4 * (uint32_t)P.ldc;
+    gptr<float> C = as_global(static_cast<float*>(P.C)) + m0 + n0 * P.ldc;
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void*)C, 0, buffer_records<float>((cols - 1) * P.ldc + rows), 0x00027000);
+    const float alpha = (float)P.alpha;
+#pragma unroll
+    for (int i = 0; i < IB; ++i) {
+      const int r = wm0 + 32 * i + l32;
+      const uint32_t vo = 4 * (uint32_t)r + (uint32_t)(wn0 + 4 * hl) * ld;
+      if (r < rows) {
+#pragma unroll
+        for (int j = 0; j < JB; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(alpha * (acc[0][i][j][e] + acc[1][i][j][e])), rs, vo,
+                                                  (32 * j + 8 * (e / 4) + e % 4) * ld, 0);
+      }
+    }
+#endif
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < IB; ++i)
 #pragma unroll

@@ -34,7 +34,8 @@ def check(ta, tb, A, B, C0, got, alpha=1.5, beta=0.5):
 
 @pytest.mark.parametrize("cfg", [0, 1, 3, 4, 5])
 @pytest.mark.parametrize("splitk", [1, 2])
-def test_x3_tiles_edges(gpu, cfg, splitk, tmp_path):
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+def test_x3_tiles_edges(gpu, cfg, splitk, beta, tmp_path):
     jb.tune_reset()
     write_table(str(tmp_path / "t.json"), "f32_bf16x3", SHAPES, cfg, splitk)
     try:
@@ -46,11 +47,13 @@ def test_x3_tiles_edges(gpu, cfg, splitk, tmp_path):
                     B = G.matrix(30 + i, *((k, n) if tb == "N" else (n, k)), dtype=np.float32)
                     C = G.matrix(50 + i, m, n, dtype=np.float32)
                     host.append((A, B, C))
-                    descs.append(GemmDesc(ta, tb, 1.5, placed(gpu, A, i % 4, i % 3), placed(gpu, B, i % 2, i % 4), 0.5,
+                    descs.append(GemmDesc(ta, tb, 1.5, placed(gpu, A, i % 4, i % 3), placed(gpu, B, i % 2, i % 4), beta,
                                           placed(gpu, C, 1, 0)))
                 jb.gemm_grouped_("f32_bf16x3", descs)
                 for (A, B, C), d in zip(host, descs):
-                    check(ta, tb, A, B, C, to_host(d.C))
+                    check(ta, tb, A, B, C, to_host(d.C), beta=beta)
+                    buf = d.C._base
+                    assert int(buf.isnan().sum()) == buf.numel() - C.size  # nothing stored around C
     finally:
         jb.tune_reset()
 
