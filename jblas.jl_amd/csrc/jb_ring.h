@@ -48,6 +48,7 @@ typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 //     4-byte alignment only.  A vector that starts inside the contiguous extent may end
 //     past it: in the next column's elements, or, at the end of the operand, past the
 //     descriptor's record count, where the load returns zeros (checked per 4 bytes).
+//     Every stage that can reach the operand's end has that count (RingOperand::REACH).
 //     What it brings there is not used: rows past the operand feed results that are
 //     not stored (vectors wholly past it read its last one again), and a last stage
 //     shorter than BK, whose later vectors read clamped k, has its fragments past the
@@ -90,6 +91,8 @@ __device__ __forceinline__ void ring_load(gptr<const void> base, uint32_t record
 // One operand (R rows of op(A) or columns of op(B)) of the kernel below.
 //   RC: element (r, k) at P[r + k*ld], else at P[k + r*ld].
 //   WIDE: a lane's byte offset inside a stage may exceed 32 bits.
+// The address functions are host functions too: their bounds are checked there.
+#define JB_HD __host__ __device__ __forceinline__
 template <typename T, int R, int BK, bool RC, int NW, bool WIDE>
 struct RingOperand {
   static constexpr int EB = sizeof(T);
@@ -108,15 +111,15 @@ struct RingOperand {
   static_assert(RC || RPL >= 1, "a load covers whole rows");
   // The k-rows 4t..4t+3 of one fragment read must start 128 bytes (T = double,
   // two per pass over the banks) or 64 bytes (T = float) apart.
-  static __device__ __forceinline__ int rswz(int k) {
+  static JB_HD int rswz(int k) {
     if (EB == 8) return 16 * (k & 1);
     return R >= 64 ? 16 * (k & 3) : 16 * ((k >> 1) & 1);
   }
   static_assert(!RC || R >= 32, "the row swizzle stays inside a k-row");
-  static __device__ __forceinline__ int cswz(int r) { return (r / RPB) & (CPR - 1); }
+  static JB_HD int cswz(int r) { return (r / RPB) & (CPR - 1); }
 
   // LDS element of (r, k); r in [0, R), k in [0, BK)
-  static __device__ __forceinline__ int at(int r, int k) {
+  static JB_HD int at(int r, int k) {
     if (RC) return k * R + (r ^ rswz(k));
     return r * BK + (((k * EB / 16) ^ cswz(r)) * 16 + (k * EB) % 16) / EB;
   }
@@ -124,7 +127,7 @@ struct RingOperand {
   typedef typename std::conditional<WIDE, int64_t, uint32_t>::type Off;
   Off off[NP];  // this lane's byte offset in load i of a stage, from the load's wave-uniform address
   // ld: leading dimension; rmax: last row (vector start) that may be read, relative to the tile's first
-  __device__ __forceinline__ void init(int64_t ld, int rmax, int wave, int lane) {
+  JB_HD void init(int64_t ld, int rmax, int wave, int lane) {
     const int lb = lane * LB;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
@@ -140,6 +143,27 @@ struct RingOperand {
       }
     }
   }
+
+  // Whether a vector of the stage before the last can end past the operand: with more than two elements to a vector
+  // and ld below its length, it runs over the few elements of a short last stage (one row of ld 1, K = 33: the vector
+  // at k = 31 covers k = 31..34).  Earlier stages have a whole one after them; k-contiguous ones end with their k.
+  static constexpr bool REACH = RC && 16 / EB > 2;
+  // elements from a stage's base to the operand's end, kleft k from the stage's first on
+  static JB_HD int64_t extent(int64_t ld, int64_t rows, int64_t kleft) {
+    return RC ? (kleft - 1) * ld + rows : (rows - 1) * ld + kleft;
+  }
+  // First k-row of load p of a stage (uniform).  TAIL: the last stage, shorter than BK, whose last vectors start at kleft.
+  template <bool TAIL>
+  static JB_HD int krow(int p, int kleft) {
+    return RC ? (TAIL ? min(p * KPL / LPK, kleft) : p * KPL / LPK) : 0;
+  }
+  // Bytes by which this lane's vector of such a stage's load p (first k-row kp) starts past kleft.
+  static JB_HD Off past(int p, int kp, int kleft, int64_t ld, int lane) {
+    const int lb = lane * LB;
+    if (RC) return KPL > 1 ? (Off)max((lb / EB) / R - (kleft - kp), 0) * (Off)ld * EB : 0;
+    const int k = (((lb % ROWB) / 16 ^ cswz(p * RPL + lb / ROWB)) * 16 + lb % 16) / EB;
+    return (Off)max(k - kleft, 0) * EB;
+  }
   // Load i of this wave's share of the stage at k0 into LDS at `dst` (the operand's part of a slot).  P: the operand
   // at the tile's first row.  TAIL: the last stage, shorter than BK, k clamped to kmax (last vector start).
   // records: bytes from the stage's base up to the operand's end.
@@ -148,17 +172,11 @@ struct RingOperand {
                                         int lane, char* dst, int i) const {
     const int p = wave + NW * i;
     const int kleft = TAIL ? (int)(kmax - k0) : BK;
-    const int kp = RC ? (TAIL ? min(p * KPL / LPK, kleft) : p * KPL / LPK) : 0;  // uniform: first k-row of the load
+    const int kp = krow<TAIL>(p, kleft);
     Off o = off[i];
     if (TAIL) {
       asm volatile("" : "+v"(lane));  // the clamps are formed here, not ahead of the main loop
-      const int lb = lane * LB;
-      if (RC) {
-        if (KPL > 1) o -= (Off)max((lb / EB) / R - (kleft - kp), 0) * (Off)ld * EB;
-      } else {
-        const int k = (((lb % ROWB) / 16 ^ cswz(p * RPL + lb / ROWB)) * 16 + lb % 16) / EB;
-        o -= (Off)max(k - kleft, 0) * EB;
-      }
+      o -= past(p, kp, kleft, ld, lane);
     }
     if constexpr (WIDE) {
       gptr<const char> src = (gptr<const char>)(P + (RC ? (k0 + kp) * ld : k0)) + o;
@@ -200,7 +218,8 @@ struct RingTile {
   char* ring;
   int lane, wave, wm, wn, g, l16;
   gptr<const T> At, Bt;
-  uint32_t arec, brec;  // bytes from the last stage's base to the operand's end (earlier stages' vectors end inside it)
+  uint32_t arec, brec;    // bytes from the last stage's base to the operand's end,
+  uint32_t arec2, brec2;  // and from the base of the one before (RingOperand::REACH; other stages' vectors end inside it)
   int64_t lda, ldb, K, kamax, kbmax;
   int ramax, rbmax, nst, nfull;
   OA oa;
@@ -225,7 +244,9 @@ struct RingTile {
   __device__ __forceinline__ void issue(int st, int slot, int i, Tail) const {
     char* dst = ring + slot * STAGE_B;
     const int64_t k0 = (int64_t)st * BK;
-    const uint32_t records = st == nst - 1 ? (i < OA::NP ? arec : brec) : 0xffffffffu;
+    uint32_t records = st == nst - 1 ? (i < OA::NP ? arec : brec) : 0xffffffffu;
+    if constexpr (OA::REACH || OB::REACH)
+      if (st == nst - 2) records = i < OA::NP ? arec2 : brec2;
     if (i < OA::NP) oa.template issue<Tail::value>(At, records, lda, k0, kamax, wave, lane, dst, i);
     else ob.template issue<Tail::value>(Bt, records, ldb, k0, kbmax, wave, lane, dst + OA::BYTES, i - OA::NP);
   }
@@ -248,8 +269,10 @@ struct RingTile {
     nst = (int)((K + BK - 1) / BK);
     nfull = (int)(K / BK);
     const int64_t kr = K - (int64_t)(nst - 1) * BK;  // k of the last stage
-    arec = buffer_records<T>(TA ? (rows - 1) * lda + kr : (kr - 1) * lda + rows);
-    brec = buffer_records<T>(TB ? (kr - 1) * ldb + cols : (cols - 1) * ldb + kr);
+    arec = buffer_records<T>(OA::extent(lda, rows, kr));
+    brec = buffer_records<T>(OB::extent(ldb, cols, kr));
+    arec2 = OA::REACH ? buffer_records<T>(OA::extent(lda, rows, kr + BK)) : 0xffffffffu;
+    brec2 = OB::REACH ? buffer_records<T>(OB::extent(ldb, cols, kr + BK)) : 0xffffffffu;
     oa.init(lda, ramax, wave, lane);
     ob.init(ldb, rbmax, wave, lane);
 #pragma unroll
