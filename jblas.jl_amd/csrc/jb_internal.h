@@ -99,10 +99,18 @@ void timing_end(hipStream_t s, const char* kernel);
 template <typename T> using gptr = __attribute__((address_space(1))) T*;
 template <typename T> __device__ __forceinline__ gptr<T> as_global(T* p) { return (gptr<T>)p; }
 
+// Upper half of a uniform x, kept apart from it: comparisons of it are scalar instructions,
+// those of 64-bit numbers vector ones.
+__device__ __forceinline__ int upper_half(int64_t x) {
+  int hi = __builtin_amdgcn_readfirstlane((int)(x >> 32));
+  asm("" : "+s"(hi));
+  return hi;
+}
+
 // Record count of a buffer descriptor over `elements` of T, at most 2^32 - 1.
 template <typename T> __device__ __forceinline__ uint32_t buffer_records(int64_t elements) {
-  const uint64_t bytes = (uint64_t)elements * sizeof(T);
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(bytes >> 32) ? 0xffffffffu : (uint32_t)bytes));
+  const int64_t bytes = elements * (int64_t)sizeof(T);
+  return (uint32_t)__builtin_amdgcn_readfirstlane(upper_half(bytes) != 0 ? -1 : (int)bytes);
 }
 
 // Split-K partial results pass between workgroups on different XCDs, whose L2s are not

@@ -37,6 +37,12 @@ typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 //     TF/s, 2999x1777x2111 on odd leading dimensions 462 -> 359 us; FP32 8192^3 130
 //     -> 152 of 157 TF/s.
 //
+//     A short product's time is the prologue and the first stages: loads issued one by
+//     one behind vector arithmetic on uniform values, descriptors that had become vector
+//     values (a loop per load) and stages on run-time slots took 64^3 FP64 from 3.4 us
+//     (register-staged) to 4.0, 96^3 TN 3.9 to 4.9; scalar throughout and with the last
+//     stages unrolled 3.2 and 3.8, 256^3 6.4 -> 5.8 -> 5.1, FP32 256^3 9.2 -> 5.4 -> 4.7.
+//
 //     LDS images (no padding: the loads write 64 consecutive pieces):
 //       rows contiguous (A 'N', B 'T'): [k][R], row r of k-row k at r ^ rswz(k);
 //       k contiguous (A 'T', B 'N'):    [R][BK] in 16-byte chunks, chunk c of
@@ -83,7 +89,8 @@ constexpr int SCHED_ALU = 6;
 // zeros from `records` bytes after base on.
 __device__ __forceinline__ void ring_load(gptr<const void> base, uint32_t records, uint32_t vo, uint32_t so, char* dst) {
 #ifdef __HIP_DEVICE_COMPILE__  // the descriptor type exists on the device only
-  __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(const void*)base, 0, records, 0x00027000);
+  __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(const void*)base, 0,
+                                                                  __builtin_amdgcn_readfirstlane(records), 0x00027000);
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (JB_LDS void*)dst, 16, vo, so, 0, 0);
 #endif
 }
@@ -251,6 +258,10 @@ struct RingTile {
     else ob.template issue<Tail::value>(Bt, records, ldb, k0, kbmax, wave, lane, dst + OA::BYTES, i - OA::NP);
   }
 
+  // min(x, most) of a uniform x >= 0
+  static __device__ __forceinline__ int at_most(int64_t x, int most) {
+    return upper_half(x) != 0 ? most : (int)min((uint32_t)x, (uint32_t)most);
+  }
   // Takes a product: A_, B_ at the tile's first row and column and its first k; rows, cols: what is left of C
   // from there (>= 1); K_: k steps (K_ == 0: no products).  Issues the first stages' loads: every wave of the
   // block must be done with the ring.
@@ -262,12 +273,12 @@ struct RingTile {
     ldb = ldb_;
     K = K_;
     // the last vector starts
-    ramax = (int)min<int64_t>(TA ? rows - 1 : (rows - 1) / VW * VW, BTM);
-    rbmax = (int)min<int64_t>(TB ? (cols - 1) / VW * VW : cols - 1, BTN);
-    kamax = TA ? (K - 1) / VW * VW : K - 1;
-    kbmax = TB ? K - 1 : (K - 1) / VW * VW;
-    nst = (int)((K + BK - 1) / BK);
-    nfull = (int)(K / BK);
+    ramax = at_most(rows - 1, BTM) & ~(TA ? 0 : VW - 1);
+    rbmax = at_most(cols - 1, BTN) & ~(TB ? VW - 1 : 0);
+    kamax = (K - 1) & ~(int64_t)(TA ? VW - 1 : 0);
+    kbmax = (K - 1) & ~(int64_t)(TB ? 0 : VW - 1);
+    nst = (int)((uint64_t)(K + BK - 1) / BK);
+    nfull = (int)((uint64_t)K / BK);
     const int64_t kr = K - (int64_t)(nst - 1) * BK;  // k of the last stage
     arec = buffer_records<T>(OA::extent(lda, rows, kr));
     brec = buffer_records<T>(OB::extent(ldb, cols, kr));
@@ -275,13 +286,18 @@ struct RingTile {
     brec2 = OB::REACH ? buffer_records<T>(OB::extent(ldb, cols, kr + BK)) : 0xffffffffu;
     oa.init(lda, ramax, wave, lane);
     ob.init(ldb, rbmax, wave, lane);
+    // The whole stages' loads and the short one's are apart, here and in stage(): with both forms of a load in one
+    // branch the compiler merged their descriptors into vector registers and looped over the values.
 #pragma unroll
     for (int d = 0; d < NSLOT; ++d)
+      if (d < nfull) {
 #pragma unroll
-      for (int i = 0; i < NLD; ++i) {
-        if (d < nfull) issue(d, d, i, std::false_type());
-        else if (d < nst) issue(d, d, i, std::true_type());
+        for (int i = 0; i < NLD; ++i) issue(d, d, i, std::false_type());
       }
+    if (nfull < nst && nfull < NSLOT) {
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) issue(nfull, nfull, i, std::true_type());
+    }
   }
 
   template <int WI, int WJ>
@@ -343,10 +359,11 @@ struct RingTile {
         if (t + 1 == NT4) {
           constexpr int PI = (NLD + WI - 1) / WI;
 #pragma unroll
-          for (int q = PI * i; q < PI * (i + 1) && q < NLD; ++q) {
-            if (STEADY) issue(st + NSLOT, slot, q, std::false_type());
-            else if (!TAIL && st + NSLOT < nfull) issue(st + NSLOT, slot, q, std::false_type());
-            else if (!TAIL && st + NSLOT < nst) issue(st + NSLOT, slot, q, std::true_type());
+          for (int q = PI * i; q < PI * (i + 1) && q < NLD; ++q)
+            if (STEADY || (!TAIL && st + NSLOT < nfull)) issue(st + NSLOT, slot, q, std::false_type());
+          if (!STEADY && !TAIL && st + NSLOT >= nfull && st + NSLOT < nst) {
+#pragma unroll
+            for (int q = PI * i; q < PI * (i + 1) && q < NLD; ++q) issue(st + NSLOT, slot, q, std::true_type());
           }
         }
       }
@@ -378,6 +395,16 @@ struct RingTile {
       for (int d = 0; d < NSLOT; ++d)
         stage<WI, WJ>(acc, st + d, d, d + 1 == NSLOT ? 0 : d + 1, std::false_type(), std::true_type());
     int slot = 0, nslot = 1;
+    if constexpr (WIM * WIN == 1) {
+      // the last stages on constant offsets too: all of them where K is short, and little code for this tile
+      for (; st < nfull; st += NSLOT)
+#pragma unroll
+        for (int d = 0; d < NSLOT; ++d)
+          if (st + d < nfull)
+            stage<WI, WJ>(acc, st + d, d, d + 1 == NSLOT ? 0 : d + 1, std::false_type(), std::false_type());
+      st = nfull;
+      slot = nfull % NSLOT;
+    }
     for (; st < nfull; ++st) {
       stage<WI, WJ>(acc, st, slot, nslot, std::false_type(), std::false_type());
       slot = nslot;

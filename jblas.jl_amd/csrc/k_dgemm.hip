@@ -117,7 +117,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
     }
   }
   tile.begin(as_global(A) + (TA ? kb + m0 * lda : m0 + kb * lda), lda, as_global(B) + (TB ? n0 + kb * ldb : kb + n0 * ldb),
-             ldb, M - m0, N - n0, min(K - kb, split.kchunk));
+             ldb, M - m0, N - n0, upper_half(K - kb - split.kchunk) < 0 ? K - kb : split.kchunk);
   tile.run(acc);
   if (split.part && !splitk_sum<T, Tile>(acc, splits, split, id, ring)) return;
   tile.store(acc, C + m0 + n0 * ldc, ldc, M - m0, N - n0, alpha, beta);

@@ -47,3 +47,16 @@ def test_gemm_launches_without_implicit_arguments(code_objects):
                 assert "hidden_" not in k, name
     assert kernels >= 40
 
+
+def test_ring_loads_have_scalar_descriptors(code_objects):
+    """A buffer descriptor in vector registers is loaded through in a loop over its values (exec is narrowed to the
+    lanes of one value and the rest go round again)."""
+    kernels = 0
+    for co in code_objects:
+        if "ring_kernel" not in (symbols := run("llvm-readelf", "--symbols", "--wide", co)) and "gemm_mfma_kernel" not in symbols:
+            continue
+        for f in run("llvm-objdump", "-d", "--no-show-raw-insn", co).split("\n\n"):
+            if re.search("gemm_mfma_kernel|grouped_ring_kernel", f.split("\n", 1)[0]):
+                kernels += 1
+                assert not re.search(r"s_xor_b64 exec, exec", f), f.split("\n", 1)[0]
+    assert kernels >= 40
