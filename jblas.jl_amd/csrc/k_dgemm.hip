@@ -23,23 +23,35 @@ namespace {
 //     small product, per chunk of k.
 // ---------------------------------------------------------------------------
 
-// Split-K arguments, one kernel argument: the runtime looks at each pointer that is an
-// argument of its own.
+// The kernel's arguments, in one struct: the runtime looks up each pointer that is an argument
+// of its own, and a kernel that reads a grid dimension (here splits) takes the implicit arguments
+// besides, 256 bytes that the host fills in for every launch.  256^3 FP64 from Python, all of it
+// host time, eight processes each: 10.18 us with 17 arguments and the implicit ones, 9.90 so.
 template <typename T>
-struct SplitK {
-  int64_t kchunk;
-  T* part;
-  int* counters;
+struct KernelArgs {
+  int64_t M, N, K;
+  T alpha;
+  const T* A;
+  int64_t lda;
+  const T* B;
+  int64_t ldb;
+  T beta;
+  T* C;
+  int64_t ldc;
+  int tiles_m, tiles_n, acc_from_c;
+  int splits;       // gridDim.y
+  int64_t kchunk;   // k per split
+  T* part;          // the splits' results (null: one split)
+  int* counters;    // per tile
 };
 
 // Split-K: each block stores its chunk's results, thread by thread, to its slab; the
 // last block of the tile to arrive sums the slabs in split order into acc and
 // returns true.  The counters are zero between launches: the last block clears its own.
 template <typename T, typename Tile>
-__device__ __forceinline__ bool splitk_sum(typename Tile::Acc& acc, int splits, const SplitK<T>& split, int id,
-                                           char* lds) {
+__device__ __forceinline__ bool splitk_sum(typename Tile::Acc& acc, const KernelArgs<T>& p, int id, char* lds) {
   constexpr int EL = Tile::WIM * Tile::WIN * 4;
-  gptr<T> slab = as_global(split.part) + (int64_t)id * splits * (EL * Tile::NTH) + threadIdx.x;
+  gptr<T> slab = as_global(p.part) + (int64_t)id * p.splits * (EL * Tile::NTH) + threadIdx.x;
   auto at = [&](int q, int i, int j, int r) { return ((int64_t)q * EL + (i * Tile::WIN + j) * 4 + r) * Tile::NTH; };
 #pragma unroll
   for (int i = 0; i < Tile::WIM; ++i)
@@ -50,17 +62,17 @@ __device__ __forceinline__ bool splitk_sum(typename Tile::Acc& acc, int splits, 
   int* flag = reinterpret_cast<int*>(lds);
   drain_stores();
   __syncthreads();  // (every wave is done with the ring)
-  if (threadIdx.x == 0) *flag = atomicAdd(split.counters + id, 1);
+  if (threadIdx.x == 0) *flag = atomicAdd(p.counters + id, 1);
   __syncthreads();
-  if (*flag != splits - 1) return false;
-  if (threadIdx.x == 0) split.counters[id] = 0;
+  if (*flag != p.splits - 1) return false;
+  if (threadIdx.x == 0) p.counters[id] = 0;
 #pragma unroll
   for (int i = 0; i < Tile::WIM; ++i)
 #pragma unroll
     for (int j = 0; j < Tile::WIN; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = agent_load<T>(slab + at(0, i, j, r));
-  for (int q = 1; q < splits; ++q)
+  for (int q = 1; q < p.splits; ++q)
 #pragma unroll
     for (int i = 0; i < Tile::WIM; ++i)
 #pragma unroll
@@ -70,24 +82,20 @@ __device__ __forceinline__ bool splitk_sum(typename Tile::Acc& acc, int splits, 
   return true;
 }
 
-// splits: gridDim.y, as an argument.  A kernel that reads a grid dimension takes the
-// implicit arguments, 256 bytes that the host fills in for every launch: a 256^3 FP64
-// call from Python 9.7 us so (all of it host time), 9.4 without.
 template <typename T, bool TA, bool TB, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int NSLOT,
           int MINW>
-__global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
-    int64_t M, int64_t N, int64_t K, T alpha, const T* __restrict__ A, int64_t lda, const T* __restrict__ B, int64_t ldb,
-    T beta, T* __restrict__ C, int64_t ldc, int tiles_m, int tiles_n, int acc_from_c, int splits,
-    SplitK<T> split) {
+__global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(KernelArgs<T> p) {
+  const int64_t M = p.M, N = p.N, K = p.K, lda = p.lda, ldb = p.ldb, ldc = p.ldc;
+  T* const C = p.C;
   typedef RingTile<T, TA, TB, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT> Tile;
   constexpr int WIM = Tile::WIM, WIN = Tile::WIN;
   __shared__ __attribute__((aligned(1024))) char ring[Tile::SMEM];
 
-  const int nblocks = tiles_m * tiles_n;
+  const int nblocks = p.tiles_m * p.tiles_n;
   const int id = xcd_remap(blockIdx.x, nblocks, 8);
   int tm, tn;
-  tile_coords(id, tiles_m, tiles_n, 8, tm, tn);
-  const int64_t m0 = (int64_t)tm * BTM, n0 = (int64_t)tn * BTN, kb = blockIdx.y * split.kchunk;
+  tile_coords(id, p.tiles_m, p.tiles_n, 8, tm, tn);
+  const int64_t m0 = (int64_t)tm * BTM, n0 = (int64_t)tn * BTN, kb = blockIdx.y * p.kchunk;
   Tile tile(ring, threadIdx.x);
 
   // Chains start from -0.0: the first MFMA step fma(a, x, -0.0) is then exactly
@@ -103,7 +111,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
   for (int i = 0; i < WIM; ++i)
 #pragma unroll
     for (int j = 0; j < WIN; ++j) acc[i][j] = typename Tile::acc_t{acc0, acc0, acc0, acc0};
-  if (acc_from_c) {
+  if (p.acc_from_c) {
 #pragma unroll
     for (int i = 0; i < WIM; ++i) {
       const int64_t m = m0 + tile.row(i);
@@ -116,11 +124,11 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gemm_mfma_kernel(
         }
     }
   }
-  tile.begin(as_global(A) + (TA ? kb + m0 * lda : m0 + kb * lda), lda, as_global(B) + (TB ? n0 + kb * ldb : kb + n0 * ldb),
-             ldb, M - m0, N - n0, upper_half(K - kb - split.kchunk) < 0 ? K - kb : split.kchunk);
+  tile.begin(as_global(p.A) + (TA ? kb + m0 * lda : m0 + kb * lda), lda, as_global(p.B) + (TB ? n0 + kb * ldb : kb + n0 * ldb),
+             ldb, M - m0, N - n0, upper_half(K - kb - p.kchunk) < 0 ? K - kb : p.kchunk);
   tile.run(acc);
-  if (split.part && !splitk_sum<T, Tile>(acc, splits, split, id, ring)) return;
-  tile.store(acc, C + m0 + n0 * ldc, ldc, M - m0, N - n0, alpha, beta);
+  if (p.part && !splitk_sum<T, Tile>(acc, p, id, ring)) return;
+  tile.store(acc, C + m0 + n0 * ldc, ldc, M - m0, N - n0, p.alpha, p.beta);
 }
 
 // ---------------------------------------------------------------------------
@@ -250,17 +258,14 @@ template <typename T, bool WIDE, int BTM, int BTN, int WGM, int WGN, int BK, int
 static hipError_t launch_gemm_mfma_bt(const GemmArgs& g, hipStream_t s, int acc_from_c) {
   const int tiles_m = (int)((g.m + BTM - 1) / BTM), tiles_n = (int)((g.n + BTN - 1) / BTN);
   const int nblocks = tiles_m * tiles_n;
-  auto A = static_cast<const T*>(g.A);
-  auto B = static_cast<const T*>(g.B);
-  auto C = static_cast<T*>(g.C);
-  const T alpha = (T)g.alpha, beta = (T)g.beta;
   const int splits = gemm_splits(g);
-  const SplitK<T> split = {splits > 1 ? g.kchunk : g.k, static_cast<T*>(g.part), g.counters};
+  const KernelArgs<T> args = {g.m, g.n, g.k, (T)g.alpha, static_cast<const T*>(g.A), g.lda, static_cast<const T*>(g.B), g.ldb,
+                              (T)g.beta, static_cast<T*>(g.C), g.ldc, tiles_m, tiles_n, acc_from_c, splits,
+                              splits > 1 ? g.kchunk : g.k, static_cast<T*>(g.part), g.counters};
   const char* tname = sizeof(T) == 8 ? "dgemm_mfma" : "sgemm_mfma";
 #define JB_LAUNCH(TA, TB)                                                                                             \
   hipLaunchKernelGGL((gemm_mfma_kernel<T, TA, TB, WIDE, BTM, BTN, WGM, WGN, BK, NSLOT, MINW>), dim3(nblocks, splits), \
-                     dim3(64 * WGM * WGN), 0, s, g.m, g.n, g.k, alpha, A, g.lda, B, g.ldb, beta, C, g.ldc, tiles_m,   \
-                     tiles_n, acc_from_c, splits, split)
+                     dim3(64 * WGM * WGN), 0, s, args)
   timing_begin(s, tname);
   if (!g.ta && !g.tb) JB_LAUNCH(false, false);
   else if (!g.ta && g.tb) JB_LAUNCH(false, true);
