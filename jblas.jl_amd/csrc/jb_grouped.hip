@@ -180,10 +180,6 @@ __global__ __launch_bounds__(GNT, 2) void grouped_kernel(const GProb* __restrict
 }
 
 
-__global__ void zero_i32_kernel(int* p, int n) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
-}
-
 int kind_of(int method) {
   if (method == JB_F64_NATIVE) return 0;
   if (method == JB_F32_NATIVE) return 1;
@@ -696,10 +692,9 @@ int plan_build(int method, int64_t count, const jb_gemm_desc* d, const Forced& f
 // Enqueues [reset counters, 128-row/column persistent kernels, persistent kernel] on s.
 hipError_t plan_enqueue(const GroupedPlanImpl& P, hipStream_t s) {
   if (P.nitems == 0) return hipSuccess;
-  hipLaunchKernelGGL(zero_i32_kernel, dim3((P.ncounters + 255) / 256 < 1024 ? (P.ncounters + 255) / 256 : 1024),
-                     dim3(256), 0, s, P.next, P.ncounters);
+  hipError_t e = launch_zero_i32(P.next, P.ncounters, s);
+  if (e != hipSuccess) return e;
   timing_begin(s, "grouped_gemm");
-  hipError_t e = hipSuccess;
   if (P.nside > 0 && (e = hipEventRecord(P.fork, s)) != hipSuccess) return e;
   int* const tiles = P.next + NLAUNCH * NXCD;
   int j = -1;  // launch j + 1 > 0 goes to side stream j

@@ -73,6 +73,9 @@ size_t bf16x3_workspace_bytes(int64_t m, int64_t n, int64_t k, int splits = 1);
 // the two flags as in launch_dgemm_ozaki.
 hipError_t launch_sgemm_bf16x3(const GemmArgs& g, int nprod, void* ws, bool want_flag, int* sticky, hipStream_t s);
 
+// p[0..n) = 0, n >= 1: a kernel, since a captured graph takes no memset.
+hipError_t launch_zero_i32(int* p, int64_t n, hipStream_t s);
+
 // ---- generator ------------------------------------------------------------
 hipError_t launch_fill_uniform(uint64_t seed, int64_t n, double* out, hipStream_t s);
 hipError_t launch_fill_uniform_f32(uint64_t seed, int64_t n, float* out, hipStream_t s);

@@ -854,7 +854,9 @@ static int sgemm_dev_locked(const GemmArgs& g, int method, int nprod, hipStream_
 // One problem on the single-problem kernels of a grouped method (the caller
 // holds the lock and has validated `g`).  A split problem's partial results live in
 // the workspace, after the 3xBF16 planes; its user order also keeps the counters
-// to one launch at a time.
+// to one launch at a time.  The static rule splits problems that have fewer tiles than
+// the device holds workgroups; a tuned split may have any number of tiles, and past the
+// runtime's counters brings its own in the workspace, zeroed by the call.
 extern "C++" int jb::single_gemm_dev_locked(int method, const GemmArgs& g, hipStream_t s, bool report) {
   const bool x3 = method == JB_F32_BF16X3, f64 = method == JB_F64_NATIVE;
   if (!x3 && !f64 && method != JB_F32_NATIVE) return fail(-1, "unknown method %d", method);
@@ -872,18 +874,23 @@ extern "C++" int jb::single_gemm_dev_locked(int method, const GemmArgs& g, hipSt
   if (gemm_splits(g) > 1) {
     if (x3) bf16x3_split_need(g, &part, &counters);
     else gemm_mfma_split_need(g, f64 ? 8 : 4, &part, &counters);
-    // (problems are split only while they have fewer tiles than the device holds workgroups)
-    if (counters > SPLITK_COUNTERS) return fail(JB_ERR_UNSUPPORTED, "split product of %lld tiles", (long long)counters);
   }
+  const bool own = counters > SPLITK_COUNTERS;
   void* ws = nullptr;
-  int rc = ws_acquire(planes + part, s, &ws);
+  int rc = ws_acquire(planes + part + (own ? (size_t)counters * sizeof(int) : 0), s, &ws);
   if (rc) return rc;
   h.part = part ? static_cast<char*>(ws) + planes : nullptr;
   h.counters = rt().counters;
+  hipError_t e = hipSuccess;
+  if (own) {
+    h.counters = reinterpret_cast<int*>(static_cast<char*>(ws) + planes + part);
+    e = launch_zero_i32(h.counters, counters, s);
+  }
   // (word 1 of the sticky buffer: a flag nobody reads)
-  const hipError_t e = x3    ? launch_sgemm_bf16x3(h, 6, ws, false, rt().sticky + (report ? 0 : 1), s)
-                       : f64 ? launch_dgemm_mfma(h, s)
-                             : launch_sgemm_mfma(h, s);
+  if (e == hipSuccess)
+    e = x3    ? launch_sgemm_bf16x3(h, 6, ws, false, rt().sticky + (report ? 0 : 1), s)
+        : f64 ? launch_dgemm_mfma(h, s)
+              : launch_sgemm_mfma(h, s);
   rc = ws_release(s);
   return e == hipSuccess ? rc : hip_fail(e, "split-K gemm launch");
 }

@@ -21,6 +21,10 @@ __device__ __forceinline__ double unit_uniform(uint64_t x) {  // [-1, 1)
   return 2.0 * ((double)(x >> 11) * 0x1.0p-53) - 1.0;
 }
 
+__global__ void zero_i32_kernel(int* __restrict__ p, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = 0;
+}
+
 __global__ void fill_uniform_kernel(uint64_t seed, int64_t n, double* __restrict__ out) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     out[i] = unit_uniform(sm_at(seed, (uint64_t)i));
@@ -70,6 +74,11 @@ int grid_for(int64_t n) {
 }
 
 }  // namespace
+
+hipError_t launch_zero_i32(int* p, int64_t n, hipStream_t s) {
+  hipLaunchKernelGGL(zero_i32_kernel, dim3(grid_for(n)), dim3(256), 0, s, p, n);
+  return hipGetLastError();
+}
 
 hipError_t launch_fill_uniform(uint64_t seed, int64_t n, double* out, hipStream_t s) {
   hipLaunchKernelGGL(fill_uniform_kernel, dim3(grid_for(n)), dim3(256), 0, s, seed, n, out);
