@@ -25,13 +25,18 @@ struct Runtime {
   int device = -1;
   jb_device_info info{};
   hipStream_t stream = nullptr;  // used by the host-pointer entry points
-  Buffer ws;                     // emulation slices / split-K partials
+  Buffer ws;                     // emulation slices
   Buffer staging;                // host-pointer entry points: A, B, C copies
   hipEvent_t ws_event = nullptr; // last use of `ws`
   bool ws_pending = false;
   bool ws_in_graph = false;      // a graph captured a call that uses `ws`
   std::vector<void*> retired;    // workspaces that captured graphs may use (freed by jb_finalize)
-  int* counters = nullptr;       // split-K arrival counters, all zero between launches (the user holds `ws`)
+  // adjoints of small products: 3xBF16 planes, split-K partials.  Apart from `ws`, which the
+  // replays of captured emulated calls use at any time; these calls are not captured.
+  Buffer adj;
+  hipEvent_t adj_event = nullptr;  // last use of `adj`
+  bool adj_pending = false;
+  int* counters = nullptr;       // split-K arrival counters, all zero between launches (the user holds `adj`)
   int* sticky = nullptr;         // set by any emulated call that met Inf/NaN; cleared by jb_nonfinite_check
 };
 

@@ -162,6 +162,8 @@ int init_locked(int device) {
     if ((e = hipStreamCreateWithFlags(&r.stream, hipStreamNonBlocking)) != hipSuccess)
       return hip_fail(e, "hipStreamCreate");
   }
+  if (r.adj_event == nullptr && (e = hipEventCreateWithFlags(&r.adj_event, hipEventDisableTiming)) != hipSuccess)
+    return hip_fail(e, "hipEventCreate");
   if (r.ws_event == nullptr) {
     if ((e = hipEventCreateWithFlags(&r.ws_event, hipEventDisableTiming)) != hipSuccess)
       return hip_fail(e, "hipEventCreate");
@@ -276,6 +278,27 @@ int ws_release(hipStream_t s) {
   return JB_OK;
 }
 
+// The same for the adjoints' workspace, on streams that are not being captured.
+static int adj_acquire(size_t bytes, hipStream_t s, void** out) {
+  Runtime& r = rt();
+  int rc = r.adj.reserve(bytes, "adjoint workspace");
+  if (rc) return rc;
+  if (r.adj_pending) {
+    hipError_t e = hipStreamWaitEvent(s, r.adj_event, 0);
+    if (e != hipSuccess) return hip_fail(e, "hipStreamWaitEvent");
+  }
+  *out = r.adj.ptr;
+  return JB_OK;
+}
+
+static int adj_release(hipStream_t s) {
+  Runtime& r = rt();
+  hipError_t e = hipEventRecord(r.adj_event, s);
+  if (e != hipSuccess) return hip_fail(e, "hipEventRecord");
+  r.adj_pending = true;
+  return JB_OK;
+}
+
 // ---- host staging ----------------------------------------------------------
 // Copies a rows x cols column-major host matrix (leading dim ld) to device
 // memory with the same leading dimension.
@@ -339,6 +362,7 @@ void finalize_locked() {
   hipDeviceSynchronize();
   grouped_release_all();
   r.ws.release();
+  r.adj.release();
   for (void* p : r.retired) hipFree(p);
   r.retired.clear();
   r.ws_in_graph = false;
@@ -354,6 +378,9 @@ void finalize_locked() {
   if (r.ws_event) hipEventDestroy(r.ws_event);
   r.ws_event = nullptr;
   r.ws_pending = false;
+  if (r.adj_event) hipEventDestroy(r.adj_event);
+  r.adj_event = nullptr;
+  r.adj_pending = false;
   if (r.stream) hipStreamDestroy(r.stream);
   r.stream = nullptr;
   r.inited = false;
@@ -853,7 +880,7 @@ static int sgemm_dev_locked(const GemmArgs& g, int method, int nprod, hipStream_
 
 // One problem on the single-problem kernels of a grouped method (the caller
 // holds the lock and has validated `g`).  A split problem's partial results live in
-// the workspace, after the 3xBF16 planes; its user order also keeps the counters
+// the adjoints' workspace, after the 3xBF16 planes; its user order also keeps the counters
 // to one launch at a time.  The static rule splits problems that have fewer tiles than
 // the device holds workgroups; a tuned split may have any number of tiles, and past the
 // runtime's counters brings its own in the workspace, zeroed by the call.
@@ -877,7 +904,7 @@ extern "C++" int jb::single_gemm_dev_locked(int method, const GemmArgs& g, hipSt
   }
   const bool own = counters > SPLITK_COUNTERS;
   void* ws = nullptr;
-  int rc = ws_acquire(planes + part + (own ? (size_t)counters * sizeof(int) : 0), s, &ws);
+  int rc = adj_acquire(planes + part + (own ? (size_t)counters * sizeof(int) : 0), s, &ws);
   if (rc) return rc;
   h.part = part ? static_cast<char*>(ws) + planes : nullptr;
   h.counters = rt().counters;
@@ -891,7 +918,7 @@ extern "C++" int jb::single_gemm_dev_locked(int method, const GemmArgs& g, hipSt
     e = x3    ? launch_sgemm_bf16x3(h, 6, ws, false, rt().sticky + (report ? 0 : 1), s)
         : f64 ? launch_dgemm_mfma(h, s)
               : launch_sgemm_mfma(h, s);
-  rc = ws_release(s);
+  rc = adj_release(s);
   return e == hipSuccess ? rc : hip_fail(e, "split-K gemm launch");
 }
 
