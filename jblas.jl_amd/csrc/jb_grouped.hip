@@ -1289,9 +1289,12 @@ int jb_gemm_pullback(int method, char transA, char transB, int64_t m, int64_t n,
                  std::max<int64_t>(1, m), dA ? gA : nullptr, std::max<int64_t>(1, ar), dB ? gB : nullptr,
                  std::max<int64_t>(1, br), d);
   if (!d.empty()) {
-    for (auto& x : d)
-      if ((rc = validate_descs(method, 1, &x))) return rc;
-    if ((rc = pullback_run_locked(method, d, s))) return rc;
+    rc = validate_descs(method, (int64_t)d.size(), d.data());
+    if (rc == JB_OK) rc = pullback_run_locked(method, d, s);
+    if (rc) {
+      hipStreamSynchronize(s);  // the copies from the caller's memory
+      return rc;
+    }
   }
   if (dA) d2h(dA, gA, ar, ac, ldda);
   if (dB) d2h(dB, gB, br, bc, lddb);
