@@ -59,8 +59,7 @@ namespace {
 
 // The thread index as an opaque value, read once per work item: offsets derived
 // from it are then formed inside the work loop of the persistent kernel rather
-// than hoisted out of it and held in registers for all eight tile variants at
-// once (which exhausts the register file).
+// than hoisted out of it and held in registers across the items.
 __device__ __forceinline__ int work_item_tid() {
   int t = threadIdx.x;
   asm volatile("" : "+v"(t));

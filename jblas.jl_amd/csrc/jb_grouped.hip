@@ -40,8 +40,8 @@ namespace {
 // 16w..16w+15 in registers.  The workgroup first stages all of op(B) (k x n)
 // in LDS, [p][j] with rows of SB_STRIDE elements, in two batches of loads;
 // each lane then reads its row of op(A) in register chunks of 4 k (the next
-// chunk in flight) and B(p, j0..j0+15) as LDS broadcasts, 8 columns at a time
-// (registers stay within the budget of the MFMA tiles sharing this kernel).  Each element is the chain
+// chunk in flight) and B(p, j0..j0+15) as LDS broadcasts, 8 columns at a time.
+// Each element is the chain
 // acc = A(i,0) B(0,j), acc = fma(A(i,p), B(p,j), acc) for p = 1..k-1 -- the
 // plain first product of src/gemm.jl:86 and the k-steps of :165 -- then the
 // alpha/beta epilogue of the tiles (put_result).
@@ -562,9 +562,8 @@ int plan_build(int method, int64_t count, const jb_gemm_desc* d, const Forced& f
   }
   if (nall >= ((size_t)1 << 31) || (size_t)counters >= ((size_t)1 << 30))
     return fail(JB_ERR_UNSUPPORTED, "grouped plan: %zu work items is too many for one launch", nall);
-  // pass 4: work queues.  One launch per 128-row/column tile shape and
-  // transpose combination, then one for the other items (NLAUNCH); each
-  // launch has one queue per XCD.  A problem with at least 2 NXCD items is
+  // pass 4: work queues.  One launch per kernel (NLAUNCH), each with one queue
+  // per XCD.  A problem with at least 2 NXCD items is
   // cut into NXCD runs of consecutive items, one per queue: items are ordered
   // split by split, and within a split tile by tile in groups of `gr`
   // tile-rows (column by column inside a group), so a run is a compact block
@@ -689,7 +688,7 @@ int plan_build(int method, int64_t count, const jb_gemm_desc* d, const Forced& f
   return JB_OK;
 }
 
-// Enqueues [reset counters, 128-row/column persistent kernels, persistent kernel] on s.
+// Enqueues [reset counters, the launches' persistent kernels (NLAUNCH)] on s and its side streams.
 hipError_t plan_enqueue(const GroupedPlanImpl& P, hipStream_t s) {
   if (P.nitems == 0) return hipSuccess;
   hipError_t e = launch_zero_i32(P.next, P.ncounters, s);

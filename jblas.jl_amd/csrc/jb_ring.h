@@ -33,7 +33,7 @@ typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 //     none left).  So the loads are buffer loads (descriptor + scalar + lane
 //     offset, no arithmetic), the stages are unrolled over the ring (constant LDS
 //     offsets), and the next fragments are read behind the first MFMA row of a group.
-//     FP64, register-staged form -> this: 1024^3 TN 44.2 -> 35.2 us, 4096^3 64 -> 74
+//     FP64, register-staged form -> this: 1024^3 TN 44.2 -> 35.2 us, 4096^3 64 -> 76
 //     TF/s, 2999x1777x2111 on odd leading dimensions 462 -> 359 us; FP32 8192^3 130
 //     -> 152 of 157 TF/s.
 //

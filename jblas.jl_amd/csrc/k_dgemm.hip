@@ -278,7 +278,9 @@ static hipError_t launch_gemm_mfma_bt(const GemmArgs& g, hipStream_t s, int acc_
 
 // Ring configuration <waves along m, along n, k per stage, slots, waves per SIMD> of each tile.  A stage is 16 KB
 // (FP64 64-tile) to 32 KB; 128- and 64-tiles keep two slots and several workgroups per CU, whose waves fill each
-// other's barriers, the smaller tiles more slots, since their stages are shorter than a load's latency.
+// other's barriers, the smaller tiles more slots, since their stages are shorter than a load's latency.  FP64 32x32, us
+// with four slots of 16 k, three of 16 and three of 32: 128^3 4.05, 4.09 and 3.99, 256^3 5.08, 5.03 and 5.32, 512^3
+// 7.21, 7.31 and 7.48, 768^3 20.2, 21.7 and 20.5.
 template <typename T, int BTM, int BTN> struct Ring;
 template <> struct Ring<double, 128, 128> { static constexpr auto run = launch_gemm_mfma_bt<double, false, 128, 128, 2, 4, 16, 2, 4>; };
 template <> struct Ring<double, 64, 64> { static constexpr auto run = launch_gemm_mfma_bt<double, false, 64, 64, 2, 2, 16, 2, 4>; };
@@ -294,10 +296,10 @@ template <> struct Ring<float, 32, 32> { static constexpr auto run = launch_gemm
 // MFMA and run faster, smaller ones spread a grid more evenly.  Rates relative to
 // the 128-tile, measured on full grids (2048^3 to 8192^3); one 128- or 64-tile
 // alone on its CU has no other workgroup to fill its barriers (5 and 10 % slower).
-// Measured, us (128 / 64 / 64x32 / 32): FP64 512^3 63 / 19.0 / 11.7 / 8.1, 1024^3
-// 124 / 37.6 / 36.7 / 36.9, 1536^3 178 / 146 / 119 / 119, 3072^3 1023 / 811 / 876 /
-// 943, 4096^3 1826 / 1961 / 2038 / 2209; FP32 800x840x900 60 / 20.3 / 20.4 / 18.8,
-// 3072^3 519 / 426 / 475 / 526, 4096^3 922 / 986 / 1074 / 1216.
+// Measured, us (128 / 64 / 64x32 / 32): FP64 512^3 61 / 18.5 / 11.6 / 7.6, 1024^3
+// 119 / 38.5 / 34.6 / 34.8, 1536^3 176 / 134 / 114 / 117, 3072^3 1010 / 795 / 832 /
+// 888, 4096^3 1798 / 1909 / 1995 / 2192; FP32 800x840x900 56 / 19.0 / 19.1 / 16.9,
+// 3072^3 514 / 405 / 434 / 474, 4096^3 908 / 923 / 1003 / 1127.
 enum TileId { T128, T64, T64X32, T32, TWIDE };
 template <typename T>
 static TileId pick_tile(const GemmArgs& g) {

@@ -1,5 +1,6 @@
 // k_grouped_ring.h -- persistent grouped kernels of the native methods, one per
-// transpose combination and load width (instantiated in k_grouped_ring*.hip).
+// tile and transpose combination, and one per combination for leading dimensions
+// past 32-bit offsets (instantiated in k_grouped_ring*.hip).
 #pragma once
 #include "jb_grouped.h"
 #include "jb_ring.h"
@@ -7,8 +8,8 @@
 namespace jb {
 namespace {
 
-// Columns coff.. of a BM x ibn item on one ring tile: loads, MFMAs and the result, to C through the alpha/beta epilogue or, with several splits, to
-// this split's slab.  FP64 and FP32 chains start from -0.0 and each k-split is one
+// Columns coff.. of a BM x ibn item on one ring tile: loads, MFMAs and the result,
+// to C through the alpha/beta epilogue or, with several splits, to this split's slab.  FP64 and FP32 chains start from -0.0 and each k-split is one
 // fma chain in increasing k, so every split is the jmul! recurrence bit for bit.
 template <typename Tile, typename T, bool TA, bool TB, int BM>
 __device__ __forceinline__ void ring_part(const GProb& P, const GItem& w, int64_t ms, int64_t n0, int coff, int ibn,
@@ -55,7 +56,7 @@ __device__ __forceinline__ void ring_part(const GProb& P, const GItem& w, int64_
   }
 }
 
-// Pulls native items of one transpose combination and load width from their
+// Pulls native items of one tile and transpose combination from their
 // queues.  Bound: the matrix cores for k from about 256, C's bytes below (1024^2
 // problems, 128x64 tile: 70.5 TF/s of 78.6 at k = 1024, 63.5 at 256, 40.7 at 64).
 //   RING_TALL   128x64, three workgroups per CU; a 128x128 item runs as two halves

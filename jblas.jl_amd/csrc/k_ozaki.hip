@@ -929,8 +929,10 @@ void launch_split(const GemmArgs& g, const Layout& L, char* ws, int* flag, int* 
 
 // Tiles of the last round that run as two blocks each: where the tiles after the last
 // whole round over the compute units are at most half of them, so that the halves still
-// fit one round, which then takes about half as long
-// (2500 x 1900 x 3001, seven INT8 slices, 600 tiles: 406 us, 378 so).
+// fit one round, which then takes about half as long.  256 compute units, k = 3001, us
+// uncut and cut: INT8, seven slices, 320 tiles 346 and 320, 384 tiles 357 and 335, and past
+// the half 416 tiles 364 and 399; BF16, six slices, 504 and 458, 541 and 498, 551 and 626;
+// 3xBF16, six products, 235 and 216, 252 and 238, 260 and 291.
 int half_tiles(int64_t tiles) {
   const int64_t cus = std::max(runtime_compute_units(), 1), rest = tiles % cus;
   return 2 * rest <= cus ? (int)rest : 0;
